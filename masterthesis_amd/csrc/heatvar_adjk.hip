@@ -276,12 +276,17 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
 // issue (0.60 of its rate), not by HBM (0.41 of 8 TB/s).  Two 12-wave workgroups per CU would need
 // at most 80 VGPRs.
 // FP64 fields: 64 x 8 (a 1024-thread workgroup caps a thread at 128 VGPRs,
-// which the FP64 rings exceed).
+// which the FP64 rings exceed), and two steps per sweep only: on 64 x 8 each
+// further step costs two more of the eight rows (us per reverse step at 128^3
+// / 200^3: K = 2 33 / 100, K = 3 37 / 133, K = 4 60 / 222).
+// Grids with fewer workgroups than CUs at the full chunk take shorter ones
+// (fit_chunk): K = 4 FP32 at 97x80x75 123 -> 24 us per sweep, 128^3 127 -> 57.
 // FP32, K = 3: 64 x 12 (64 x 16 caps a thread at 128 VGPRs, which the
 // three-step rings exceed by a 16-byte spill).
 template <typename T, int K>
 struct AdjkTile {
-    static constexpr int TX = 64, TY = sizeof(T) == 8 ? 8 : (K == 3 ? 12 : 16), D = 2, ZC = sizeof(T) == 8 ? 32 : 64;
+    static constexpr int TX = 64, TY = sizeof(T) == 8 ? 8 : (K == 3 ? 12 : 16), D = 2, ZC = sizeof(T) == 8 ? 32 : 64,
+                         PER_CU = 1;
 };
 
 template <typename T, int K>
@@ -291,10 +296,11 @@ int adjk_launch_t(Ctx* c, const Geo& g, const void* lam, void* lamo, const void*
     typedef AdjkTile<T, K> A;
     constexpr int R = K - 1;
     const int tiles_x = ceil_div(g.nx, A::TX - 2 * R), tiles_y = ceil_div(g.ny, A::TY - 2 * R);
-    const long nb = (long)tiles_x * tiles_y * ceil_div(g.nz, A::ZC);
+    const int zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * R + 1, A::ZC, A::PER_CU, c->cu_count);
+    const long nb = (long)tiles_x * tiles_y * ceil_div(g.nz, zc);
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");
     heatvar_adjk_kernel<T, A::TX, A::TY, K, A::D><<<dim3((unsigned)nb), dim3(A::TX, A::TY), 0, c->stream>>>(
-        g, (const T*)lam, (T*)lamo, (const T*)kap, st, grad, cf, A::ZC, tiles_x, tiles_y);
+        g, (const T*)lam, (T*)lamo, (const T*)kap, st, grad, cf, zc, tiles_x, tiles_y);
     SCAFES_HIP(hipGetLastError());
     return SCAFES_OK;
 }
@@ -303,12 +309,12 @@ template <typename T>
 int adjk_launch_k(Ctx* c, const Geo& g, int K, const void* lam, void* lamo, const void* kap, const AdjkStates& st,
                   double* grad, const AdjVarCoef& cf)
 {
-    switch (K) {
-    case 2: return adjk_launch_t<T, 2>(c, g, lam, lamo, kap, st, grad, cf);
-    case 3: return adjk_launch_t<T, 3>(c, g, lam, lamo, kap, st, grad, cf);
-    case 4: return adjk_launch_t<T, 4>(c, g, lam, lamo, kap, st, grad, cf);
-    default: return fail(SCAFES_ERR_ARG, "multi-step var-kappa adjoint: K must be 2..4");
+    if (K == 2) return adjk_launch_t<T, 2>(c, g, lam, lamo, kap, st, grad, cf);
+    if constexpr (sizeof(T) == 4) {
+        if (K == 3) return adjk_launch_t<T, 3>(c, g, lam, lamo, kap, st, grad, cf);
+        if (K == 4) return adjk_launch_t<T, 4>(c, g, lam, lamo, kap, st, grad, cf);
     }
+    return fail(SCAFES_ERR_ARG, "multi-step var-kappa adjoint: K out of range");
 }
 
 }  // namespace
@@ -322,12 +328,15 @@ bool heatvar_adjk_supported(const Geo& geo)
     return geo.dim == 3 && (kPlanes * geo.e01 + geo.base + geo.e01) * 8L < (long)kRecords;
 }
 
+int heatvar_adjk_max(int dtype) { return dtype == SCAFES_F64 ? 2 : kAdjMaxK; }
+
 int heatvar_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, int K, const void* lam,
                         void* lamo, const void* kap, const void* const* u, double* grad, double tau)
 {
     if (!heatvar_adjk_supported(geo))
         return fail(SCAFES_ERR_UNSUPPORTED, "multi-step var-kappa adjoint needs a 3-D grid");
-    if (K < 2 || K > kAdjMaxK) return fail(SCAFES_ERR_ARG, "multi-step var-kappa adjoint: K must be 2..4");
+    if (K < 2 || K > heatvar_adjk_max(dtype))
+        return fail(SCAFES_ERR_ARG, "multi-step var-kappa adjoint: K out of range");
     AdjkStates st{};
     for (int l = 0; l < K; ++l) {
         if (!u[l]) return fail(SCAFES_ERR_ARG, "multi-step var-kappa adjoint: missing state");

@@ -905,10 +905,12 @@ static constexpr int kNumTb = sizeof(kTbCfgs) / sizeof(kTbCfgs[0]);
 
 template <int STEPS, typename T, int MODE, int TX, int TY, int D, bool MO = false>
 static int tb_launch_t(Ctx* c, const Geo& g, const void* u, const void* cin, const void* kap, void* uo, void* co,
-                       const VarCoef& cf, int zc, void* const* mid = nullptr)
+                       const VarCoef& cf, int zc, bool fit, void* const* mid = nullptr)
 {
     constexpr int RING = STEPS - 1;  // ring width of the thread tile on each side
+    constexpr int kPerCu = TX * TY > 768 ? 1 : 2;
     const int tiles_x = ceil_div(g.nx, TX - 2 * RING), tiles_y = ceil_div(g.ny, TY - 2 * RING);
+    if (fit) zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * RING + 1, zc, kPerCu, c->cu_count);
     const int tiles_z = ceil_div(g.nz, zc);
     const long nb = (long)tiles_x * tiles_y * tiles_z;
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");
@@ -929,12 +931,12 @@ static int tb_launch_t(Ctx* c, const Geo& g, const void* u, const void* cin, con
 
 template <typename T, int MODE>
 static int tb_dispatch(Ctx* c, const Geo& g, const void* u, const void* cin, const void* kap, void* uo, void* co,
-                       const VarCoef& cf, int cfg)
+                       const VarCoef& cf, int cfg, bool fit)
 {
     const TbCfg t = kTbCfgs[cfg];
 #define SCAFES_TB(S, X, Y, DD)                                                                    \
     case S * 10000000 + X * 100000 + Y * 100 + DD:                                                \
-        return tb_launch_t<S, T, MODE, X, Y, DD>(c, g, u, cin, kap, uo, co, cf, t.zc);
+        return tb_launch_t<S, T, MODE, X, Y, DD>(c, g, u, cin, kap, uo, co, cf, t.zc, fit);
     switch (t.steps * 10000000 + t.tx * 100000 + t.ty * 100 + t.d) {
         SCAFES_TB(2, 64, 16, 2)
         SCAFES_TB(2, 64, 8, 2)
@@ -963,15 +965,15 @@ static int tb_dispatch(Ctx* c, const Geo& g, const void* u, const void* cin, con
 // four-step tile with prefetch depth 2.
 template <typename T, int MODE>
 static int tb_dispatch_mo(Ctx* c, const Geo& g, const void* u, const void* cin, const void* kap, void* uo, void* co,
-                          const VarCoef& cf, int cfg, void* const* mid)
+                          const VarCoef& cf, int cfg, bool fit, void* const* mid)
 {
     const TbCfg t = kTbCfgs[cfg];
     if (t.steps == 3 && t.tx == 64 && t.ty == 16 && t.d == 2)
-        return tb_launch_t<3, T, MODE, 64, 16, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, mid);
+        return tb_launch_t<3, T, MODE, 64, 16, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, fit, mid);
     if (t.steps == 3 && t.tx == 64 && t.ty == 12 && t.d == 2)
-        return tb_launch_t<3, T, MODE, 64, 12, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, mid);
+        return tb_launch_t<3, T, MODE, 64, 12, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, fit, mid);
     if (t.steps == 4 && t.tx == 64 && t.ty == 16 && t.d == 2)
-        return tb_launch_t<4, T, MODE, 64, 16, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, mid);
+        return tb_launch_t<4, T, MODE, 64, 16, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, fit, mid);
     return fail(SCAFES_ERR_UNSUPPORTED, "no state-writing variant of this multi-step tile");
 }
 
@@ -1005,7 +1007,7 @@ bool heatvar_tb2_supported(const Geo& geo, int mode)
 // The configuration's number of steps u -> uo (and Kahan compensation cin -> co).
 int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, const void* u, void* uo,
                        const void* cin, void* co, const void* kap, double tau, int border_mode, double border_value,
-                       int cfg, void* const* mid)
+                       int cfg, bool fit, void* const* mid)
 {
     if (cfg < 0 || cfg >= kNumTb) return fail(SCAFES_ERR_ARG, "bad multi-step tile configuration");
     if (!heatvar_tb2_supported(geo, mode)) return fail(SCAFES_ERR_UNSUPPORTED, "multi-step sweep needs a 3-D grid");
@@ -1023,14 +1025,14 @@ int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, c
     cf.border_mode = border_mode;
     if (mid) {
         if (mode == SCAFES_HEATVAR_F64)
-            return tb_dispatch_mo<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, mid);
+            return tb_dispatch_mo<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit, mid);
         if (mode == SCAFES_HEATVAR_F32)
-            return tb_dispatch_mo<float, 1>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, mid);
-        return tb_dispatch_mo<float, 2>(c, geo, u, cin, kap, uo, co, cf, cfg, mid);
+            return tb_dispatch_mo<float, 1>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit, mid);
+        return tb_dispatch_mo<float, 2>(c, geo, u, cin, kap, uo, co, cf, cfg, fit, mid);
     }
-    if (mode == SCAFES_HEATVAR_F64) return tb_dispatch<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg);
-    if (mode == SCAFES_HEATVAR_F32) return tb_dispatch<float, 1>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg);
-    return tb_dispatch<float, 2>(c, geo, u, cin, kap, uo, co, cf, cfg);
+    if (mode == SCAFES_HEATVAR_F64) return tb_dispatch<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit);
+    if (mode == SCAFES_HEATVAR_F32) return tb_dispatch<float, 1>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit);
+    return tb_dispatch<float, 2>(c, geo, u, cin, kap, uo, co, cf, cfg, fit);
 }
 
 }  // namespace scafes

@@ -334,6 +334,16 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(W))) voi
 // sweep do not pay: K = 5 on 64x16 (9.6 B per step, 118 VGPRs, one
 // workgroup per CU) gave the 2000-step gradient with 62 snapshots in 302.6
 // ms against 300.4 for K = 4 on 64x12, and K = 6 (8.7 B per step) 335 ms.
+// FP64 fields and the Tumor border stop at K = 3.  FP64, us per reverse step at
+// 97^3 / 128^3 / 200^3: K = 2 10.4 / 17.4 / 63, K = 3 9.2 / 18.4 / 56, K = 4
+// 10.0 / 23.6 / 68.  Under the Tumor border the four-step sweep needs more than
+// the 80 VGPRs of two workgroups per CU and spills (267 us per launch at 256^3
+// FP32, 67 us per step), the three-step one does not (161 us, 54 per step):
+// the 2000-step gradient with 500 snapshots took 293 ms with at most three
+// reverse steps per sweep against 312 with four (355 with four at one
+// workgroup per CU).
+// Smaller grids shorten the chunks (fit_chunk): K = 4 FP32 at 128^3 50 -> 37 us
+// per sweep, 97x80x75 36 -> 18.
 constexpr int kKTX = 64, kKTY = 12, kKZC = 32, kKD = 2;
 
 template <typename T, bool LO, int K, bool TU>
@@ -342,11 +352,12 @@ int adjk_launch_t(Ctx* c, const Geo& g, const void* lam, void* lamo, const void*
 {
     constexpr int R = K - 1;
     const int tiles_x = ceil_div(g.nx, kKTX - 2 * R), tiles_y = ceil_div(g.ny, kKTY - 2 * R);
-    const int tiles_z = ceil_div(g.nz, kKZC);
+    const int zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * R + 1, kKZC, 2, c->cu_count);
+    const int tiles_z = ceil_div(g.nz, zc);
     const long nb = (long)tiles_x * tiles_y * tiles_z;
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");
     pennes_adjk_kernel<T, LO, kKTX, kKTY, K, kKD, TU><<<dim3((unsigned)nb), dim3(kKTX, kKTY), 0, c->stream>>>(
-        g, (const T*)lam, (T*)lamo, (const T*)w, st, grad, cf, kKZC, tiles_x, tiles_y);
+        g, (const T*)lam, (T*)lamo, (const T*)w, st, grad, cf, zc, tiles_x, tiles_y);
     SCAFES_HIP(hipGetLastError());
     return SCAFES_OK;
 }
@@ -358,9 +369,11 @@ int adjk_launch_k(Ctx* c, const Geo& g, int K, const void* lam, void* lamo, cons
     switch (K) {
     case 2: return adjk_launch_t<T, LO, 2, TU>(c, g, lam, lamo, w, st, grad, cf);
     case 3: return adjk_launch_t<T, LO, 3, TU>(c, g, lam, lamo, w, st, grad, cf);
-    case 4: return adjk_launch_t<T, LO, 4, TU>(c, g, lam, lamo, w, st, grad, cf);
-    default: return fail(SCAFES_ERR_ARG, "multi-step adjoint: K must be 2..4");
+    default: break;
     }
+    if constexpr (sizeof(T) == 4 && !TU)
+        if (K == 4) return adjk_launch_t<T, LO, 4, TU>(c, g, lam, lamo, w, st, grad, cf);
+    return fail(SCAFES_ERR_ARG, "multi-step adjoint: K out of range");
 }
 
 }  // namespace
@@ -373,12 +386,14 @@ bool pennes_adjk_supported(const Geo& geo)
                                (long)kRecords;
 }
 
+int pennes_adjk_max(int dtype, bool tumor) { return dtype == SCAFES_F64 || tumor ? 3 : kAdjMaxK; }
+
 int pennes_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, int K, const void* lam,
                        void* lam_out, const void* w, const void* const* t, const void* const* tlo, double* grad,
                        const scafes_pennes_params* p)
 {
     if (!pennes_adjk_supported(geo)) return fail(SCAFES_ERR_UNSUPPORTED, "multi-step adjoint needs a 3-D grid");
-    if (K < 2 || K > kAdjMaxK) return fail(SCAFES_ERR_ARG, "multi-step adjoint: K must be 2..4");
+    if (K < 2 || K > kAdjMaxK) return fail(SCAFES_ERR_ARG, "multi-step adjoint: K out of range");
     if (p->border_mode != SCAFES_BORDER_KEEP && p->border_mode != SCAFES_BORDER_TUMOR)
         return fail(SCAFES_ERR_ARG, "multi-step adjoint: border_mode must be KEEP or TUMOR");
     const bool tumor = p->border_mode == SCAFES_BORDER_TUMOR;

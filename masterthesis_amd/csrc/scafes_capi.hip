@@ -238,6 +238,37 @@ void coef_invalidate(Ctx* c, const void* p, size_t bytes)
     c->ncoef = k;
 }
 
+// A workgroup runs its chunk plus `fill` planes (the rings along z and the
+// pipeline behind them), so long chunks waste least and short ones fill the
+// CUs: per_cu workgroups run at once on a CU, a last round of at most one
+// workgroup per CU takes about 0.65 of one of two, and the chunk with the
+// least rounds x (planes + fill) is taken (the longest of equals).  Where the
+// full chunk already makes four rounds it stays: there the measured default
+// tiles hold.  Measured on an MI355X against chunks of 4..64 planes on grids
+// of 48^3 to 384x300x320, the choice is within 8 % of the best of them for
+// every sweep; the var-kappa sweeps, us with the full 64 (128) planes -> fitted:
+// FP64 three steps 201x150x131 140 -> 79, 64^3 127 -> 20; FP32 three steps
+// 128^3 46 -> 23; FP32 + Kahan four steps 97x80x75 69 -> 17, 256^3 217 -> 189.
+int fit_chunk(long nxy, int nz, int fill, int zmax, int per_cu, int cu_count)
+{
+    const long cus = cu_count > 0 ? cu_count : 256;
+    const long slots = cus * per_cu;
+    if (nxy * ceil_div(nz, zmax) >= 4 * slots) return zmax;
+    int best = 1;
+    double least = 0.0;
+    for (int zc = zmax < nz ? zmax : nz; zc >= 1; --zc) {
+        const long nb = nxy * ceil_div(nz, zc);
+        const long rem = nb % slots;
+        const double rounds = (double)(nb / slots) + (rem == 0 ? 0.0 : rem <= cus && per_cu > 1 ? 0.65 : 1.0);
+        const double cost = rounds * (zc + fill);
+        if (least == 0.0 || cost < least) {
+            least = cost;
+            best = zc;
+        }
+    }
+    return best;
+}
+
 double diffusion_rate(const scafes_geom* g, double dmax)
 {
     double r = 0.0;

@@ -119,6 +119,10 @@ __device__ inline int xcd_remap(int b, int nb)
 
 inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 
+// z planes per workgroup (at most zmax) of a z-streaming sweep over nz
+// planes of nxy tiles whose workgroups run `fill` planes besides their chunk.
+int fit_chunk(long nxy, int nz, int fill, int zmax, int per_cu, int cu_count);
+
 // Pennes forward / adjoint launches (defined in stencil3d.hip).
 // dtype SCAFES_F32_KAHAN: compensated FP32 forward (cin/cout compensation fields);
 // tprev_lo != null: the adjoint reads the forward state as a (hi, lo) pair.
@@ -173,9 +177,11 @@ constexpr int kAdjMaxK = 4;
 // heatvar_adjk.hip): lam^n -> lam^{n-K} with u[l] = u^{n-1-l} (value parts),
 // bit-identical to K heatvar_adj_launch calls.
 bool heatvar_adjk_supported(const Geo& geo);
+int heatvar_adjk_max(int dtype);  // largest K for these fields
 int heatvar_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, int K, const void* lam,
                         void* lamo, const void* kap, const void* const* u, double* grad, double tau);
 bool pennes_adjk_supported(const Geo& geo);
+int pennes_adjk_max(int dtype, bool tumor);  // largest K for these fields
 int pennes_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, int K, const void* lam,
                        void* lam_out, const void* w, const void* const* t, const void* const* tlo, double* grad,
                        const scafes_pennes_params* p);
@@ -186,11 +192,13 @@ int pennes_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
 int heatvar_tb2_num_cfgs();
 void heatvar_tb2_cfg(int cfg, int* tx, int* ty, int* zc, int* d, int* steps);
 bool heatvar_tb2_supported(const Geo& geo, int mode);  // 3-D grids with 32-bit in-plane offsets
+// fit: the z chunk shortened to fill the CUs (fit_chunk) instead of the
+// configuration's.
 // mid = nullptr, or the steps - 1 intermediate state outputs of a
 // configuration with a state-writing variant (heatvar_tb_states_supported).
 int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, const void* u, void* uo,
                        const void* cin, void* co, const void* kap, double tau, int border_mode, double border_value,
-                       int cfg, void* const* mid = nullptr);
+                       int cfg, bool fit, void* const* mid = nullptr);
 bool heatvar_tb_states_supported(int cfg);
 
 // Yee box of N cells per axis; fields hold N+1 nodes per axis, x fastest.

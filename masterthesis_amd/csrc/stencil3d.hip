@@ -857,11 +857,20 @@ int pennes_step_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
     return launch<PennesOp<float>, float>(c, op, geo, -1);
 }
 
+// The one-step tile of a mode: the 512^3 one where its long chunks make at
+// least four workgroups per CU, else the short-chunk launch (cfg = -1).
+static int one_step_cfg(const Ctx* c, const Geo& g, int mode)
+{
+    const TileCfg t = kCfgs[kOneStepCfgByMode[mode]];
+    const long nb = (long)ceil_div(g.nx, t.tx) * ceil_div(g.ny, t.ty) * ceil_div(g.nz, t.zc);
+    return nb < 4L * (c->cu_count > 0 ? c->cu_count : 256) ? -1 : kOneStepCfgByMode[mode];
+}
+
 int heat7var_step_one(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, const void* u, void* un,
                       const void* cin, void* cout, const void* kap, double tau, int border_mode, double border_value)
 {
     return heat7var_launch(c, geo, g, mode, u, un, cin, cout, kap, tau, border_mode, border_value,
-                           kOneStepCfgByMode[mode]);
+                           one_step_cfg(c, geo, mode));
 }
 
 int heatvar_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, const void* lam, void* lam_new,
@@ -1239,7 +1248,7 @@ int scafes_heat7var_run(scafes_ctx* ctx, const scafes_geom* g, int hw, int mode,
         heatvar_tb2_cfg(cfg - kNumCfgs, &tx_, &ty_, &zc_, &d_, &st);
         for (; s + st <= nsteps; s += st, ++launches) {
             rc = heatvar_tb2_launch(c, geo, g, mode, a, b, ca, cb, kappa, tau, border_mode, border_value,
-                                    cfg - kNumCfgs);
+                                    cfg - kNumCfgs, false);
             if (rc) return rc;
             std::swap(a, b);
             std::swap(ca, cb);
@@ -1247,7 +1256,7 @@ int scafes_heat7var_run(scafes_ctx* ctx, const scafes_geom* g, int hw, int mode,
         // two steps left behind a three-step tile: one two-step sweep
         if (nsteps - s == 2) {
             rc = heatvar_tb2_launch(c, geo, g, mode, a, b, ca, cb, kappa, tau, border_mode, border_value,
-                                    kTwoStepCfgByMode[mode] - kNumCfgs);
+                                    kTwoStepCfgByMode[mode] - kNumCfgs, false);
             if (rc) return rc;
             std::swap(a, b);
             std::swap(ca, cb);
@@ -1255,6 +1264,8 @@ int scafes_heat7var_run(scafes_ctx* ctx, const scafes_geom* g, int hw, int mode,
             ++launches;
         }
         cfg = kOneStepCfgByMode[mode];  // a last step one per sweep
+    } else if (planned && cfg != tuned_cfg(c, geo, mode)) {
+        cfg = one_step_cfg(c, geo, mode);
     }
     for (; s < nsteps; ++s, ++launches) {
         rc = heat7var_launch(c, geo, g, mode, a, b, ca, cb, kappa, tau, border_mode, border_value, cfg);
@@ -1522,7 +1533,7 @@ int heat7var_sweep_k(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, int
     if (cfg < kNumCfgs || cfg_steps(cfg) != k || !heatvar_tb2_supported(geo, mode))
         return fail(SCAFES_ERR_UNSUPPORTED, "no sweep of this many steps for this grid and mode");
     return heatvar_tb2_launch(c, geo, g, mode, u, un, cin, cout, kap, tau, border_mode, border_value,
-                              cfg - kNumCfgs);
+                              cfg - kNumCfgs, cfg != tuned_cfg(c, geo, mode));
 }
 
 bool heat7var_states_sweep_ok(const Ctx* c, const Geo& geo, int mode)
@@ -1546,7 +1557,7 @@ int heat7var_sweep_states(Ctx* c, const Geo& geo, const scafes_geom* g, int mode
     if (k == 4 && heat7var_states4_ok(c, geo, mode)) cfg = kFourStepCfgByMode[mode];
     if (cfg < kNumCfgs) return fail(SCAFES_ERR_UNSUPPORTED, "no state-writing sweep of this many steps for this grid");
     return heatvar_tb2_launch(c, geo, g, mode, u, un, cin, cout, kap, tau, border_mode, border_value,
-                              cfg - kNumCfgs, mid);
+                              cfg - kNumCfgs, cfg != tuned_cfg(c, geo, mode), mid);
 }
 
 }  // namespace scafes

@@ -357,8 +357,28 @@ __global__ void yee_pulse_kernel(YeeDims d, T* f, double sigma)
     }
 }
 
-constexpr int kYTX = 64, kYTY = 4, kYZC = 64;         // two-pass in-place tiles
-constexpr int kFTX = 64, kFTY = 8, kFZC = 64, kFD = 2;  // fused out-of-place tile
+// Two-pass in-place tiles: no LDS and no prefetch ring, so a pass lives on
+// the number of waves in flight and takes short z chunks; the H and the E
+// pass, us on an MI355X with chunks of 64 / 16 / 4 planes: FP32 64^3 41 / 12
+// / 5.6 and 49 / 14 / 5.7, 384^3 576 / 490 / 473 and 525 / 450 / 436, FP64
+// 320^3 667 / 602 / 567 and 635 / 556 / 525.  Boxes of more than kYBlocks
+// workgroups double the chunk (up to 64 planes), which bounds the energy
+// partials.
+constexpr int kYTX = 64, kYTY = 4, kYZC = 4, kYZMax = 64;
+constexpr long kYBlocks = 32768;
+// Fused out-of-place tile.  Chunks of at most 32 (FP32) and 16 (FP64)
+// planes; us per step at FP32 192^3 115 with the fitted 28 planes, 141 with
+// 64, FP64 256^3 470 with 16, 490 with 32, 538 with 64.
+constexpr int kFTX = 64, kFTY = 8, kFD = 2;
+template <typename T>
+constexpr int kFZC = sizeof(T) == 8 ? 16 : 32;
+
+static int yee_inplace_chunk(const Ctx* c, long nxy, int planes)
+{
+    int zc = fit_chunk(nxy, planes, 1, kYZC, 8, c->cu_count);
+    while (zc < kYZMax && nxy * ceil_div(planes, zc) > kYBlocks) zc *= 2;
+    return std::min(zc, kYZMax);
+}
 
 // energy: host array of the records (allocating path: the partials and the
 // device records come from the stream-ordered allocator and the records are
@@ -377,9 +397,12 @@ static int yee_run_t(Ctx* c, int N, double s, T* f, T* f2, int nsteps, int energ
     const bool fused = f2 != nullptr;
     if (fused && d.M2 * (long)sizeof(T) >= (1L << 32)) return fail(SCAFES_ERR_ARG, "yee: plane too large");
     const bool tb2 = fused && yee_tb2_supported(d, (int)sizeof(T));
-    const int TX = fused ? kFTX : kYTX, TY = fused ? kFTY : kYTY, ZC = fused ? kFZC : kYZC;
+    const int TX = fused ? kFTX : kYTX, TY = fused ? kFTY : kYTY;
     const int OX = fused ? TX - 1 : TX, OY = fused ? TY - 1 : TY;
-    const int tiles_x = ceil_div(N + 1, OX), tiles_y = ceil_div(N + 1, OY), tiles_z = ceil_div(N + 1, ZC);
+    const int tiles_x = ceil_div(N + 1, OX), tiles_y = ceil_div(N + 1, OY);
+    const long nxy = (long)tiles_x * tiles_y;
+    const int ZC = fused ? fit_chunk(nxy, N + 1, 3, kFZC<T>, 2, c->cu_count) : yee_inplace_chunk(c, nxy, N + 1);
+    const int tiles_z = ceil_div(N + 1, ZC);
     const long nb = (long)tiles_x * tiles_y * tiles_z;
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "yee: grid too large");
     const Tb2Plan plan = yee_tb2_plan(d, (int)sizeof(T), c->cu_count);
@@ -455,10 +478,11 @@ int yee_fused_eps_launch(Ctx* c, const YeeDims& d, T s, const T* a, T* b, const 
 {
     if (d.M2 * (long)sizeof(T) >= (1L << 32)) return fail(SCAFES_ERR_ARG, "yee: plane too large");
     const int tiles_x = ceil_div(d.N + 1, kFTX - 1), tiles_y = ceil_div(d.N + 1, kFTY - 1);
-    const long nb = (long)tiles_x * tiles_y * ceil_div(d.N + 1, kFZC);
+    const int zc = fit_chunk((long)tiles_x * tiles_y, d.N + 1, 3, kFZC<T>, 2, c->cu_count);
+    const long nb = (long)tiles_x * tiles_y * ceil_div(d.N + 1, zc);
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "yee: grid too large");
     yee_fused_kernel<T, kFTX, kFTY, kFD, true><<<dim3((unsigned)nb), dim3(kFTX, kFTY), 0, c->stream>>>(
-        d, s, a, b, kFZC, tiles_x, tiles_y, nullptr, ce);
+        d, s, a, b, zc, tiles_x, tiles_y, nullptr, ce);
     SCAFES_HIP(hipGetLastError());
     return SCAFES_OK;
 }

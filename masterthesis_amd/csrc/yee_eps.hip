@@ -303,10 +303,13 @@ constexpr int kInitBlocks = 2048;
 // 32 or 64 planes, 64 x 4 and a four-plane queue; the 200-step gradient with
 // 100 snapshots took 434 ms with 32-plane chunks, 441, 436 and 458 with 48,
 // 64 and 128); FP64: 64 x 4 (its four LDS planes take twice the space) with
-// 64-plane chunks.
+// at most 16-plane chunks (us per step with 64 / 16: 192^3 513 / 400, 256^3
+// 935 / 844).  Smaller boxes fit the chunk to the CUs: FP32 128^3 91 -> 58 us
+// per step, 64^3 59 -> 12.
 template <typename T>
 struct AdjTile {
-    static constexpr int TX = 64, TY = sizeof(T) == 4 ? 16 : 4, D = 2, ZC = sizeof(T) == 4 ? 32 : 64;
+    static constexpr int TX = 64, TY = sizeof(T) == 4 ? 16 : 4, D = 2, ZC = sizeof(T) == 4 ? 32 : 16,
+                         PER_CU = sizeof(T) == 4 ? 1 : 4;
 };
 
 template <typename T>
@@ -315,10 +318,11 @@ int adj_t(Ctx* c, const YeeDims& d, double s, const T* ce, const T* eps, const T
 {
     typedef AdjTile<T> A;
     const int tiles_x = ceil_div(d.M, A::TX - 1), tiles_y = ceil_div(d.M, A::TY - 1);
-    const long nb = (long)tiles_x * tiles_y * ceil_div(d.M, A::ZC);
+    const int zc = fit_chunk((long)tiles_x * tiles_y, (int)d.M, 3, A::ZC, A::PER_CU, c->cu_count);
+    const long nb = (long)tiles_x * tiles_y * ceil_div(d.M, zc);
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "yee eps: grid too large");
     adj_fused<T, A::TX, A::TY, A::D><<<dim3((unsigned)nb), dim3(A::TX, A::TY), 0, c->stream>>>(
-        d, (T)s, st, la, lb, ce, eps, grad, A::ZC, tiles_x, tiles_y);
+        d, (T)s, st, la, lb, ce, eps, grad, zc, tiles_x, tiles_y);
     SCAFES_HIP(hipGetLastError());
     return SCAFES_OK;
 }

@@ -1,0 +1,72 @@
+"""Launches whose z chunk follows the grid: the result does not depend on how
+the planes are split over workgroups, so the planned sweeps equal one-step
+launches of a fixed tile, and the two Yee schedules equal each other, bit for
+bit, on grids from one plane per workgroup to several rounds."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from masterthesis_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+MODES = [capi.HEATVAR_F64, capi.HEATVAR_F32, capi.HEATVAR_F32_KAHAN]
+
+
+@pytest.fixture(scope="module")
+def ctx(hip):
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("n", [(3, 4, 5), (61, 9, 64), (97, 80, 75), (130, 33, 257), (40, 300, 2)])
+@pytest.mark.parametrize("steps", [3, 8, 11])
+def test_planned_sweeps_equal_one_step_launches(ctx, mode, n, steps):
+    dt = np.float64 if mode == capi.HEATVAR_F64 else np.float32
+    rng = np.random.default_rng(sum(n) + steps)
+    g = capi.geom(n)
+    shape = tuple(m + 2 for m in reversed(n))
+    u0 = rng.standard_normal(shape).astype(dt)
+    kap = (1.0 + 0.5 * rng.random(shape)).astype(dt)
+    tau = 0.9 / sum(2 * 1.5 * (m - 1.0) ** 2 for m in n)
+    out = []
+    for cfg in (-1, 3):
+        bufs = [ctx.upload(a) for a in (u0, u0, 0 * u0, 0 * u0, kap)]
+        which = C.c_int(0)
+        p = [b.ptr for b in bufs]
+        capi.check(ctx.L.scafes_heat7var_run(ctx.h, C.byref(g), 1, mode, p[0], p[1], p[2], p[3], p[4], tau, steps,
+                                             capi.BORDER_VALUE, 0.25, cfg, C.byref(which)))
+        w = which.value
+        out.append([bufs[w].read(shape)[1:-1, 1:-1, 1:-1], bufs[2 + w].read(shape)[1:-1, 1:-1, 1:-1]])
+        for b in bufs:
+            b.free()
+    assert np.array_equal(out[0][0], out[1][0])
+    if mode == capi.HEATVAR_F32_KAHAN:
+        assert np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("dtype", [capi.F32, capi.F64])
+@pytest.mark.parametrize("n", [2, 5, 33, 64, 90])
+@pytest.mark.parametrize("steps", [1, 5])
+def test_yee_schedules_equal(ctx, dtype, n, steps):
+    rng = np.random.default_rng(n)
+    f0 = rng.standard_normal(6 * (n + 1) ** 3).astype(np.float32 if dtype == capi.F32 else np.float64)
+    got, energy = [], []
+    for second in (False, True):
+        a = ctx.upload(f0)
+        b = ctx.upload(0 * f0) if second else None
+        e = np.zeros(steps)
+        which = C.c_int(0)
+        capi.check(ctx.L.scafes_yee_run(ctx.h, n, dtype, 0.5, a.ptr, b.ptr if second else None, steps, 1,
+                                        e.ctypes.data_as(C.POINTER(C.c_double)), C.byref(which)))
+        got.append((b if which.value else a).read())
+        energy.append(e)
+        a.free()
+        if second:
+            b.free()
+    assert np.array_equal(got[0], got[1])
+    # the same FP64 terms summed in another order: nodes x 2^-53 at most
+    np.testing.assert_allclose(energy[0], energy[1], rtol=6 * (n + 1) ** 3 * 2.0 ** -53)
