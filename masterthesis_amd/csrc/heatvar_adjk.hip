@@ -346,9 +346,7 @@ int heatvar_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype,
     double hh[3];
     for (int p = 0; p < 3; ++p) hh[p] = g->h[p] * g->h[p];
     cf.v.tau = tau;
-    cf.v.hh0 = hh[0];
-    cf.v.hh1 = hh[1];
-    cf.v.hh2 = hh[2];
+    cf.v.hh = make_by_hh(hh);
     cf.v.c0 = (float)(0.5 * tau / hh[0]);
     cf.v.c1 = (float)(0.5 * tau / hh[1]);
     cf.v.c2 = (float)(0.5 * tau / hh[2]);

@@ -7,10 +7,13 @@
 
 #include <hip/hip_runtime.h>
 
+#include "exact_quot.hpp"
+
 namespace scafes {
 
 struct VarCoef {
-    double tau, hh0, hh1, hh2;  // FP64 path (CPU operation order)
+    ByHH hh;                    // FP64 path (CPU operation order)
+    double tau;
     float c0, c1, c2;           // 0.5*tau/h_p^2, FP32 paths
     double border_value;
     int border_mode;
@@ -41,12 +44,10 @@ __device__ inline T var_update(const VarCoef& cf, T uc, T uw, T ue, T us, T un, 
                                T* cout)
 {
     if constexpr (MODE == 0) {
-        double v = uc;
-        v += (cf.tau * (f.e * (ue - uc) - f.w * (uc - uw))) / cf.hh0;
-        v += (cf.tau * (f.n * (un - uc) - f.s * (uc - us))) / cf.hh1;
-        v += (cf.tau * (f.u * (uu - uc) - f.d * (uc - ud))) / cf.hh2;
         *cout = T(0);
-        return (T)v;
+        return (T)add_by_hh(cf.hh, 3, uc, cf.tau * (f.e * (ue - uc) - f.w * (uc - uw)),
+                            cf.tau * (f.n * (un - uc) - f.s * (uc - us)),
+                            cf.tau * (f.u * (uu - uc) - f.d * (uc - ud)));
     } else {
         float d = cf.c0 * __builtin_fmaf(f.e, ue - uc, -(f.w * (uc - uw)));
         d = __builtin_fmaf(cf.c1, __builtin_fmaf(f.n, un - uc, -(f.s * (uc - us))), d);

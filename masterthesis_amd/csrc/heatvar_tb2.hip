@@ -870,9 +870,7 @@ int heatvar_adj2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype,
     double hh[3];
     for (int p = 0; p < 3; ++p) hh[p] = g->h[p] * g->h[p];
     cf.v.tau = tau;
-    cf.v.hh0 = hh[0];
-    cf.v.hh1 = hh[1];
-    cf.v.hh2 = hh[2];
+    cf.v.hh = make_by_hh(hh);
     cf.v.c0 = (float)(0.5 * tau / hh[0]);
     cf.v.c1 = (float)(0.5 * tau / hh[1]);
     cf.v.c2 = (float)(0.5 * tau / hh[2]);
@@ -1015,9 +1013,7 @@ int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, c
     double hh[3];
     for (int p = 0; p < 3; ++p) hh[p] = g->h[p] * g->h[p];
     cf.tau = tau;
-    cf.hh0 = hh[0];
-    cf.hh1 = hh[1];
-    cf.hh2 = hh[2];
+    cf.hh = make_by_hh(hh);
     cf.c0 = (float)(0.5 * tau / hh[0]);
     cf.c1 = (float)(0.5 * tau / hh[1]);
     cf.c2 = (float)(0.5 * tau / hh[2]);

@@ -32,6 +32,7 @@
 #include <cstdint>
 
 #include "buffer_chunk.hpp"
+#include "exact_quot.hpp"
 #include "scafes_common.hpp"
 
 namespace scafes {
@@ -41,7 +42,8 @@ namespace {
 using namespace chunk;
 
 struct AdjCoef {
-    double ctd, ctp, ta, hh0, hh1, hh2;  // FP64 path
+    ByHH hh;                             // FP64 path
+    double ctd, ctp, ta;
     float fd0, fd1, fd2, fp;             // FP32 path: ctd/h_p^2, ctp
     double a2h2, hc;                     // Tumor border: (2 h_z)/K and H (Cauchy face z = nz-1)
     float fa2h2, fhc;                    // the same rounded to FP32
@@ -58,10 +60,8 @@ template <typename T>
 __device__ inline T adj_update(const AdjCoef& cf, T c, T w_, T e, T s, T n, T d, T u, T wf)
 {
     if constexpr (sizeof(T) == 8) {
-        double v = c;
-        v += (cf.ctd * ((w_ + e) - 2.0 * c)) / cf.hh0;
-        v += (cf.ctd * ((s + n) - 2.0 * c)) / cf.hh1;
-        v += (cf.ctd * ((d + u) - 2.0 * c)) / cf.hh2;
+        double v = add_by_hh(cf.hh, 3, c, cf.ctd * ((w_ + e) - 2.0 * c), cf.ctd * ((s + n) - 2.0 * c),
+                             cf.ctd * ((d + u) - 2.0 * c));
         v -= (cf.ctp * wf) * c;
         return v;
     } else {
@@ -99,10 +99,7 @@ __device__ inline T adj_update_tumor(const AdjCoef& cf, const Geo& g, int i, int
     const T t1 = tumor_t<T>(j, g.ny, false, T(0), s, n, c);
     if constexpr (sizeof(T) == 8) {
         const T t2 = tumor_t<T>(k, g.nz, true, cf.a2h2 * cf.hc, d, u, c);
-        double v = c;
-        v += (cf.ctd * t0) / cf.hh0;
-        v += (cf.ctd * t1) / cf.hh1;
-        v += (cf.ctd * t2) / cf.hh2;
+        double v = add_by_hh(cf.hh, 3, c, cf.ctd * t0, cf.ctd * t1, cf.ctd * t2);
         v -= (cf.ctp * wf) * c;
         return v;
     } else {
@@ -411,9 +408,7 @@ int pennes_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
     cf.ctd = p->tau * p->cdiff;
     cf.ctp = p->tau * p->cperf;
     cf.ta = p->t_a;
-    cf.hh0 = hh[0];
-    cf.hh1 = hh[1];
-    cf.hh2 = hh[2];
+    cf.hh = make_by_hh(hh);
     cf.fd0 = (float)(cf.ctd / hh[0]);
     cf.fd1 = (float)(cf.ctd / hh[1]);
     cf.fd2 = (float)(cf.ctd / hh[2]);

@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "exact_quot.hpp"
 #include "heatvar_ops.hpp"
 #include "scafes_common.hpp"
 
@@ -176,7 +177,8 @@ struct HeatConstOp {
     const double* g_old;
     const double* g_new;
     Geo gk;  // layout of the stencil-0 known fields
-    double ctau_a, ctw, ctf, hh0, hh1, hh2, border_value;
+    ByHH hh;
+    double ctau_a, ctw, ctf, border_value;
     double a2[3], alpha, epsilon, sigma;  // flux borders: a2[p] = 2 h_p / lambda
     int has_perf, has_source, border_mode;
     // Second difference along one axis at a flux border node: the outer
@@ -200,10 +202,8 @@ struct HeatConstOp {
     {
         const long m = at(g, i, j, k);
         if (!is_border(g, i, j, k)) {
-            double v = s.c;
-            v += (ctau_a * ((s.w + s.e) - 2.0 * s.c)) / hh0;
-            if (g.dim > 1) v += (ctau_a * ((s.s + s.n) - 2.0 * s.c)) / hh1;
-            if (g.dim > 2) v += (ctau_a * ((s.d + s.u) - 2.0 * s.c)) / hh2;
+            double v = add_by_hh(hh, g.dim, s.c, ctau_a * ((s.w + s.e) - 2.0 * s.c),
+                                 ctau_a * ((s.s + s.n) - 2.0 * s.c), ctau_a * ((s.d + s.u) - 2.0 * s.c));
             if (has_perf) v -= ctw * s.c;
             if (has_source) v += ctf * f_old[at(gk, i, j, k)];
             out[m] = v;
@@ -219,11 +219,11 @@ struct HeatConstOp {
             }
             const double gold = g_old[q];
             double v = s.c;
-            v += (ctau_a * (i == g.nx - 1 ? flux_diff(s.w, s.c, a2[0], gold) : (s.w + s.e) - 2.0 * s.c)) / hh0;
+            v += (ctau_a * (i == g.nx - 1 ? flux_diff(s.w, s.c, a2[0], gold) : (s.w + s.e) - 2.0 * s.c)) / hh.d[0];
             if (g.dim > 1)
-                v += (ctau_a * (j == g.ny - 1 ? flux_diff(s.s, s.c, a2[1], gold) : (s.s + s.n) - 2.0 * s.c)) / hh1;
+                v += (ctau_a * (j == g.ny - 1 ? flux_diff(s.s, s.c, a2[1], gold) : (s.s + s.n) - 2.0 * s.c)) / hh.d[1];
             if (g.dim > 2)
-                v += (ctau_a * (k == g.nz - 1 ? flux_diff(s.d, s.c, a2[2], gold) : (s.d + s.u) - 2.0 * s.c)) / hh2;
+                v += (ctau_a * (k == g.nz - 1 ? flux_diff(s.d, s.c, a2[2], gold) : (s.d + s.u) - 2.0 * s.c)) / hh.d[2];
             if (has_perf) v -= ctw * s.c;
             if (has_source) v += ctf * f_old[q];
             out[m] = v;
@@ -247,7 +247,8 @@ struct HeatVarOp {
     const T* x[1];  // x[0] = incoming compensation (Kahan mode)
     T* out;
     T* cout;
-    double tau, hh0, hh1, hh2;  // FP64 path
+    ByHH hh;                    // FP64 path
+    double tau;
     float c0, c1, c2;           // 0.5*tau/h_p^2 for the FP32 paths
     T border_value;
     int border_mode;
@@ -257,13 +258,10 @@ struct HeatVarOp {
         const long m = at(g, i, j, k);
         if (!is_border(g, i, j, k)) {
             if constexpr (MODE == 0) {
-                double v = s.c;
-                v += (tau * (0.5 * (q.e + q.c) * (s.e - s.c) - 0.5 * (q.c + q.w) * (s.c - s.w))) / hh0;
-                if (g.dim > 1)
-                    v += (tau * (0.5 * (q.n + q.c) * (s.n - s.c) - 0.5 * (q.c + q.s) * (s.c - s.s))) / hh1;
-                if (g.dim > 2)
-                    v += (tau * (0.5 * (q.u + q.c) * (s.u - s.c) - 0.5 * (q.c + q.d) * (s.c - s.d))) / hh2;
-                out[m] = v;
+                out[m] = add_by_hh(hh, g.dim, s.c,
+                                   tau * (0.5 * (q.e + q.c) * (s.e - s.c) - 0.5 * (q.c + q.w) * (s.c - s.w)),
+                                   tau * (0.5 * (q.n + q.c) * (s.n - s.c) - 0.5 * (q.c + q.s) * (s.c - s.s)),
+                                   tau * (0.5 * (q.u + q.c) * (s.u - s.c) - 0.5 * (q.c + q.d) * (s.c - s.d)));
             } else {
                 float d = c0 * __builtin_fmaf(q.e + q.c, s.e - s.c, -((q.c + q.w) * (s.c - s.w)));
                 if (g.dim > 1)
@@ -301,9 +299,10 @@ struct PennesOp {
     const T* x[3];  // perfusion w, source Q, incoming compensation (KAHAN)
     T* out;
     T* cout;
-    double ctd, ctp, ctq, ta, hh0, hh1, hh2;  // FP64 path
-    float fd0, fd1, fd2, fp, fq, fta;         // FP32 path
-    int tumor;                                // border rule of the Tumor example
+    ByHH hh;                           // FP64 path
+    double ctd, ctp, ctq, ta;
+    float fd0, fd1, fd2, fp, fq, fta;  // FP32 path
+    int tumor;                         // border rule of the Tumor example
     double a2h[3], hconv, tinf, qbc;          // (2 h_p)/K, H, T_INF, Q_BC
     // One axis of TumorHeatEqnFDM::updateBorder (TumorHeatEqnFDM.hpp:300-345):
     // the missing neighbour replaced by the inner one plus a flux term.
@@ -334,10 +333,7 @@ struct PennesOp {
             const T t1 = g.dim > 1 ? tumor_term(j, g.ny, g.dim == 2, 1, s.s, s.n, s.c) : (T)0;
             const T t2 = g.dim > 2 ? tumor_term(k, g.nz, true, 2, s.d, s.u, s.c) : (T)0;
             if constexpr (sizeof(T) == 8) {
-                double v = s.c;
-                v += (ctd * t0) / hh0;
-                if (g.dim > 1) v += (ctd * t1) / hh1;
-                if (g.dim > 2) v += (ctd * t2) / hh2;
+                double v = add_by_hh(hh, g.dim, s.c, ctd * t0, ctd * t1, ctd * t2);
                 v += (ctp * xv[0]) * (ta - s.c);
                 v += ctq * xv[1];
                 out[m] = v;
@@ -359,10 +355,8 @@ struct PennesOp {
             return;
         }
         if constexpr (sizeof(T) == 8) {
-            double v = s.c;
-            v += (ctd * ((s.w + s.e) - 2.0 * s.c)) / hh0;
-            if (g.dim > 1) v += (ctd * ((s.s + s.n) - 2.0 * s.c)) / hh1;
-            if (g.dim > 2) v += (ctd * ((s.d + s.u) - 2.0 * s.c)) / hh2;
+            double v = add_by_hh(hh, g.dim, s.c, ctd * ((s.w + s.e) - 2.0 * s.c), ctd * ((s.s + s.n) - 2.0 * s.c),
+                                 ctd * ((s.d + s.u) - 2.0 * s.c));
             v += (ctp * xv[0]) * (ta - s.c);
             v += ctq * xv[1];
             out[m] = v;
@@ -408,7 +402,8 @@ struct MriOp {
     const double* lam;   // lambda, layout gk
     const double* surf;  // surface flag, layout gk
     Geo gk;
-    double hh0, hh1, hh2, h[3];
+    ByHH hh;
+    double h[3];
     double hconv, tamb, qbc, qskull, epsilon, sigma, tamb4;  // tamb4 = (T_AMB + 273.15)^4
     // One axis of updateBorder (MRIDataPBHEqnFDM.hpp:193-262): the missing
     // neighbour replaced by the inner one plus the face's flux term.  On the
@@ -441,15 +436,14 @@ struct MriOp {
         const long m = at(g, i, j, k);
         double v = s.c;
         if (!is_border(g, i, j, k)) {
-            v += (xv[0] * ((s.w + s.e) - 2.0 * s.c)) / hh0;
-            if (g.dim > 1) v += (xv[0] * ((s.s + s.n) - 2.0 * s.c)) / hh1;
-            if (g.dim > 2) v += (xv[0] * ((s.d + s.u) - 2.0 * s.c)) / hh2;
+            v = add_by_hh(hh, g.dim, v, xv[0] * ((s.w + s.e) - 2.0 * s.c), xv[0] * ((s.s + s.n) - 2.0 * s.c),
+                          xv[0] * ((s.d + s.u) - 2.0 * s.c));
         } else {
             const long q = at(gk, i, j, k);
             const double kk = lam[q];
-            v += (xv[0] * term(i, g.nx, g.dim == 1, h[0], kk, s.w, s.e, s.c, v, q)) / hh0;
-            if (g.dim > 1) v += (xv[0] * term(j, g.ny, g.dim == 2, h[1], kk, s.s, s.n, s.c, v, q)) / hh1;
-            if (g.dim > 2) v += (xv[0] * term(k, g.nz, true, h[2], kk, s.d, s.u, s.c, v, q)) / hh2;
+            v += (xv[0] * term(i, g.nx, g.dim == 1, h[0], kk, s.w, s.e, s.c, v, q)) / hh.d[0];
+            if (g.dim > 1) v += (xv[0] * term(j, g.ny, g.dim == 2, h[1], kk, s.s, s.n, s.c, v, q)) / hh.d[1];
+            if (g.dim > 2) v += (xv[0] * term(k, g.nz, true, h[2], kk, s.d, s.u, s.c, v, q)) / hh.d[2];
         }
         v += xv[1] * (xv[2] - s.c);
         v += xv[3];
@@ -500,7 +494,8 @@ struct HeatVarAdjOp {
     const T* x[1];
     T* out;       // lam^{n-1}
     double* grad;
-    double tau, hh0, hh1, hh2, th0, th1, th2;  // th_p = tau / hh_p
+    ByHH hh;
+    double tau, th0, th1, th2;                 // th_p = tau / hh_p
     float c0, c1, c2;                          // 0.5*tau/h_p^2 (FP32 update)
     float f0, f1, f2;                          // 0.5 th_p rounded to FP32 (FP32 gradient terms)
     __device__ static double face_sum(bool lo, bool hi, double lc, double lm, double lp, double uc, double um,
@@ -539,11 +534,10 @@ struct HeatVarAdjOp {
             return;
         }
         if constexpr (sizeof(T) == 8) {
-            double v = l.c;
-            v += (tau * (0.5 * (q.e + q.c) * (l.e - l.c) - 0.5 * (q.c + q.w) * (l.c - l.w))) / hh0;
-            if (g.dim > 1) v += (tau * (0.5 * (q.n + q.c) * (l.n - l.c) - 0.5 * (q.c + q.s) * (l.c - l.s))) / hh1;
-            if (g.dim > 2) v += (tau * (0.5 * (q.u + q.c) * (l.u - l.c) - 0.5 * (q.c + q.d) * (l.c - l.d))) / hh2;
-            out[m] = v;
+            out[m] = add_by_hh(hh, g.dim, l.c,
+                               tau * (0.5 * (q.e + q.c) * (l.e - l.c) - 0.5 * (q.c + q.w) * (l.c - l.w)),
+                               tau * (0.5 * (q.n + q.c) * (l.n - l.c) - 0.5 * (q.c + q.s) * (l.c - l.s)),
+                               tau * (0.5 * (q.u + q.c) * (l.u - l.c) - 0.5 * (q.c + q.d) * (l.c - l.d)));
         } else {
             float d = c0 * __builtin_fmaf(q.e + q.c, l.e - l.c, -((q.c + q.w) * (l.c - l.w)));
             if (g.dim > 1) d = __builtin_fmaf(c1, __builtin_fmaf(q.n + q.c, l.n - l.c, -((q.c + q.s) * (l.c - l.s))), d);
@@ -566,7 +560,8 @@ struct PennesAdjOp {
     const T* x[3];  // perfusion w, previous forward state T^{n-1} (hi, lo)
     T* out;         // lambda^{n-1}
     double* grad;
-    double ctd, ctp, ta, hh0, hh1, hh2;
+    ByHH hh;
+    double ctd, ctp, ta;
     float fd0, fd1, fd2, fp;
     int tumor;                   // the Tumor border rule (every node updated)
     double a2h[3], hconv;        // (2 h_p)/K, H
@@ -601,10 +596,8 @@ struct PennesAdjOp {
         if constexpr (LO) tp += (double)xv[2];
         grad[m] += (double)s.c * (ctp * (ta - tp));
         if constexpr (sizeof(T) == 8) {
-            double v = s.c;
-            v += (ctd * ((s.w + s.e) - 2.0 * s.c)) / hh0;
-            if (g.dim > 1) v += (ctd * ((s.s + s.n) - 2.0 * s.c)) / hh1;
-            if (g.dim > 2) v += (ctd * ((s.d + s.u) - 2.0 * s.c)) / hh2;
+            double v = add_by_hh(hh, g.dim, s.c, ctd * ((s.w + s.e) - 2.0 * s.c), ctd * ((s.s + s.n) - 2.0 * s.c),
+                                 ctd * ((s.d + s.u) - 2.0 * s.c));
             v -= (ctp * xv[0]) * s.c;
             out[m] = v;
         } else {
@@ -624,10 +617,7 @@ struct PennesAdjOp {
         const T t1 = g.dim > 1 ? tumor_adj(j, g.ny, g.dim == 2, 1, s.s, s.n, s.c) : T(0);
         const T t2 = g.dim > 2 ? tumor_adj(k, g.nz, true, 2, s.d, s.u, s.c) : T(0);
         if constexpr (sizeof(T) == 8) {
-            double v = s.c;
-            v += (ctd * t0) / hh0;
-            if (g.dim > 1) v += (ctd * t1) / hh1;
-            if (g.dim > 2) v += (ctd * t2) / hh2;
+            double v = add_by_hh(hh, g.dim, s.c, ctd * t0, ctd * t1, ctd * t2);
             v -= (ctp * xv[0]) * s.c;
             out[m] = v;
         } else {
@@ -762,9 +752,7 @@ int heat7var_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, cons
         op.b = (const double*)kap;
         op.out = (double*)un;
         op.tau = tau;
-        op.hh0 = hh[0];
-        op.hh1 = hh[1];
-        op.hh2 = hh[2];
+        op.hh = make_by_hh(hh);
         op.border_value = border_value;
         op.border_mode = border_mode;
         return launch<HeatVarOp<double, 0>, double>(c, op, geo, cfg);
@@ -824,9 +812,7 @@ int pennes_step_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
         op.ctp = p->tau * p->cperf;
         op.ctq = p->tau * p->csrc;
         op.ta = p->t_a;
-        op.hh0 = hh[0];
-        op.hh1 = hh[1];
-        op.hh2 = hh[2];
+        op.hh = make_by_hh(hh);
         if (p->border_mode == SCAFES_BORDER_TUMOR) tumor(op);
         return launch<PennesOp<double>, double>(c, op, geo, -1);
     }
@@ -880,9 +866,7 @@ int heatvar_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
     hh_of(g, hh);
     auto fill = [&](auto& op) {
         op.tau = tau;
-        op.hh0 = hh[0];
-        op.hh1 = hh[1];
-        op.hh2 = hh[2];
+        op.hh = make_by_hh(hh);
         op.th0 = tau / hh[0];
         op.th1 = tau / hh[1];
         op.th2 = tau / hh[2];
@@ -937,9 +921,7 @@ int pennes_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, c
         op.ctd = p->tau * p->cdiff;
         op.ctp = p->tau * p->cperf;
         op.ta = p->t_a;
-        op.hh0 = hh[0];
-        op.hh1 = hh[1];
-        op.hh2 = hh[2];
+        op.hh = make_by_hh(hh);
         tumor(op);
         return launch<PennesAdjOp<double>, double>(c, op, geo, -1);
     }
@@ -1072,9 +1054,7 @@ static int heat7_const_op(Ctx* c, const scafes_geom* g, int hw, const double* u_
     op->ctau_a = p->tau * p->coeff_a;
     op->ctw = (p->tau * p->perf_c) * p->perf_w;
     op->ctf = p->tau * p->rhoc_inv;
-    op->hh0 = hh[0];
-    op->hh1 = hh[1];
-    op->hh2 = hh[2];
+    op->hh = make_by_hh(hh);
     op->has_perf = p->has_perf;
     op->has_source = p->has_source;
     op->border_mode = p->border_mode;
@@ -1457,9 +1437,7 @@ int scafes_mri_step_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, const dou
     op.lam = mat[SCAFES_MRI_LAMBDA];
     op.surf = mat[SCAFES_MRI_SURFACE];
     op.gk = gk;
-    op.hh0 = hh[0];
-    op.hh1 = hh[1];
-    op.hh2 = hh[2];
+    op.hh = make_by_hh(hh);
     for (int q = 0; q < 3; ++q) op.h[q] = q < g->dim ? g->h[q] : 1.0;
     op.hconv = p->h_conv;
     op.tamb = p->t_amb;
