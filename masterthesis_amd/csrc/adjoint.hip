@@ -234,7 +234,7 @@ struct Rev {
         lam_ready = true;
         return SCAFES_OK;
     }
-    // Reverse steps the next sweep takes when `left` (>= 2) remain with
+    // Reverse steps the next sweep takes when `left` (>= 1) remain with
     // their states at hand: as many as the kernel allows, but one fewer where
     // that would leave a single step (a one-step launch costs about two steps
     // of a multi-step sweep), so 5 -> 3 + 2 instead of 4 + 1.
@@ -242,7 +242,7 @@ struct Rev {
     {
         int kmax;
         if (family == FAMILY_HEATVAR)
-            kmax = heatvar_adjk_supported(geo) ? heatvar_adjk_max(lam_dtype) : 2;
+            kmax = heatvar_adjk_supported(geo) ? heatvar_adjk_max(lam_dtype) : lam_dtype == SCAFES_F64 ? 1 : 2;
         else
             kmax = pennes_adjk_max(lam_dtype, p && p->border_mode == SCAFES_BORDER_TUMOR);
         int K = (int)std::min<long>(kmax, left);
@@ -401,11 +401,11 @@ struct Rev {
                 r = first_leaf(chain[n - 1 - a]);
                 if (r) break;
             }
-            if (n - a < 2) {
+            const int K = sweep_k(n - a);
+            if (K == 1) {
                 r = adjoint((int)n, chain[n - 1 - a]);
                 n -= 1;
             } else {
-                const int K = sweep_k(n - a);
                 const void* sk[kAdjMaxK];
                 for (int l = 0; l < K; ++l) sk[l] = chain[n - 1 - l - a];
                 r = adjointk(K, sk);
@@ -473,11 +473,11 @@ int Rev::treeverse(long a, long b, int s, const void* base)
                     r = first_leaf(st[n - 1 - a]);
                     if (r) break;
                 }
-                if (n - a < 2) {
+                const int K = sweep_k(n - a);
+                if (K == 1) {
                     r = adjoint((int)n, st[n - 1 - a]);
                     n -= 1;
                 } else {
-                    const int K = sweep_k(n - a);
                     const void* sk[kAdjMaxK];
                     for (int l = 0; l < K; ++l) sk[l] = st[n - 1 - l - a];
                     r = adjointk(K, sk);

@@ -263,10 +263,10 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
     }
 }
 
-// Tile: 64 x 16 threads, prefetch depth 2, 64-plane z chunks for FP32 (the
+// Tile: 64 x 16 threads, prefetch depth 2, 64-plane z chunks (the
 // 20-step gradient at 512^3 with every state stored: 18.9-19.4 ms with 64-
 // and 128-plane chunks, 19.5-19.9 with 48 and 96, 19.6-19.9 with 32, 20.9-21.4
-// with 16), 32 for FP64.  Measured on
+// with 16).  Measured on
 // an MI355X (512^3 FP32 + Kahan, 20 steps store-all, whole gradient in ms):
 // K <= 4 64x16 24.0, 64x12 27.9; K <= 3 64x12 24.6, 64x16 25.2; K = 2
 // 64x8 24.5, 64x16 24.1; the two-step kernel of heatvar_tb2.hip 25.0.
@@ -275,18 +275,18 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
 // chunks) and still needs 123 VGPRs: one workgroup per CU, bound by vector
 // issue (0.60 of its rate), not by HBM (0.41 of 8 TB/s).  Two 12-wave workgroups per CU would need
 // at most 80 VGPRs.
-// FP64 fields: 64 x 8 (a 1024-thread workgroup caps a thread at 128 VGPRs,
-// which the FP64 rings exceed), and two steps per sweep only: on 64 x 8 each
-// further step costs two more of the eight rows (us per reverse step at 128^3
-// / 200^3: K = 2 33 / 100, K = 3 37 / 133, K = 4 60 / 222).
+// FP64 fields take one reverse step per launch: a 1024-thread workgroup caps a
+// thread at 128 VGPRs, which the FP64 rings exceed, and on 64 x 8 each step
+// costs two of the eight rows (us per reverse step at 128^3: K = 2 33, K = 3
+// 37, K = 4 60, the one-step row kernel 21; the 30-step gradient with every
+// state stored 5407 us with K = 2, 4843 with single steps, 256^3 48.6 and 47.8 ms).
 // Grids with fewer workgroups than CUs at the full chunk take shorter ones
 // (fit_chunk): K = 4 FP32 at 97x80x75 123 -> 24 us per sweep, 128^3 127 -> 57.
 // FP32, K = 3: 64 x 12 (64 x 16 caps a thread at 128 VGPRs, which the
 // three-step rings exceed by a 16-byte spill).
 template <typename T, int K>
 struct AdjkTile {
-    static constexpr int TX = 64, TY = sizeof(T) == 8 ? 8 : (K == 3 ? 12 : 16), D = 2, ZC = sizeof(T) == 8 ? 32 : 64,
-                         PER_CU = 1;
+    static constexpr int TX = 64, TY = K == 3 ? 12 : 16, D = 2, ZC = 64, PER_CU = 1;
 };
 
 template <typename T, int K>
@@ -310,10 +310,8 @@ int adjk_launch_k(Ctx* c, const Geo& g, int K, const void* lam, void* lamo, cons
                   double* grad, const AdjVarCoef& cf)
 {
     if (K == 2) return adjk_launch_t<T, 2>(c, g, lam, lamo, kap, st, grad, cf);
-    if constexpr (sizeof(T) == 4) {
-        if (K == 3) return adjk_launch_t<T, 3>(c, g, lam, lamo, kap, st, grad, cf);
-        if (K == 4) return adjk_launch_t<T, 4>(c, g, lam, lamo, kap, st, grad, cf);
-    }
+    if (K == 3) return adjk_launch_t<T, 3>(c, g, lam, lamo, kap, st, grad, cf);
+    if (K == 4) return adjk_launch_t<T, 4>(c, g, lam, lamo, kap, st, grad, cf);
     return fail(SCAFES_ERR_ARG, "multi-step var-kappa adjoint: K out of range");
 }
 
@@ -328,7 +326,7 @@ bool heatvar_adjk_supported(const Geo& geo)
     return geo.dim == 3 && (kPlanes * geo.e01 + geo.base + geo.e01) * 8L < (long)kRecords;
 }
 
-int heatvar_adjk_max(int dtype) { return dtype == SCAFES_F64 ? 2 : kAdjMaxK; }
+int heatvar_adjk_max(int dtype) { return dtype == SCAFES_F64 ? 1 : kAdjMaxK; }
 
 int heatvar_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, int K, const void* lam,
                         void* lamo, const void* kap, const void* const* u, double* grad, double tau)
@@ -358,7 +356,6 @@ int heatvar_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype,
     cf.f0 = (float)(0.5 * cf.th0);
     cf.f1 = (float)(0.5 * cf.th1);
     cf.f2 = (float)(0.5 * cf.th2);
-    if (dtype == SCAFES_F64) return adjk_launch_k<double>(c, geo, K, lam, lamo, kap, st, grad, cf);
     return adjk_launch_k<float>(c, geo, K, lam, lamo, kap, st, grad, cf);
 }
 

@@ -833,13 +833,14 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
     }
 }
 
-// 64 x 8 threads, two planes in flight; FP32 64-plane z chunks, FP64 32.
+// 64 x 8 threads, two planes in flight, 64-plane z chunks (FP32 fields; FP64
+// takes one reverse step per launch).
 // Measured at 512^3 FP32 on an MI355X (us per two-step launch): 64x8 with
 // 64-plane chunks 1372, with 32 1395; 64x16 with 64 1408, with 32 1461;
 // 64x12 with 32 1724 (the results are bit-identical across tiles).
 template <typename T>
 struct Adj2Tile {
-    static constexpr int TX = 64, TY = 8, D = 2, ZC = sizeof(T) == 4 ? 64 : 32;
+    static constexpr int TX = 64, TY = 8, D = 2, ZC = 64;
 };
 
 // 3-D grids whose in-plane byte offsets of the FP64 gradient fit 32 bits.
@@ -882,7 +883,7 @@ int heatvar_adj2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype,
     cf.f0 = (float)(0.5 * cf.th0);
     cf.f1 = (float)(0.5 * cf.th1);
     cf.f2 = (float)(0.5 * cf.th2);
-    if (dtype == SCAFES_F64) return adj2_launch_t<double>(c, geo, lam, lamo, kap, u1, u2, grad, cf);
+    if (dtype == SCAFES_F64) return fail(SCAFES_ERR_UNSUPPORTED, "FP64 kappa adjoints take one step per launch");
     return adj2_launch_t<float>(c, geo, lam, lamo, kap, u1, u2, grad, cf);
 }
 

@@ -1,6 +1,9 @@
-// stencil3d.hip -- 2.5D z-streaming 7-point stencil kernels for gfx950.
+// stencil3d.hip -- 7-point stencil kernels for gfx950, one step per launch.
 //
-// One workgroup owns a TX x TY tile of an xy plane and walks a chunk of z
+// row_kernel (below stream_kernel) carries every update that names no tile:
+// 16 bytes of a row per thread, neighbours through the caches.  stream_kernel
+// is the 2.5D z-streaming form of the var-kappa update's tiles, which are
+// chosen by index or by the autotuner: one workgroup owns a TX x TY tile of an xy plane and walks a chunk of z
 // planes.  The centre column of the stencil field lives in a 3-deep
 // register queue (z-1, z, z+1); the current xy plane plus a one-node halo
 // is staged in LDS (double buffered, one barrier per plane), so every
@@ -8,8 +11,8 @@
 // halo, which neighbouring tiles on the same XCD bring into L2.  Tiles
 // are mapped XCD-contiguously (xcd_remap).
 //
-// Kernels never read ghost layers: every coordinate is clamped to the node
-// range, and only GLOBAL_INNER nodes (whose neighbours are nodes) use
+// Ghost values never enter a result: y and z coordinates are clamped to the
+// node range, x windows may read a ghost node, and only GLOBAL_INNER nodes (whose neighbours are nodes) use
 // neighbour values.  Ghost layers of the output are never written.
 //
 // Replaces the OpenMP node loop evalTypeTwoAt (src/ScaFES_Problem.hpp:5397-5476),
@@ -31,6 +34,12 @@ struct St7 {
     T c, w, e, s, n, d, u;  // centre, x-, x+, y-, y+, z-, z+
 };
 
+template <typename T>
+struct Res {
+    T v, c;
+    double g;
+};
+
 // ---------------------------------------------------------------- skeleton
 // D = prefetch depth in planes (even, >= 2).  Every value a thread needs for
 // plane k (its centre, the halo value it stages for the tile, and the
@@ -38,7 +47,9 @@ struct St7 {
 // ring, so each plane's barrier waits on loads issued D iterations before.
 // Op interface: kTwo (second stencil field b, e.g. kappa), kThree (third
 // stencil field c, with kTwo), kNX centre-only fields x[0..kNX-1] of type T,
-// apply(g, i, j, k, a7, b7, c7, xv).
+// apply(g, i, j, k, a7, b7, c7, xv, res): the node's new value res.v, its new
+// compensation res.c (kComp) and the increment res.g of the FP64 gradient
+// (kGrad), which the kernel stores.
 template <class Op, typename T, int TX, int TY, int D>
 __global__ __launch_bounds__(TX* TY) void stream_kernel(Op op, Geo g, int zc, int tiles_x,
                                                          int tiles_y)
@@ -151,12 +162,153 @@ __global__ __launch_bounds__(TX* TY) void stream_kernel(Op op, Geo g, int zc, in
                 if constexpr (THREE)
                     sC = St7<T>{cc, sc[buf][ty + 1][tx], sc[buf][ty + 1][tx + 2], sc[buf][ty][tx + 1],
                                 sc[buf][ty + 2][tx + 1], cm, cp};
-                op.apply(g, i, j, k, sA, sB, sC, xv);
+                const long m = oc + g.e01 * k;
+                Res<T> res{};
+                op.apply(g, i, j, k, sA, sB, sC, xv, res);
+                op.out[m] = res.v;
+                if constexpr (Op::kComp) op.cout[m] = res.c;
+                if constexpr (Op::kGrad) op.grad[m] += res.g;
             }
             am = ac;
             bm = bc;
             cm = cc;
         }
+    }
+}
+
+// ---------------------------------------------------------------- rows
+// One step without LDS or barriers: a thread owns V consecutive nodes of a
+// row (16 bytes) and walks zc planes.  Per plane it loads its window of V + 2
+// nodes of the next plane (the x neighbours ride along), the two y neighbour
+// vectors and the centre-only fields, all 16-byte accesses of which the
+// neighbour rows hit the L1, one plane ahead of their use; the z neighbours
+// stay in registers.  The last thread of a row shifts its window back into
+// the row and stores only the nodes it owns.  Windows reach one ghost node to
+// either side (hw >= 1); y and z neighbours are clamped to the node range.
+template <typename T, int V>
+struct VecOf {
+    typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+};
+
+template <class Op, typename T>
+__global__ __launch_bounds__(256) void row_kernel(Op op, Geo g, int zc, int cpr, int blocks_xy)
+{
+    constexpr int V = 16 / (int)sizeof(T);
+    constexpr int NF = Op::kThree ? 3 : Op::kTwo ? 2 : 1;
+    constexpr int NX = Op::kNX;
+    constexpr int NXA = NX > 0 ? NX : 1;
+    typedef typename VecOf<T, V>::type vec;
+    typedef typename VecOf<T, 2>::type vec2;
+    typedef typename VecOf<double, V>::type dvec;
+    const int lb = xcd_remap(blockIdx.x, gridDim.x);
+    const int tz = lb / blocks_xy;
+    const int idx = (lb - tz * blocks_xy) * 256 + (int)threadIdx.x;
+    const int j = idx / cpr;
+    if (j >= g.ny) return;
+    const int i0 = (idx - j * cpr) * V;
+    const int is = min(i0, g.nx - V);
+    const int skip = i0 - is;  // window nodes that belong to the thread before
+    const int k0 = tz * zc, k1 = min(k0 + zc, g.nz);
+    const long o = at(g, is, j, 0);
+    const long os = j > 0 ? o - g.e0 : o, on = j < g.ny - 1 ? o + g.e0 : o;
+    const T* __restrict__ F[3] = {op.a, op.b, op.c3};
+    const T* __restrict__ X[NXA];
+#pragma unroll
+    for (int x = 0; x < NX; ++x) X[x] = op.x[x];
+
+    struct Win {
+        T v[V + 2];
+    };
+    auto window = [&](const T* p, const int k) {
+        Win w;
+        const T* q = p + o + g.e01 * min(k, g.nz - 1) - 1;
+        const vec lo = *(const vec*)q;
+        const vec2 hi = *(const vec2*)(q + V);
+#pragma unroll
+        for (int x = 0; x < V; ++x) w.v[x] = lo[x];
+        w.v[V] = hi[0];
+        w.v[V + 1] = hi[1];
+        return w;
+    };
+    struct Side {
+        vec s[3], n[3], x[NXA];
+    };
+    auto sides = [&](const int k) {
+        Side r;
+        const long z = g.e01 * min(k, g.nz - 1);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            r.s[f] = *(const vec*)(F[f] + os + z);
+            r.n[f] = *(const vec*)(F[f] + on + z);
+        }
+#pragma unroll
+        for (int x = 0; x < NX; ++x) r.x[x] = *(const vec*)(X[x] + o + z);
+        return r;
+    };
+
+    vec dn[3];
+    Win cur[3], up[3];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        dn[f] = *(const vec*)(F[f] + o + g.e01 * max(k0 - 1, 0));
+        cur[f] = window(F[f], k0);
+        up[f] = window(F[f], k0 + 1);
+    }
+    Side sd = sides(k0);
+    for (int k = k0; k < k1; ++k) {
+        Win up2[3];
+        Side sd2 = sd;
+        if (k + 1 < k1) {  // uniform over the launch's chunk
+#pragma unroll
+            for (int f = 0; f < NF; ++f) up2[f] = window(F[f], k + 2);
+            sd2 = sides(k + 1);
+        } else {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) up2[f] = up[f];
+        }
+        const long m = o + g.e01 * k;
+        vec rv, rc;
+#pragma unroll
+        for (int x = 0; x < V; ++x) rc[x] = T(0);
+        dvec rg;
+        if constexpr (Op::kGrad) rg = *(const dvec*)(op.grad + m);
+#pragma unroll
+        for (int x = 0; x < V; ++x) {
+            St7<T> st[3] = {};
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+                st[f] = St7<T>{cur[f].v[x + 1], cur[f].v[x], cur[f].v[x + 2], sd.s[f][x],
+                               sd.n[f][x],      dn[f][x],    up[f].v[x + 1]};
+            T xv[NXA];
+#pragma unroll
+            for (int q = 0; q < NX; ++q) xv[q] = sd.x[q][x];
+            Res<T> res{};
+            op.apply(g, is + x, j, k, st[0], st[1], st[2], xv, res);
+            rv[x] = res.v;
+            if constexpr (Op::kComp) rc[x] = res.c;
+            if constexpr (Op::kGrad) rg[x] += res.g;
+        }
+        if (skip == 0) {
+            *(vec*)(op.out + m) = rv;
+            if constexpr (Op::kComp) *(vec*)(op.cout + m) = rc;
+            if constexpr (Op::kGrad) *(dvec*)(op.grad + m) = rg;
+        } else {
+#pragma unroll
+            for (int x = 1; x < V; ++x) {
+                if (x < skip) continue;
+                op.out[m + x] = rv[x];
+                if constexpr (Op::kComp) op.cout[m + x] = rc[x];
+                if constexpr (Op::kGrad) op.grad[m + x] = rg[x];
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+#pragma unroll
+            for (int x = 0; x < V; ++x) dn[f][x] = cur[f].v[x + 1];
+            cur[f] = up[f];
+            up[f] = up2[f];
+        }
+        sd = sd2;
     }
 }
 
@@ -168,6 +320,7 @@ struct HeatConstOp {
     static constexpr bool kTwo = false;
     static constexpr bool kThree = false;
     static constexpr int kNX = 0;
+    static constexpr bool kComp = false, kGrad = false;
     const double* a;
     const double* b;
     const double* c3;
@@ -198,23 +351,22 @@ struct HeatConstOp {
         return t - 2.0 * u;
     }
     __device__ void apply(const Geo& g, int i, int j, int k, const St7<double>& s,
-                          const St7<double>&, const St7<double>&, const double*) const
+                          const St7<double>&, const St7<double>&, const double*, Res<double>& r) const
     {
-        const long m = at(g, i, j, k);
         if (!is_border(g, i, j, k)) {
             double v = add_by_hh(hh, g.dim, s.c, ctau_a * ((s.w + s.e) - 2.0 * s.c),
                                  ctau_a * ((s.s + s.n) - 2.0 * s.c), ctau_a * ((s.d + s.u) - 2.0 * s.c));
             if (has_perf) v -= ctw * s.c;
             if (has_source) v += ctf * f_old[at(gk, i, j, k)];
-            out[m] = v;
+            r.v = v;
         } else if (border_mode == SCAFES_BORDER_FIELD) {
-            out[m] = g_new[at(gk, i, j, k)];
+            r.v = g_new[at(gk, i, j, k)];
         } else if (border_mode == SCAFES_BORDER_VALUE) {
-            out[m] = border_value;
+            r.v = border_value;
         } else if (border_mode >= SCAFES_BORDER_NEUMANN) {
             const long q = at(gk, i, j, k);
             if (i == 0 || (g.dim > 1 && j == 0) || (g.dim > 2 && k == 0)) {
-                out[m] = g_new[q];
+                r.v = g_new[q];
                 return;
             }
             const double gold = g_old[q];
@@ -226,9 +378,9 @@ struct HeatConstOp {
                 v += (ctau_a * (k == g.nz - 1 ? flux_diff(s.d, s.c, a2[2], gold) : (s.d + s.u) - 2.0 * s.c)) / hh.d[2];
             if (has_perf) v -= ctw * s.c;
             if (has_source) v += ctf * f_old[q];
-            out[m] = v;
+            r.v = v;
         } else {
-            out[m] = s.c;
+            r.v = s.c;
         }
     }
 };
@@ -241,6 +393,7 @@ struct HeatVarOp {
     static constexpr bool kTwo = true;
     static constexpr bool kThree = false;
     static constexpr int kNX = MODE == 2 ? 1 : 0;
+    static constexpr bool kComp = MODE == 2, kGrad = false;
     const T* a;  // u
     const T* b;  // kappa
     const T* c3;
@@ -253,13 +406,12 @@ struct HeatVarOp {
     T border_value;
     int border_mode;
     __device__ void apply(const Geo& g, int i, int j, int k, const St7<T>& s,
-                          const St7<T>& q, const St7<T>&, const T* xv) const
+                          const St7<T>& q, const St7<T>&, const T* xv, Res<T>& r) const
     {
-        const long m = at(g, i, j, k);
         if (!is_border(g, i, j, k)) {
             if constexpr (MODE == 0) {
-                out[m] = add_by_hh(hh, g.dim, s.c,
-                                   tau * (0.5 * (q.e + q.c) * (s.e - s.c) - 0.5 * (q.c + q.w) * (s.c - s.w)),
+                r.v = add_by_hh(hh, g.dim, s.c,
+                                tau * (0.5 * (q.e + q.c) * (s.e - s.c) - 0.5 * (q.c + q.w) * (s.c - s.w)),
                                    tau * (0.5 * (q.n + q.c) * (s.n - s.c) - 0.5 * (q.c + q.s) * (s.c - s.s)),
                                    tau * (0.5 * (q.u + q.c) * (s.u - s.c) - 0.5 * (q.c + q.d) * (s.c - s.d)));
             } else {
@@ -271,15 +423,15 @@ struct HeatVarOp {
                 if constexpr (MODE == 2) {
                     const float y = d + xv[0];
                     const float t = s.c + y;
-                    cout[m] = y - (t - s.c);
-                    out[m] = t;
+                    r.c = y - (t - s.c);
+                    r.v = t;
                 } else {
-                    out[m] = s.c + d;
+                    r.v = s.c + d;
                 }
             }
         } else {
-            out[m] = border_mode == SCAFES_BORDER_VALUE ? border_value : s.c;
-            if constexpr (MODE == 2) cout[m] = border_mode == SCAFES_BORDER_VALUE ? 0.0f : xv[0];
+            r.v = border_mode == SCAFES_BORDER_VALUE ? border_value : s.c;
+            if constexpr (MODE == 2) r.c = border_mode == SCAFES_BORDER_VALUE ? 0.0f : xv[0];
         }
     }
 };
@@ -293,6 +445,7 @@ struct PennesOp {
     static constexpr bool kTwo = false;
     static constexpr bool kThree = false;
     static constexpr int kNX = KAHAN ? 3 : 2;
+    static constexpr bool kComp = KAHAN, kGrad = false;
     const T* a;  // T_old
     const T* b;
     const T* c3;
@@ -317,16 +470,15 @@ struct PennesOp {
         return (wv + ev) - (T)2 * c;
     }
     __device__ void apply(const Geo& g, int i, int j, int k, const St7<T>& s, const St7<T>&,
-                          const St7<T>&, const T* xv) const
+                          const St7<T>&, const T* xv, Res<T>& r) const
     {
-        const long m = at(g, i, j, k);
         // Tumor border: every node takes the border form, a branch uniform
         // over the launch (per node only selects); away from the faces it is
         // the interior form term for term, so inner nodes get the same value.
         if (tumor || is_border(g, i, j, k)) {
             if (!tumor) {
-                out[m] = s.c;
-                if constexpr (KAHAN) cout[m] = xv[2];
+                r.v = s.c;
+                if constexpr (KAHAN) r.c = xv[2];
                 return;
             }
             const T t0 = tumor_term(i, g.nx, g.dim == 1, 0, s.w, s.e, s.c);
@@ -336,7 +488,7 @@ struct PennesOp {
                 double v = add_by_hh(hh, g.dim, s.c, ctd * t0, ctd * t1, ctd * t2);
                 v += (ctp * xv[0]) * (ta - s.c);
                 v += ctq * xv[1];
-                out[m] = v;
+                r.v = v;
             } else {
                 float d = fd0 * t0;
                 if (g.dim > 1) d = __builtin_fmaf(fd1, t1, d);
@@ -346,10 +498,10 @@ struct PennesOp {
                 if constexpr (KAHAN) {
                     const float y = d + xv[2];
                     const float t = s.c + y;
-                    cout[m] = y - (t - s.c);
-                    out[m] = t;
+                    r.c = y - (t - s.c);
+                    r.v = t;
                 } else {
-                    out[m] = s.c + d;
+                    r.v = s.c + d;
                 }
             }
             return;
@@ -359,7 +511,7 @@ struct PennesOp {
                                  ctd * ((s.d + s.u) - 2.0 * s.c));
             v += (ctp * xv[0]) * (ta - s.c);
             v += ctq * xv[1];
-            out[m] = v;
+            r.v = v;
         } else {
             float d = fd0 * ((s.w + s.e) - 2.0f * s.c);
             if (g.dim > 1) d = __builtin_fmaf(fd1, (s.s + s.n) - 2.0f * s.c, d);
@@ -369,10 +521,10 @@ struct PennesOp {
             if constexpr (KAHAN) {
                 const float y = d + xv[2];
                 const float t = s.c + y;
-                cout[m] = y - (t - s.c);
-                out[m] = t;
+                r.c = y - (t - s.c);
+                r.v = t;
             } else {
-                out[m] = s.c + d;
+                r.v = s.c + d;
             }
         }
     }
@@ -394,6 +546,7 @@ struct MriOp {
     static constexpr bool kTwo = false;
     static constexpr bool kThree = false;
     static constexpr int kNX = 4;
+    static constexpr bool kComp = false, kGrad = false;
     const double* a;  // T_old
     const double* b;
     const double* c3;
@@ -431,9 +584,8 @@ struct MriOp {
         return (wv + ev) - 2.0 * c;
     }
     __device__ void apply(const Geo& g, int i, int j, int k, const St7<double>& s, const St7<double>&,
-                          const St7<double>&, const double* xv) const
+                          const St7<double>&, const double* xv, Res<double>& r) const
     {
-        const long m = at(g, i, j, k);
         double v = s.c;
         if (!is_border(g, i, j, k)) {
             v = add_by_hh(hh, g.dim, v, xv[0] * ((s.w + s.e) - 2.0 * s.c), xv[0] * ((s.s + s.n) - 2.0 * s.c),
@@ -447,7 +599,7 @@ struct MriOp {
         }
         v += xv[1] * (xv[2] - s.c);
         v += xv[3];
-        out[m] = v;
+        r.v = v;
     }
 };
 
@@ -488,6 +640,7 @@ struct HeatVarAdjOp {
     static constexpr bool kTwo = true;
     static constexpr bool kThree = true;
     static constexpr int kNX = 0;
+    static constexpr bool kComp = false, kGrad = true;
     const T* a;   // lam^n
     const T* b;   // kappa
     const T* c3;  // u^{n-1}
@@ -507,9 +660,8 @@ struct HeatVarAdjOp {
         return sp;
     }
     __device__ void apply(const Geo& g, int i, int j, int k, const St7<T>& l, const St7<T>& q, const St7<T>& u,
-                          const T*) const
+                          const T*, Res<T>& r) const
     {
-        const long m = at(g, i, j, k);
         double t = 0.0;  // the gradient increment 0.5 * (the step's term)
         if constexpr (sizeof(T) == 8) {
             t += th0 * face_sum(i > 0, i < g.nx - 1, (double)l.c, (double)l.w, (double)l.e, (double)u.c,
@@ -528,13 +680,13 @@ struct HeatVarAdjOp {
             if (g.dim > 2) tf = __builtin_fmaf(f2, adj_face_sum_f(k > 0, k < g.nz - 1, l.c, l.d, l.u, u.c, u.d, u.u), tf);
             t = (double)tf;
         }
-        grad[m] += t;
+        r.g = t;
         if (is_border(g, i, j, k)) {
-            out[m] = T(0);
+            r.v = T(0);
             return;
         }
         if constexpr (sizeof(T) == 8) {
-            out[m] = add_by_hh(hh, g.dim, l.c,
+            r.v = add_by_hh(hh, g.dim, l.c,
                                tau * (0.5 * (q.e + q.c) * (l.e - l.c) - 0.5 * (q.c + q.w) * (l.c - l.w)),
                                tau * (0.5 * (q.n + q.c) * (l.n - l.c) - 0.5 * (q.c + q.s) * (l.c - l.s)),
                                tau * (0.5 * (q.u + q.c) * (l.u - l.c) - 0.5 * (q.c + q.d) * (l.c - l.d)));
@@ -542,7 +694,7 @@ struct HeatVarAdjOp {
             float d = c0 * __builtin_fmaf(q.e + q.c, l.e - l.c, -((q.c + q.w) * (l.c - l.w)));
             if (g.dim > 1) d = __builtin_fmaf(c1, __builtin_fmaf(q.n + q.c, l.n - l.c, -((q.c + q.s) * (l.c - l.s))), d);
             if (g.dim > 2) d = __builtin_fmaf(c2, __builtin_fmaf(q.u + q.c, l.u - l.c, -((q.c + q.d) * (l.c - l.d))), d);
-            out[m] = l.c + d;
+            r.v = l.c + d;
         }
     }
 };
@@ -554,6 +706,7 @@ struct PennesAdjOp {
     static constexpr bool kTwo = false;
     static constexpr bool kThree = false;
     static constexpr int kNX = LO ? 3 : 2;
+    static constexpr bool kComp = false, kGrad = true;
     const T* a;  // lambda^n
     const T* b;
     const T* c3;
@@ -581,51 +734,50 @@ struct PennesAdjOp {
         return (lw + le) - (T)2 * l;
     }
     __device__ void apply(const Geo& g, int i, int j, int k, const St7<T>& s, const St7<T>&,
-                          const St7<T>&, const T* xv) const
+                          const St7<T>&, const T* xv, Res<T>& r) const
     {
-        const long m = at(g, i, j, k);
         if (tumor) {
-            apply_tumor(g, i, j, k, m, s, xv);
+            apply_tumor(g, i, j, k, s, xv, r);
             return;
         }
         if (is_border(g, i, j, k)) {
-            out[m] = T(0);
+            r.v = T(0);
             return;
         }
         double tp = (double)xv[1];
         if constexpr (LO) tp += (double)xv[2];
-        grad[m] += (double)s.c * (ctp * (ta - tp));
+        r.g = (double)s.c * (ctp * (ta - tp));
         if constexpr (sizeof(T) == 8) {
             double v = add_by_hh(hh, g.dim, s.c, ctd * ((s.w + s.e) - 2.0 * s.c), ctd * ((s.s + s.n) - 2.0 * s.c),
                                  ctd * ((s.d + s.u) - 2.0 * s.c));
             v -= (ctp * xv[0]) * s.c;
-            out[m] = v;
+            r.v = v;
         } else {
             float d = fd0 * ((s.w + s.e) - 2.0f * s.c);
             if (g.dim > 1) d = __builtin_fmaf(fd1, (s.s + s.n) - 2.0f * s.c, d);
             if (g.dim > 2) d = __builtin_fmaf(fd2, (s.d + s.u) - 2.0f * s.c, d);
             d = __builtin_fmaf(-fp * xv[0], s.c, d);
-            out[m] = s.c + d;
+            r.v = s.c + d;
         }
     }
-    __device__ void apply_tumor(const Geo& g, int i, int j, int k, long m, const St7<T>& s, const T* xv) const
+    __device__ void apply_tumor(const Geo& g, int i, int j, int k, const St7<T>& s, const T* xv, Res<T>& r) const
     {
         double tp = (double)xv[1];
         if constexpr (LO) tp += (double)xv[2];
-        grad[m] += (double)s.c * (ctp * (ta - tp));
+        r.g = (double)s.c * (ctp * (ta - tp));
         const T t0 = tumor_adj(i, g.nx, g.dim == 1, 0, s.w, s.e, s.c);
         const T t1 = g.dim > 1 ? tumor_adj(j, g.ny, g.dim == 2, 1, s.s, s.n, s.c) : T(0);
         const T t2 = g.dim > 2 ? tumor_adj(k, g.nz, true, 2, s.d, s.u, s.c) : T(0);
         if constexpr (sizeof(T) == 8) {
             double v = add_by_hh(hh, g.dim, s.c, ctd * t0, ctd * t1, ctd * t2);
             v -= (ctp * xv[0]) * s.c;
-            out[m] = v;
+            r.v = v;
         } else {
             float d = fd0 * t0;
             if (g.dim > 1) d = __builtin_fmaf(fd1, t1, d);
             if (g.dim > 2) d = __builtin_fmaf(fd2, t2, d);
             d = __builtin_fmaf(-fp * xv[0], s.c, d);
-            out[m] = s.c + d;
+            r.v = s.c + d;
         }
     }
 };
@@ -678,31 +830,38 @@ static int launch_t(Ctx* c, const Op& op, const Geo& g, int zc)
     return SCAFES_OK;
 }
 
-// Tile of the one-step launches that take no configuration (heat7, Pennes
-// forward and adjoint, MRI): 128 x 2 threads, 8 z planes per workgroup.
-// Short z chunks give enough workgroups to fill 256 CUs on small grids and
-// cost one extra halo plane per 4 streamed ones, served from L2.  Measured on
-// an MI355X (us per step, this tile vs the best of 15 tiles x 5 chunk
-// lengths): Pennes FP32 256^3 50.5 (best), 512^3 482 (best); Pennes FP64
-// 256^3 112 vs 109; MRI FP64 256^3 200 vs 192, 120x120x50 16.0 (best); the
-// previous 64 x 8, 128-plane default took 87, 515, 127, 263 and 102.
-// Rows of at most 64 nodes take 64 x 4 threads instead (a 128-wide row
-// would leave half its lanes idle), and where 8-plane chunks would give
-// fewer workgroups than CUs the chunks shrink towards four workgroups per
-// CU (heat 64^3 FP64, 100 steps: 7.2 us per step with 128 x 2 and 8-plane
-// chunks, 256 workgroups).
-constexpr int kAutoZc = 8;
-
+// The one-step launches that take no configuration (heat7, Pennes forward and
+// adjoint, MRI, one var-kappa step on grids that do not fill the CUs with the
+// tiles above) run row_kernel.  z planes per workgroup: a chunk of one keeps
+// the most waves in flight and re-reads every neighbour plane from the caches;
+// with enough workgroups the re-reads cost more, so the chunk grows to 2 above
+// 8 workgroups per CU (at one plane each) and to 4 above 24, for two and three
+// stencil fields to 8, and stays at 2 where most of the traffic is centre-only
+// fields.  Measured on an MI355X, us per step, LDS tiles (128 x 2, 8 planes) ->
+// rows with 1 / 2 / 4 / 8 planes: Pennes FP32 128^3 10.1 -> 7.3 / 7.2 / 7.3 /
+// 8.8, 256^3 49.2 -> 47.7 / 47.1 / 47.3 / 49.3; heat FP64 97x80x75 9.3 -> 5.6 /
+// 6.1 / 7.7 / 10.7, 201x150x131 23.1 -> 19.9 / 17.6 / 16.9 / 16.8, 256^3 75 -> 77 /
+// 67 / 63 / 63; MRI 120x120x50 15.7 -> 10.1 / 10.6 / 13.1 / 19.1, 201x150x131
+// 49.5 -> 34.6 / 35.9 / 36.9 / 40.8; Pennes adjoint FP32 97x80x75 10.3 -> 6.0 /
+// 6.0 / 7.1 / 10.1; kappa adjoint FP64 201x150x131 69 -> 45 / 40 / 37 / 37.
+// Rows shorter than a vector take the LDS tile.
 template <class Op, typename T>
 static int launch_auto(Ctx* c, const Op& op, const Geo& g)
 {
-    if (g.nx > 64) return launch_t<Op, T, 128, 2, 4>(c, op, g, kAutoZc);
-    const long per_plane = ceil_div(g.ny, 4);
+    constexpr int V = 16 / (int)sizeof(T);
+    if (g.nx < V) return launch_t<Op, T, 64, 4, 4>(c, op, g, 8);
+    const int cpr = ceil_div(g.nx, V);
+    const long bxy = ceil_div((long)cpr * g.ny, 256);
     const long cus = c->cu_count > 0 ? c->cu_count : 256;
-    int zc = kAutoZc;
-    if (per_plane * ceil_div(g.nz, zc) < cus)
-        zc = (int)std::max(1L, std::min((long)kAutoZc, per_plane * g.nz / (4 * cus)));
-    return launch_t<Op, T, 64, 4, 4>(c, op, g, zc);
+    const int zmax = Op::kTwo ? 8 : Op::kNX >= 3 ? 2 : 4;
+    int zc = 1;
+    if (bxy * g.nz > 8 * cus) zc = 2;
+    if (bxy * g.nz > 24 * cus) zc = zmax;
+    const long nb = bxy * ceil_div(g.nz, zc);
+    if (nb > 0x7fffffffL || (long)cpr * g.ny > 0x7fffffffL - 256) return fail(SCAFES_ERR_ARG, "grid too large");
+    row_kernel<Op, T><<<dim3((unsigned)nb), dim3(256), 0, c->stream>>>(op, g, zc, cpr, (int)bxy);
+    SCAFES_HIP(hipGetLastError());
+    return SCAFES_OK;
 }
 
 template <class Op, typename T>

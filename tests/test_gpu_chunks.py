@@ -70,3 +70,47 @@ def test_yee_schedules_equal(ctx, dtype, n, steps):
     assert np.array_equal(got[0], got[1])
     # the same FP64 terms summed in another order: nodes x 2^-53 at most
     np.testing.assert_allclose(energy[0], energy[1], rtol=6 * (n + 1) ** 3 * 2.0 ** -53)
+
+
+def _nodes(rng, n, fill):
+    """A field on memAll with NaN ghosts."""
+    a = np.full(tuple(m + 2 for m in reversed(n)), np.nan)
+    a[tuple(slice(1, -1) for _ in n)] = fill(tuple(reversed(n)))
+    return a
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [(1, 5, 4), (2, 3, 5), (3, 6, 4), (4, 4, 4), (5, 3, 3), (6, 9, 3), (7, 4, 9), (9, 70, 3),
+                               (257, 3, 4), (11, 5), (6,)])
+def test_pennes_row_ends(ctx, dtype, n):
+    """One Pennes step and one adjoint step on rows around the vector length:
+    every node once, NaN ghosts never used.  FP32 bound: about 20 roundings of
+    terms below 4 (values around 1, the explicit step's positivity)."""
+    rng = np.random.default_rng(sum(n))
+    t, w, q = (_nodes(rng, n, f).astype(dtype) for f in (rng.standard_normal, rng.random, rng.random))
+    h = [0.5 + 0.1 * p for p in range(len(n))]
+    g = capi.geom(n, h=h)
+    p = capi.PennesParams(tau=0.05, cdiff=0.3, cperf=0.7, csrc=0.4, t_a=0.25)
+    code = capi.F32 if dtype == np.float32 else capi.F64
+    a, b, dw, dq, grad = ctx.upload(t), ctx.upload(t), ctx.upload(w), ctx.upload(q), ctx.upload(np.ones(t.shape))
+    inner = tuple(slice(1, -1) for _ in n)
+    T, W, Q = (v[inner].astype(np.float64) for v in (t, w, q))
+    core = tuple(slice(1, -1) for _ in n)
+    d = 0.0
+    for ax in range(len(n)):
+        lo = tuple(slice(0, -2) if x == ax else slice(1, -1) for x in range(len(n)))
+        hi = tuple(slice(2, None) if x == ax else slice(1, -1) for x in range(len(n)))
+        d = d + 0.05 * 0.3 * (T[lo] + T[hi] - 2 * T[core]) / h[len(n) - 1 - ax] ** 2
+    step, lam, gr = T.copy(), np.zeros_like(T), np.ones_like(T)
+    step[core] += d + 0.05 * 0.7 * W[core] * (0.25 - T[core]) + 0.05 * 0.4 * Q[core]
+    lam[core] = T[core] + d - 0.05 * 0.7 * W[core] * T[core]
+    gr[core] += T[core] * (0.05 * 0.7 * (0.25 - Q[core]))
+    tol = 20 * 4 * (2.0 ** -24 if dtype == np.float32 else 2.0 ** -53)
+    capi.check(ctx.L.scafes_pennes_step(ctx.h, C.byref(g), 1, code, a.ptr, b.ptr, dw.ptr, dq.ptr, C.byref(p)))
+    np.testing.assert_allclose(b.read(t.shape)[inner], step, rtol=0, atol=tol)
+    capi.check(ctx.L.scafes_pennes_adjoint_step(ctx.h, C.byref(g), 1, code, a.ptr, b.ptr, dw.ptr, dq.ptr, grad.ptr,
+                                                C.byref(p)))
+    np.testing.assert_allclose(b.read(t.shape)[inner], lam, rtol=0, atol=tol)
+    np.testing.assert_allclose(grad.read(t.shape)[inner], gr, rtol=0, atol=20 * 4 * 2.0 ** -53)
+    for x in (a, b, dw, dq, grad):
+        x.free()
