@@ -47,53 +47,58 @@ struct EmTables {
 
 struct EmArgs {
     int n, d;
+    int cpr, blocks_xy;  // pairs per row, blocks per plane
     long nn;  // n^3
     double s;  // Courant factor
     long src, sink;
 };
 
-__device__ __forceinline__ long nidx(int n, int i, int j, int k)
+// Two consecutive nodes of a row per thread (16-byte accesses at any 8-byte
+// alignment).
+typedef double dv __attribute__((ext_vector_type(2), aligned(8)));
+
+__device__ __forceinline__ dv ld(const double* p) { return *(const dv*)p; }
+
+// A thread's pair (is, is + 1) of row j in plane k; the last pair of an odd
+// row shifts back by one and owns only its second node (skip = 1).
+struct Pair {
+    int is, skip, j, k;
+    long m;  // node (is, j, k)
+    bool on;
+    __device__ __forceinline__ void store(double* p, dv v) const
+    {
+        if (skip) p[1] = v[1];
+        else *(dv*)p = v;
+    }
+};
+
+__device__ __forceinline__ Pair pair_of(const EmArgs& a)
 {
-    return (long)i + (long)n * ((long)j + (long)n * k);
+    const int lb = xcd_remap(blockIdx.x, gridDim.x);
+    Pair p;
+    p.k = lb / a.blocks_xy;
+    const int idx = (lb - p.k * a.blocks_xy) * 256 + (int)threadIdx.x;
+    p.j = idx / a.cpr;
+    const int i0 = 2 * (idx - p.j * a.cpr);
+    p.on = p.j < a.n;
+    p.is = min(i0, a.n - 2);
+    p.skip = i0 - p.is;
+    p.m = (long)p.is + (long)a.n * ((long)p.j + (long)a.n * p.k);
+    return p;
 }
 
-// One CompleteCurlCPMLStencil evaluation.  OL / OR: offsets of the two
-// differenced fields; LO: first valid index per axis; END: last valid index
-// relative to n-1 (the stencil's I_, J_, K_ = n - 1 + END).  The PML index of
-// each term is the distance to the nearer end of the stencil's range along
-// the offset's axis, clamped to d.  FULL: read and write psi everywhere.
-template <int OL0, int OL1, int OL2, int OR0, int OR1, int OR2, int LO0, int LO1, int LO2, int E0, int E1, int E2,
-          bool FULL>
-__device__ __forceinline__ double curl(const EmArgs& a, const EmTables& t, int i, int j, int k, long m,
-                                       double dest_old, double cst, const double* __restrict__ from_l,
-                                       double* __restrict__ psi_l, const double* __restrict__ from_r,
-                                       double* __restrict__ psi_r)
+// The psi recursion of one differenced term at PML index q (d: interior):
+// psi' = b psi + c df, df' = df / kappa + psi'.  Interior terms are left alone
+// (b = c = 0, 1/kappa = 1) unless FULL.
+template <bool FULL>
+__device__ __forceinline__ double cpml(const EmArgs& a, const EmTables& t, bool in, int q, double df, double& psi)
 {
-    const int n = a.n;
-    const int I = n - 1 + E0, J = n - 1 + E1, K = n - 1 + E2;
-    if (i < LO0 || i > I || j < LO1 || j > J || k < LO2 || k > K) return 0.;
-    const int mi = min(i, I - i), mj = min(j, J - j), mk = min(k, K - k);
-    const int dlo = (OL0 ? mi : 0) + (OL1 ? mj : 0) + (OL2 ? mk : 0);
-    const int dro = (OR0 ? mi : 0) + (OR1 ? mj : 0) + (OR2 ? mk : 0);
-    const int dl = min(dlo, a.d), dr = min(dro, a.d);
-    const int li = i + OL0, lj = j + OL1, lk = k + OL2;
-    const int ri = i + OR0, rj = j + OR1, rk = k + OR2;
-    // only the Dx stencil reaches index -1 (j - 1 at j = 0): the zero ghost
-    const double fl = (OL1 < 0 && lj < 0) ? 0.0 : from_l[nidx(n, li, lj, lk)];
-    const double fr = (OR1 < 0 && rj < 0) ? 0.0 : from_r[nidx(n, ri, rj, rk)];
-    double dfdl = fl - from_l[m];
-    if (FULL || dl < a.d) {
-        const double pl = (t.b[dl] * psi_l[m]) + (t.c[dl] * dfdl);
-        dfdl = (t.ook[dl] * dfdl) + pl;
-        psi_l[m] = pl;
+    if (in && (FULL || q < a.d)) {
+        const int w = min(q, a.d);
+        psi = (t.b[w] * psi) + (t.c[w] * df);
+        df = (t.ook[w] * df) + psi;
     }
-    double dfdr = fr - from_r[m];
-    if (FULL || dr < a.d) {
-        const double pr = (t.b[dr] * psi_r[m]) + (t.c[dr] * dfdr);
-        dfdr = (t.ook[dr] * dfdr) + pr;
-        psi_r[m] = pr;
-    }
-    return dest_old + (cst * (dfdl - dfdr));
+    return df;
 }
 
 struct EmFields {
@@ -115,68 +120,204 @@ __host__ EmFields fields_of(double* s, long nn)
     return f;
 }
 
-// updateInner: H from E (EMFDTD.hpp:295-313, stencil types :167-169,
-// ranges and constants :208-210).
+// Both phases: one thread per pair of nodes, every field and psi load issued
+// before the first use (the psi ones under their PML condition), so a wave
+// waits once; blocks of one plane, XCD-contiguous, so the neighbour rows and
+// planes come from that XCD's L2.  Bound by HBM: 72 B (H) and 104 B (E) per
+// node and the psi of the PML.  Measured on an MI355X at 200^3, d = 10, us per
+// step, one node per thread with 64 x 4 blocks and psi loaded at its use ->
+// pairs: H 213 -> 157, E 262 -> 213 (134 and 186 at the rate of a large copy).
+
+// updateInner: H from E (EMFDTD.hpp:295-313, stencil types :167-169, ranges
+// and constants :208-210).  The PML index along an axis is the distance to the
+// nearer end of 0..n-2.
 template <bool FULL>
 __global__ __launch_bounds__(256) void em_h_kernel(EmArgs a, EmTables t, EmFields f)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y;
-    const int k = blockIdx.z;
-    if (i >= a.n || j >= a.n) return;
-    const long m = nidx(a.n, i, j, k);
+    const Pair p = pair_of(a);
+    if (!p.on) return;
+    const int n = a.n, e = n - 2;
+    const long m = p.m;
+    const long jp = p.j < n - 1 ? m + n : m, kp = p.k < n - 1 ? m + (long)n * n : m;
+    const long ip = p.is < n - 2 ? m + 2 : m + 1;
+    const dv ex = ld(f.ex + m), exj = ld(f.ex + jp), exk = ld(f.ex + kp);
+    const dv ey = ld(f.ey + m), eyk = ld(f.ey + kp), ez = ld(f.ez + m), ezj = ld(f.ez + jp);
+    const double eyp = f.ey[ip], ezp = f.ez[ip];
+    dv hx = ld(f.hx + m), hy = ld(f.hy + m), hz = ld(f.hz + m);
+    const int qj = min(p.j, e - p.j), qk = min(p.k, e - p.k);
+    const int q0 = min(p.is, e - p.is), q1 = min(p.is + 1, e - p.is - 1);
+    const bool pj = FULL || qj < a.d, pk = FULL || qk < a.d, pi = FULL || min(q0, q1) < a.d;
+    dv ezdy = {}, exdy = {}, eydz = {}, exdz = {}, ezdx = {}, eydx = {};
+    if (pj) {
+        ezdy = ld(f.p_ezdy + m);
+        exdy = ld(f.p_exdy + m);
+    }
+    if (pk) {
+        eydz = ld(f.p_eydz + m);
+        exdz = ld(f.p_exdz + m);
+    }
+    if (pi) {
+        ezdx = ld(f.p_ezdx + m);
+        eydx = ld(f.p_eydx + m);
+    }
     const double S = a.s;
-    f.hx[m] = curl<0, 0, 1, 0, 1, 0, 1, 0, 0, 0, -1, -1, FULL>(a, t, i, j, k, m, f.hx[m], S, f.ey, f.p_eydz, f.ez,
-                                                               f.p_ezdy);
-    f.hy[m] = curl<1, 0, 0, 0, 0, 1, 0, 1, 0, -1, 0, -1, FULL>(a, t, i, j, k, m, f.hy[m], S, f.ez, f.p_ezdx, f.ex,
-                                                               f.p_exdz);
-    f.hz[m] = curl<0, 1, 0, 1, 0, 0, 0, 0, 1, -1, -1, 0, FULL>(a, t, i, j, k, m, f.hz[m], S, f.ex, f.p_exdy, f.ey,
-                                                               f.p_eydx);
+    const dv eyi = {ey[1], eyp}, ezi = {ez[1], ezp};
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const int i = p.is + x, qi = x ? q1 : q0;
+        const bool inx = i >= 1 && p.j <= e && p.k <= e;
+        const bool iny = p.j >= 1 && i <= e && p.k <= e;
+        const bool inz = p.k >= 1 && i <= e && p.j <= e;
+        double l, r, pl, pr;
+        pl = eydz[x];
+        pr = ezdy[x];
+        l = cpml<FULL>(a, t, inx, qk, eyk[x] - ey[x], pl);
+        r = cpml<FULL>(a, t, inx, qj, ezj[x] - ez[x], pr);
+        hx[x] = inx ? hx[x] + (S * (l - r)) : 0.;
+        eydz[x] = pl;
+        ezdy[x] = pr;
+        pl = ezdx[x];
+        pr = exdz[x];
+        l = cpml<FULL>(a, t, iny, qi, ezi[x] - ez[x], pl);
+        r = cpml<FULL>(a, t, iny, qk, exk[x] - ex[x], pr);
+        hy[x] = iny ? hy[x] + (S * (l - r)) : 0.;
+        ezdx[x] = pl;
+        exdz[x] = pr;
+        pl = exdy[x];
+        pr = eydx[x];
+        l = cpml<FULL>(a, t, inz, qj, exj[x] - ex[x], pl);
+        r = cpml<FULL>(a, t, inz, qi, eyi[x] - ey[x], pr);
+        hz[x] = inz ? hz[x] + (S * (l - r)) : 0.;
+        exdy[x] = pl;
+        eydx[x] = pr;
+    }
+    p.store(f.hx + m, hx);
+    p.store(f.hy + m, hy);
+    p.store(f.hz + m, hz);
+    if (pj) {
+        p.store(f.p_ezdy + m, ezdy);
+        p.store(f.p_exdy + m, exdy);
+    }
+    if (pk) {
+        p.store(f.p_eydz + m, eydz);
+        p.store(f.p_exdz + m, exdz);
+    }
+    if (pi) {
+        p.store(f.p_ezdx + m, ezdx);
+        p.store(f.p_eydx + m, eydx);
+    }
 }
 
 // updateInner2: D from H, E = ga (D - I), I += gb E, hard source, sink
 // (EMFDTD.hpp:330-386, stencil types :170-172, ranges and constants :211-213).
+// The PML index along an axis is the distance to the nearer end of 0..n-1.
+// Hz(i, -1, k) is the zero ghost.
 template <bool FULL, bool VACUUM>
 __global__ __launch_bounds__(256) void em_e_kernel(EmArgs a, EmTables t, EmFields f, double src_value,
                                                    double* __restrict__ sink)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y;
-    const int k = blockIdx.z;
-    if (i >= a.n || j >= a.n) return;
-    const long m = nidx(a.n, i, j, k);
-    const double S = -a.s;
-    const double Dx = curl<0, -1, 0, 0, 0, -1, 0, 0, 1, -1, 0, 0, FULL>(a, t, i, j, k, m, f.dx[m], S, f.hz,
-                                                                        f.p_hzdy, f.hy, f.p_hydz);
-    const double Dy = curl<0, 0, -1, -1, 0, 0, 1, 0, 1, 0, -1, 0, FULL>(a, t, i, j, k, m, f.dy[m], S, f.hx,
-                                                                        f.p_hxdz, f.hz, f.p_hzdx);
-    const double Dz = curl<-1, 0, 0, 0, -1, 0, 1, 1, 0, 0, 0, -1, FULL>(a, t, i, j, k, m, f.dz[m], S, f.hy,
-                                                                        f.p_hydx, f.hx, f.p_hxdy);
-    const double gb = f.gb[m];
-    double Ex, Ey, Ez;
-    if (VACUUM && gb == 0.0) {
-        // ga = 1, I = 0: E = 1 * (D - 0) = D, I unchanged
-        Ex = Dx;
-        Ey = Dy;
-        Ez = Dz;
-    } else {
-        const double ga = f.ga[m];
-        const double ix = f.ix[m], iy = f.iy[m], iz = f.iz[m];
-        Ex = ga * (Dx - ix);
-        Ey = ga * (Dy - iy);
-        Ez = ga * (Dz - iz);
-        f.ix[m] = ix + (gb * Ex);
-        f.iy[m] = iy + (gb * Ey);
-        f.iz[m] = iz + (gb * Ez);
+    const Pair p = pair_of(a);
+    if (!p.on) return;
+    const int n = a.n, e = n - 1;
+    const long m = p.m;
+    const long jm = p.j > 0 ? m - n : m, km = p.k > 0 ? m - (long)n * n : m;
+    const long im = p.is > 0 ? m - 1 : m;
+    dv dx = ld(f.dx + m), dy = ld(f.dy + m), dz = ld(f.dz + m);
+    const dv hx = ld(f.hx + m), hxj = ld(f.hx + jm), hxk = ld(f.hx + km);
+    const dv hy = ld(f.hy + m), hyk = ld(f.hy + km), hz = ld(f.hz + m);
+    dv hzj = ld(f.hz + jm);
+    const double hym = f.hy[im], hzm = f.hz[im];
+    const dv gb = ld(f.gb + m);
+    const int qj = min(p.j, e - p.j), qk = min(p.k, e - p.k);
+    const int q0 = min(p.is, e - p.is), q1 = min(p.is + 1, e - p.is - 1);
+    const bool pj = FULL || qj < a.d, pk = FULL || qk < a.d, pi = FULL || min(q0, q1) < a.d;
+    dv hzdy = {}, hxdy = {}, hydz = {}, hxdz = {}, hzdx = {}, hydx = {};
+    if (pj) {
+        hzdy = ld(f.p_hzdy + m);
+        hxdy = ld(f.p_hxdy + m);
     }
-    f.dx[m] = Dx;
-    f.dy[m] = Dy;
-    f.dz[m] = Dz;
-    f.ex[m] = Ex;
-    f.ey[m] = Ey;
-    const double ez = m == a.src ? src_value : Ez;
-    f.ez[m] = ez;
-    if (sink && m == a.sink) *sink = ez;
+    if (pk) {
+        hydz = ld(f.p_hydz + m);
+        hxdz = ld(f.p_hxdz + m);
+    }
+    if (pi) {
+        hzdx = ld(f.p_hzdx + m);
+        hydx = ld(f.p_hydx + m);
+    }
+    if (p.j == 0) hzj = dv{0.0, 0.0};
+    const double S = -a.s;
+    const dv hyi = {hym, hy[0]}, hzi = {hzm, hz[0]};
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const int i = p.is + x, qi = x ? q1 : q0;
+        const bool inx = i <= e - 1 && p.k >= 1;
+        const bool iny = i >= 1 && p.j <= e - 1 && p.k >= 1;
+        const bool inz = i >= 1 && p.j >= 1 && p.k <= e - 1;
+        double l, r, pl, pr;
+        pl = hzdy[x];
+        pr = hydz[x];
+        l = cpml<FULL>(a, t, inx, qj, hzj[x] - hz[x], pl);
+        r = cpml<FULL>(a, t, inx, qk, hyk[x] - hy[x], pr);
+        dx[x] = inx ? dx[x] + (S * (l - r)) : 0.;
+        hzdy[x] = pl;
+        hydz[x] = pr;
+        pl = hxdz[x];
+        pr = hzdx[x];
+        l = cpml<FULL>(a, t, iny, qk, hxk[x] - hx[x], pl);
+        r = cpml<FULL>(a, t, iny, qi, hzi[x] - hz[x], pr);
+        dy[x] = iny ? dy[x] + (S * (l - r)) : 0.;
+        hxdz[x] = pl;
+        hzdx[x] = pr;
+        pl = hydx[x];
+        pr = hxdy[x];
+        l = cpml<FULL>(a, t, inz, qi, hyi[x] - hy[x], pl);
+        r = cpml<FULL>(a, t, inz, qj, hxj[x] - hx[x], pr);
+        dz[x] = inz ? dz[x] + (S * (l - r)) : 0.;
+        hydx[x] = pl;
+        hxdy[x] = pr;
+    }
+    // vacuum (gb = 0): ga = 1, I = 0, so E = 1 * (D - 0) = D and I is unchanged
+    dv ex = dx, ey = dy, ez = dz;
+    if (!VACUUM || gb[0] != 0.0 || gb[1] != 0.0) {
+        const dv ga = ld(f.ga + m);
+        dv ix = ld(f.ix + m), iy = ld(f.iy + m), iz = ld(f.iz + m);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            if (VACUUM && gb[x] == 0.0) continue;
+            ex[x] = ga[x] * (dx[x] - ix[x]);
+            ey[x] = ga[x] * (dy[x] - iy[x]);
+            ez[x] = ga[x] * (dz[x] - iz[x]);
+            ix[x] = ix[x] + (gb[x] * ex[x]);
+            iy[x] = iy[x] + (gb[x] * ey[x]);
+            iz[x] = iz[x] + (gb[x] * ez[x]);
+        }
+        p.store(f.ix + m, ix);
+        p.store(f.iy + m, iy);
+        p.store(f.iz + m, iz);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        if (m + x == a.src) ez[x] = src_value;
+        if (sink && m + x == a.sink && x >= p.skip) *sink = ez[x];
+    }
+    p.store(f.dx + m, dx);
+    p.store(f.dy + m, dy);
+    p.store(f.dz + m, dz);
+    p.store(f.ex + m, ex);
+    p.store(f.ey + m, ey);
+    p.store(f.ez + m, ez);
+    if (pj) {
+        p.store(f.p_hzdy + m, hzdy);
+        p.store(f.p_hxdy + m, hxdy);
+    }
+    if (pk) {
+        p.store(f.p_hydz + m, hydz);
+        p.store(f.p_hxdz + m, hxdz);
+    }
+    if (pi) {
+        p.store(f.p_hzdx + m, hzdx);
+        p.store(f.p_hydx + m, hydx);
+    }
 }
 
 // 1 when some gb = 0 node has ga != 1 or a nonzero conduction current.
@@ -253,27 +394,34 @@ double scafes_emfdtd_source(double t, double dt, double f_mod, double t0, double
     return v * mod;
 }
 
+// Launches the vacuum check; its flag (an int in the context's pinned memory)
+// is valid once c->ready has passed.
+static int vacuum_check(Ctx* c, const EmFields& f, long nn)
+{
+    volatile int* flag = reinterpret_cast<int*>(c->host_result);
+    *flag = 0;
+    em_vacuum_check<<<(unsigned)std::min<long>((nn + 255) / 256, 4096), 256, 0, c->stream>>>(
+        nn, f, reinterpret_cast<int*>(c->host_result_dev));
+    SCAFES_HIP(hipGetLastError());
+    SCAFES_HIP(hipEventRecord(c->ready, c->stream));
+    return SCAFES_OK;
+}
+
+static int vacuum_result(Ctx* c, int* ok)
+{
+    SCAFES_HIP(hipEventSynchronize(c->ready));
+    *ok = *reinterpret_cast<volatile int*>(c->host_result) == 0 ? 1 : 0;
+    return SCAFES_OK;
+}
+
 int scafes_emfdtd_vacuum_ok(scafes_ctx* ctx, const scafes_emfdtd_params* p, const double* state, int* ok)
 {
     Ctx* c = as_ctx(ctx);
     if (!c || !p || !state || !ok) return fail(SCAFES_ERR_ARG, "emfdtd_vacuum_ok: null pointer");
     if (p->n < 2 || p->n > 4096) return fail(SCAFES_ERR_ARG, "emfdtd_vacuum_ok: n must be 2..4096");
     const long nn = (long)p->n * p->n * p->n;
-    const EmFields f = fields_of(const_cast<double*>(state), nn);
-    int* bad = nullptr;
-    SCAFES_HIP(hipMalloc((void**)&bad, sizeof(int)));
-    int hbad = 0;
-    hipError_t e = hipMemcpyAsync(bad, &hbad, sizeof(int), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) {
-        em_vacuum_check<<<(unsigned)std::min<long>((nn + 255) / 256, 4096), 256, 0, c->stream>>>(nn, f, bad);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(bad);
-    if (e != hipSuccess) return check_hip(e, "emfdtd vacuum check");
-    *ok = hbad == 0 ? 1 : 0;
-    return SCAFES_OK;
+    const int rc = vacuum_check(c, fields_of(const_cast<double*>(state), nn), nn);
+    return rc ? rc : vacuum_result(c, ok);
 }
 
 int scafes_emfdtd_run(scafes_ctx* ctx, const scafes_emfdtd_params* p, double* state, int nsteps, double t_start,
@@ -303,16 +451,17 @@ int scafes_emfdtd_run(scafes_ctx* ctx, const scafes_emfdtd_params* p, double* st
         t.ook[w] = w <= p->d ? p->ook[w] : 1.0;
     }
     const EmFields f = fields_of(state, a.nn);
-    // vacuum shortcut allowed?
-    int ok = (p->flags & SCAFES_EMFDTD_VACUUM_OK) ? 1 : 0;
-    if (!ok) {
-        const int rc = scafes_emfdtd_vacuum_ok(ctx, p, state, &ok);
-        if (rc != SCAFES_OK) return rc;
-    }
-    const bool vacuum = ok != 0;
-    const dim3 blk(64, 4, 1);
-    const dim3 grid((unsigned)ceil_div(n, 64), (unsigned)ceil_div(n, 4), (unsigned)n);
+    a.cpr = (n + 1) / 2;
+    a.blocks_xy = ceil_div((long)a.cpr * n, 256);
+    const dim3 blk(256), grid((unsigned)((long)a.blocks_xy * n));
     const double dt = p->dt;
+    // Vacuum shortcut allowed?  The first H phase does not depend on it and
+    // runs while the host waits for the check.
+    int vacuum = (p->flags & SCAFES_EMFDTD_VACUUM_OK) ? 1 : -1;
+    if (vacuum < 0) {
+        const int rc = vacuum_check(c, f, a.nn);
+        if (rc) return rc;
+    }
     for (int s = 1; s <= nsteps; ++s) {
         // the source reads the old field's time t_start + (s-1) tau, tau = 1
         const double sv = scafes_emfdtd_source(t_start + (double)(s - 1) * 1.0, dt, p->f_mod, p->t0, p->spread);
@@ -320,6 +469,10 @@ int scafes_emfdtd_run(scafes_ctx* ctx, const scafes_emfdtd_params* p, double* st
         const bool full = s == 1 && !(p->flags & SCAFES_EMFDTD_PSI_SETTLED);
         if (full) em_h_kernel<true><<<grid, blk, 0, c->stream>>>(a, t, f);
         else em_h_kernel<false><<<grid, blk, 0, c->stream>>>(a, t, f);
+        if (vacuum < 0) {
+            const int rc = vacuum_result(c, &vacuum);
+            if (rc) return rc;
+        }
         if (full && vacuum) em_e_kernel<true, true><<<grid, blk, 0, c->stream>>>(a, t, f, sv, sk);
         else if (full) em_e_kernel<true, false><<<grid, blk, 0, c->stream>>>(a, t, f, sv, sk);
         else if (vacuum) em_e_kernel<false, true><<<grid, blk, 0, c->stream>>>(a, t, f, sv, sk);

@@ -329,6 +329,8 @@ int scafes_ctx_create(int device, scafes_ctx** out)
     SCAFES_HIP(hipMalloc(&c->red_partial, sizeof(double) * c->red_capacity));
     SCAFES_HIP(hipMalloc(&c->red_result, sizeof(double) * 8));
     SCAFES_HIP(hipHostMalloc(&c->host_result, sizeof(double) * 8, hipHostMallocDefault));
+    SCAFES_HIP(hipHostGetDevicePointer((void**)&c->host_result_dev, c->host_result, 0));
+    SCAFES_HIP(hipEventCreateWithFlags(&c->ready, hipEventDisableTiming));
     for (int i = 0; i < 8; ++i) SCAFES_HIP(hipEventCreate(&c->events[i]));
     // device address of the no-allocation entry point's scratch array, looked
     // up once per device with that device current
@@ -379,6 +381,7 @@ int scafes_ctx_destroy(scafes_ctx* ctx)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (int i = 0; i < 8; ++i)
         if (c->events[i]) (void)hipEventDestroy(c->events[i]);
+    if (c->ready) (void)hipEventDestroy(c->ready);
     if (c->grad_ws) (void)hipFree(c->grad_ws);
     if (c->batch_exec) (void)hipGraphExecDestroy(c->batch_exec);
     if (c->red_partial) (void)hipFree(c->red_partial);

@@ -34,7 +34,11 @@ struct Ctx {
     hipStream_t stream = nullptr;
     double* red_partial = nullptr;  // per-block reduction partials (device)
     double* red_result = nullptr;   // final reduction values (device, 8 slots)
-    double* host_result = nullptr;  // pinned host mirror of red_result
+    // pinned host memory that kernels write their results to (8 slots), and the
+    // device's address of it; a call that uses it waits before it returns
+    double* host_result = nullptr;
+    double* host_result_dev = nullptr;
+    hipEvent_t ready = nullptr;  // no timing: a result is in host_result
     int red_capacity = 0;           // number of partial slots
     int cu_count = 0;
     // autotuned heat7var tile per grid and mode (scafes_autotune_heat7var)
