@@ -56,35 +56,41 @@ __global__ __launch_bounds__(256) void lam_init_kernel(Geo g, const T* __restric
                                                        T* __restrict__ lam2, int every_node,
                                                        double* __restrict__ partial)
 {
-    __shared__ double sh[256];
+    __shared__ double sh[4];
     double acc = 0.0;
-    // work items: 256-node chunks of x-rows (indices formed once per chunk)
-    const int cpr = (g.nx + 255) / 256;
-    const long items = (long)g.ny * g.nz * cpr;
-    for (long w = blockIdx.x; w < items; w += gridDim.x) {
-        const long r = w / cpr;
-        const int i = (int)(w - r * cpr) * 256 + (int)threadIdx.x;
-        const int j = (int)(r % g.ny), k = (int)(r / g.ny);
+    // work items: 64-node chunks of x-rows, one per wave (indices formed once
+    // per chunk)
+    const int cpr = (g.nx + 63) / 64, lane = (int)threadIdx.x & 63;
+    const unsigned items = (unsigned)g.ny * (unsigned)g.nz * (unsigned)cpr;
+    for (unsigned w = blockIdx.x * 4u + (threadIdx.x >> 6); w < items; w += gridDim.x * 4u) {
+        const unsigned r = w / (unsigned)cpr;
+        const int i = (int)(w - r * (unsigned)cpr) * 64 + lane;
+        const int k = (int)(r / (unsigned)g.ny), j = (int)(r - (unsigned)k * (unsigned)g.ny);
         if (i >= g.nx) continue;
         const long m = at(g, i, j, k);
         double v = (double)t[m] - (double)target[m];
         if (tlo) v += (double)tlo[m];
-        const T l = (every_node || !is_border(g, i, j, k)) ? (T)v : T(0);
+        // is_border as one mask: written with short-circuit branches, ROCm 7.2's
+        // clang zeroes l on every lane of the FP64 instance of this loop
+        const bool inner = (i >= g.nl0) & (i <= g.nx - 1 - g.nl0) & (j >= g.nl1) & (j <= g.ny - 1 - g.nl1) &
+                           (k >= g.nl2) & (k <= g.nz - 1 - g.nl2);
+        const T l = (every_node != 0) | inner ? (T)v : T(0);
         lam[m] = l;
         lam2[m] = T(0);
         acc += (double)l * (double)l;
     }
-    sh[threadIdx.x] = acc;
+    for (int w = 32; w > 0; w >>= 1) acc += __shfl_down(acc, w, 64);
+    if (lane == 0) sh[threadIdx.x >> 6] = acc;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
+    if (threadIdx.x == 0) partial[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
 }
 
 // A forward state is one array (F32, F64) or a (hi, lo) pair stored as two
 // consecutive arrays of ne elements (F32_KAHAN).
+// host_result slots of a gradient: 2 J (Yee: J), read when the schedule is done
+// (slot 0 takes the stability checks' reductions).
+constexpr int kSlotJ = 1;
+
 enum { FAMILY_PENNES = 0, FAMILY_HEATVAR = 1, FAMILY_YEE_EPS = 2 };
 
 struct Rev {
@@ -96,13 +102,13 @@ struct Rev {
     double tau = 0.0, border_value = 0.0;
     int border_mode = SCAFES_BORDER_KEEP;
     // FAMILY_YEE_EPS: box, Courant number, ce = s/eps and eps fields, J
-    // partials and J on the device
+    // partials
     YeeDims yd{};
     double yee_s = 0.0;
     const void* ce = nullptr;
     const void* eps = nullptr;
     double* partial = nullptr;
-    double* jdev = nullptr;
+    size_t reserved = 0;  // bytes of the workspace in use before the schedule's (ce, partials)
     Ctx* c;
     Geo geo;
     const scafes_geom* g;
@@ -124,7 +130,6 @@ struct Rev {
     bool pair;  // several adjoint steps per sweep where their states are at hand
     bool lam_ready = false;  // lam^N and J set (first_leaf)
     long fwd_steps, adj_steps;
-    double J;
 
     bool kahan() const { return dtype == SCAFES_F32_KAHAN; }
     const void* lo(const void* s) const { return kahan() ? (const void*)((const float*)s + ne) : nullptr; }
@@ -180,10 +185,11 @@ struct Rev {
     int adjoint(int n, const void* tprev)
     {
         if (family == FAMILY_YEE_EPS) {
-            // J^N goes to the device and is read at the end
+            // J goes to host_result and is read at the end
             if (n == nsteps) {
                 int r = step(tprev, tmp[0]);
-                if (!r) r = yee_eps_lam_init(c, yd, dtype, tmp[0], target, lam[lcur], partial, jdev);
+                if (!r) r = yee_eps_lam_init(c, yd, dtype, tmp[0], target, lam[lcur], partial,
+                                            c->host_result_dev + kSlotJ);
                 if (r) return r;
             }
             ++adj_steps;
@@ -213,7 +219,7 @@ struct Rev {
             int r = tprev ? step(tprev, tmp[0]) : SCAFES_OK;
             if (r) return r;
             const long total = (long)geo.nx * geo.ny * geo.nz;
-            const int blocks = (int)std::min<long>((total + 255) / 256, c->red_capacity);
+            const int blocks = (int)std::max(1L, std::min((total + 1023) / 1024, (long)c->red_capacity));
             // J over the nodes the step updates: every node under the
             // Tumor border, the inner nodes otherwise
             const int every = family == FAMILY_PENNES && p->border_mode == SCAFES_BORDER_TUMOR;
@@ -227,9 +233,8 @@ struct Rev {
                                                                       (float*)lam[0], (float*)lam[1], every,
                                                                       c->red_partial);
             SCAFES_HIP(hipGetLastError());
-            r = reduce_partials(c, blocks, &J);
+            r = reduce_partials(c, blocks, kSlotJ);
             if (r) return r;
-            J *= 0.5;
         }
         lam_ready = true;
         return SCAFES_OK;
@@ -534,6 +539,33 @@ static long count_forward(long a, long b, int s, int nsteps)
 
 using namespace scafes;
 
+static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Workspace of a schedule: [compensated initial state] tmp[0] tmp[1] work
+// lam[0] lam[1] and the snapshots.
+static size_t schedule_bytes(int dtype, size_t abytes, int nsteps, int max_snapshots)
+{
+    const int snaps = std::max(0, std::min(max_snapshots, nsteps - 1));
+    const bool kahan0 = dtype == SCAFES_F32_KAHAN;
+    const size_t sb = round256(kahan0 ? 2 * abytes : abytes);
+    return (kahan0 ? sb : 0) + 3 * sb + 2 * round256(abytes) + (size_t)snaps * sb;
+}
+
+static int grow_workspace(Ctx* c, size_t need)
+{
+    if (c->grad_ws_bytes >= need) return SCAFES_OK;
+    if (c->grad_ws) (void)hipFree(c->grad_ws);
+    c->grad_ws = nullptr;
+    c->grad_ws_bytes = 0;
+    hipError_t e = hipMalloc(&c->grad_ws, need);
+    if (e != hipSuccess) {
+        c->grad_ws = nullptr;
+        return check_hip(e, "gradient workspace");
+    }
+    c->grad_ws_bytes = need;
+    return SCAFES_OK;
+}
+
 // Reverse sweep with binomial checkpointing: R carries the family's fields;
 // t0 is the initial state (FP32 fields in the FP32 modes); a state is one
 // array of abytes (two in the compensated mode), an adjoint field abytes,
@@ -555,29 +587,17 @@ static int run_schedule(Rev& R, Ctx* c, int dtype, const void* t0, size_t abytes
     R.pair = (R.family == FAMILY_PENNES && pennes_adjk_supported(R.geo)) ||
              (R.family == FAMILY_HEATVAR && heatvar_adj2_supported(R.geo));
     R.fwd_steps = R.adj_steps = 0;
-    R.J = 0.0;
     R.work = nullptr;
     // Workspace: [compensated initial state] tmp[0] tmp[1] work lam[0]
     // lam[1] and the snapshot pool (a store-all budget of a 256^3 x
     // 2000-step FP32 run is 134 GB; HBM holds 288 GB), carved from one
     // buffer the context keeps for the next gradient call: re-allocating
     // freed memory makes the driver clear it first (about 0.5 s per 137 GB).
-    auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const bool kahan0 = dtype == SCAFES_F32_KAHAN;
-    const size_t sb = up(R.sbytes), lb = up(abytes);
-    const size_t need = (kahan0 ? sb : 0) + 3 * sb + 2 * lb + (size_t)snaps * sb;
-    if (c->grad_ws_bytes < need) {
-        if (c->grad_ws) (void)hipFree(c->grad_ws);
-        c->grad_ws = nullptr;
-        c->grad_ws_bytes = 0;
-        hipError_t e = hipMalloc(&c->grad_ws, need);
-        if (e != hipSuccess) {
-            c->grad_ws = nullptr;
-            return check_hip(e, "gradient workspace");
-        }
-        c->grad_ws_bytes = need;
-    }
-    char* ws = (char*)c->grad_ws;
+    const size_t sb = round256(R.sbytes), lb = round256(abytes);
+    rc = grow_workspace(c, R.reserved + schedule_bytes(dtype, abytes, nsteps, max_snapshots));
+    if (rc) return rc;
+    char* ws = (char*)c->grad_ws + R.reserved;
     // the initial state as a state (a (t0, 0) pair in the compensated mode)
     const void* base = t0;
     if (kahan0) {
@@ -607,7 +627,8 @@ static int run_schedule(Rev& R, Ctx* c, int dtype, const void* t0, size_t abytes
         if (e != hipSuccess) rc = check_hip(e, "gradient");
     }
     if (rc) return rc;
-    *J = R.J;
+    const double j = ((volatile double*)c->host_result)[kSlotJ];
+    *J = R.family == FAMILY_YEE_EPS ? j : 0.5 * j;
     if (stats) {
         stats[0] = (double)R.fwd_steps;
         stats[1] = (double)R.adj_steps;
@@ -732,26 +753,16 @@ int scafes_yee_eps_gradient(scafes_ctx* ctx, int ncell, int dtype, double s, con
     R.ne = 6 * d.nf;
     R.w = R.q = nullptr;
     R.p = nullptr;
-    void* ce = nullptr;
-    void* aux = nullptr;  // J partials, then J
-    const size_t naux = (size_t)yee_eps_partials() + 1;
-    hipError_t e = hipMalloc(&ce, (size_t)d.nf * es);
-    if (e == hipSuccess) e = hipMalloc(&aux, naux * sizeof(double));
-    int rc = e == hipSuccess ? SCAFES_OK : check_hip(e, "yee eps gradient buffers");
-    if (!rc) rc = yee_eps_coef(c, d, dtype, s, eps, ce);
-    if (!rc) {
-        R.ce = ce;
-        R.partial = (double*)aux;
-        R.jdev = (double*)aux + yee_eps_partials();
-        rc = run_schedule(R, c, dtype, f0, 6 * (size_t)d.nf * es, d.nf, target, nsteps, max_snapshots, grad, J,
-                          stats);
-    }
-    if (!rc) {
-        e = hipMemcpy(J, R.jdev, sizeof(double), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) rc = check_hip(e, "yee eps gradient J");
-    }
-    (void)hipFree(ce);
-    (void)hipFree(aux);
+    // ce and the J partials stand at the front of the context's workspace
+    const size_t abytes = 6 * (size_t)d.nf * es;
+    const size_t cb = round256((size_t)d.nf * es);
+    R.reserved = cb + round256((size_t)yee_eps_partials() * sizeof(double));
+    int rc = grow_workspace(c, R.reserved + schedule_bytes(dtype, abytes, nsteps, max_snapshots));
+    if (rc) return rc;
+    R.ce = c->grad_ws;
+    R.partial = (double*)((char*)c->grad_ws + cb);
+    rc = yee_eps_coef(c, d, dtype, s, eps, c->grad_ws);
+    if (!rc) rc = run_schedule(R, c, dtype, f0, abytes, d.nf, target, nsteps, max_snapshots, grad, J, stats);
     return rc;
 }
 

@@ -1,4 +1,5 @@
 // scafes_capi.hip -- context, memory, errors and FP64 reductions of the C ABI.
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -92,102 +93,160 @@ __global__ void convert_kernel(D* d, const S* s, size_t n)
         d[i] = (D)s[i];
 }
 
-// Per-block FP64 partials of a node reduction.  Work items are 256-node
-// chunks of x-rows: a block takes items blockIdx.x, + gridDim.x, ..., one
-// node per thread, so the row and plane indices are formed once per chunk
-// (uniform over the block) rather than by 64-bit divisions per node.
-template <typename T>
+// Node reductions in FP64.  A thread takes 16-byte vectors of x-rows (V nodes;
+// V = 1 where a row is shorter), the last vector of a row shifting back into it
+// and counting only its own nodes; vector numbers run over the rows of all
+// planes, so small grids fill their lanes (a row-per-block loop kept 32 of 256
+// lanes busy at nx = 32).  Up to kOnePassBlocks blocks the one that ends last
+// sums the partials, so a small reduction is one launch and one wait; the
+// blocks' count is an atomic that all XCDs contend for (about 25 ns each), so
+// more blocks leave the sum to a second launch.  The result goes to pinned host
+// memory, without a copy.  us on an MI355X, the two launches of the row loop
+// and their copy -> now: 32x24x20 FP64 37 + 5 -> 7, 128^3 FP32 15 + 3 -> 5 + 2,
+// 512^3 FP32 354 + 9 -> 145 + 4.
+constexpr int kOnePassBlocks = 64;
+
+template <int WAVES>
+__device__ inline double wave_block_reduce(double acc, bool is_max, double* sh)
+{
+    for (int w = 32; w > 0; w >>= 1) {
+        const double o = __shfl_down(acc, w, 64);
+        acc = is_max ? fmax(acc, o) : acc + o;
+    }
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    double r = sh[0];
+    for (int w = 1; w < WAVES; ++w) r = is_max ? fmax(r, sh[w]) : r + sh[w];
+    __syncthreads();
+    return r;  // the same in every thread
+}
+
+template <typename T, int V, typename I>
 __global__ __launch_bounds__(256) void reduce_kernel(Geo ga, Geo gb, const T* __restrict__ a,
-                                                     const T* __restrict__ b, int op, int inner_only,
-                                                     double* partial)
+                                                     const T* __restrict__ b, int op, int inner_only, int cpr,
+                                                     I items, double* partial, unsigned* done, double* out)
 {
-    __shared__ double sh[256];
+    typedef T vec __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+    __shared__ double sh[4];
+    __shared__ bool last;
+    const bool is_max = op == RED_MAX_ABS_DIFF;
     double acc = 0.0;
-    const int cpr = (ga.nx + 255) / 256;  // chunks per x-row
-    const long items = (long)ga.ny * ga.nz * cpr;
-    for (long w = blockIdx.x; w < items; w += gridDim.x) {
-        const long r = w / cpr;
-        const int i = (int)(w - r * cpr) * 256 + (int)threadIdx.x;
-        const int j = (int)(r % ga.ny);
-        const int k = (int)(r / ga.ny);
-        if (i >= ga.nx) continue;
-        if (inner_only && is_border(ga, i, j, k)) continue;
-        const double x = (double)a[at(ga, i, j, k)];
-        const double y = b ? (double)b[at(gb, i, j, k)] : 0.0;
-        if (op == RED_MAX_ABS_DIFF) {
-            const double d = fabs(x - y);
-            acc = d > acc ? d : acc;
-        } else if (op == RED_SUM_SQ_DIFF) {
-            const double d = x - y;
-            acc += d * d;
-        } else {
-            acc += x * y;
+    // four vectors' loads in flight per thread
+    constexpr int U = 4;
+    const I stride = gridDim.x * 256u;
+    for (I base = blockIdx.x * 256u + threadIdx.x; base < items; base += U * stride) {
+        vec x[U], y[U];
+        int i0[U], is[U], j[U], k[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const I w = base + u * stride < items ? base + u * stride : items - 1;
+            const I r = w / (unsigned)cpr;
+            i0[u] = (int)(w - r * (unsigned)cpr) * V;
+            is[u] = min(i0[u], ga.nx - V);
+            if (base + u * stride >= items) i0[u] = ga.nx;  // none of its nodes
+            k[u] = (int)(r / (unsigned)ga.ny);
+            j[u] = (int)(r - (I)k[u] * (unsigned)ga.ny);
+            x[u] = *(const vec*)(a + at(ga, is[u], j[u], k[u]));
+#pragma unroll
+            for (int q = 0; q < V; ++q) y[u][q] = T(0);
+            if (b) y[u] = *(const vec*)(b + at(gb, is[u], j[u], k[u]));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool plane = (inner_only == 0) | ((j[u] >= ga.nl1) & (j[u] <= ga.ny - 1 - ga.nl1) &
+                                                    (k[u] >= ga.nl2) & (k[u] <= ga.nz - 1 - ga.nl2));
+#pragma unroll
+            for (int q = 0; q < V; ++q) {
+                const int i = is[u] + q;
+                const bool use = plane & (i >= i0[u]) &
+                                 ((inner_only == 0) | ((i >= ga.nl0) & (i <= ga.nx - 1 - ga.nl0)));
+                const double xd = (double)x[u][q], d = xd - (double)y[u][q];
+                if (is_max) acc = use & (fabs(d) > acc) ? fabs(d) : acc;
+                else if (use) acc += op == RED_SUM_SQ_DIFF ? d * d : xd * (double)y[u][q];
+            }
         }
     }
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            if (op == RED_MAX_ABS_DIFF) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-            else sh[threadIdx.x] += sh[threadIdx.x + s];
+    acc = wave_block_reduce<4>(acc, is_max, sh);
+    if (gridDim.x > kOnePassBlocks) {
+        if (threadIdx.x == 0) partial[blockIdx.x] = acc;
+        return;
+    }
+    if (gridDim.x > 1) {
+        if (threadIdx.x == 0) {
+            partial[blockIdx.x] = acc;
+            __threadfence();
+            last = atomicAdd(done, 1u) == gridDim.x - 1;
         }
         __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
-}
-
-__global__ __launch_bounds__(256) void reduce_final(const double* partial, int n, int op, double* out)
-{
-    __shared__ double sh[256];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        if (op == RED_MAX_ABS_DIFF) acc = fmax(acc, partial[i]);
-        else acc += partial[i];
-    }
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            if (op == RED_MAX_ABS_DIFF) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-            else sh[threadIdx.x] += sh[threadIdx.x + s];
+        if (!last) return;
+        __threadfence();
+        acc = 0.0;
+        for (unsigned q = threadIdx.x; q < gridDim.x; q += 256u) {
+            const double v = __hip_atomic_load(&partial[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            acc = is_max ? fmax(acc, v) : acc + v;
         }
-        __syncthreads();
+        acc = wave_block_reduce<4>(acc, is_max, sh);
+        if (threadIdx.x == 0) *done = 0;  // for the next reduction on this stream
     }
-    if (threadIdx.x == 0) out[0] = sh[0];
+    if (threadIdx.x == 0) *out = acc;
 }
 
-int reduce_partials(Ctx* c, int nblocks, double* out)
+__global__ __launch_bounds__(256) void reduce_final(const double* partial, int n, bool is_max, double* out)
 {
-    reduce_final<<<1, 256, 0, c->stream>>>(c->red_partial, nblocks, RED_SUM_SQ_DIFF, c->red_result);
+    __shared__ double sh[4];
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) acc = is_max ? fmax(acc, partial[i]) : acc + partial[i];
+    acc = wave_block_reduce<4>(acc, is_max, sh);
+    if (threadIdx.x == 0) *out = acc;
+}
+
+int reduce_partials(Ctx* c, int nblocks, int slot)
+{
+    reduce_final<<<1, 256, 0, c->stream>>>(c->red_partial, nblocks, false, c->host_result_dev + slot);
     SCAFES_HIP(hipGetLastError());
-    SCAFES_HIP(hipMemcpyAsync(c->host_result, c->red_result, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SCAFES_HIP(hipStreamSynchronize(c->stream));
-    *out = c->host_result[0];
     return SCAFES_OK;
+}
+
+template <typename T, int V>
+static int reduce_launch_v(Ctx* c, const Geo& ga, const Geo& gb, const T* a, const T* b, int op, int inner_only)
+{
+    const int cpr = ceil_div(ga.nx, V);
+    const unsigned long items = (unsigned long)cpr * ga.ny * ga.nz;
+    // one round of four vectors a thread while the partials last
+    const int blocks = (int)std::max(1UL, std::min((items + 1023) / 1024, (unsigned long)c->red_capacity));
+    unsigned* done = reinterpret_cast<unsigned*>(c->red_done);
+    if (items < 0xf0000000UL)  // 32-bit vector numbers, the stride's overshoot included
+        reduce_kernel<T, V, unsigned><<<blocks, 256, 0, c->stream>>>(ga, gb, a, b, op, inner_only, cpr,
+                                                                     (unsigned)items, c->red_partial, done,
+                                                                     c->host_result_dev);
+    else
+        reduce_kernel<T, V, unsigned long><<<blocks, 256, 0, c->stream>>>(ga, gb, a, b, op, inner_only, cpr, items,
+                                                                          c->red_partial, done, c->host_result_dev);
+    SCAFES_HIP(hipGetLastError());
+    if (blocks > kOnePassBlocks) {
+        reduce_final<<<1, 256, 0, c->stream>>>(c->red_partial, blocks, op == RED_MAX_ABS_DIFF, c->host_result_dev);
+        SCAFES_HIP(hipGetLastError());
+    }
+    return SCAFES_OK;
+}
+
+template <typename T>
+static int reduce_launch(Ctx* c, const Geo& ga, const Geo& gb, const T* a, const T* b, int op, int inner_only)
+{
+    constexpr int W = 16 / (int)sizeof(T);
+    return ga.nx >= W ? reduce_launch_v<T, W>(c, ga, gb, a, b, op, inner_only)
+                      : reduce_launch_v<T, 1>(c, ga, gb, a, b, op, inner_only);
 }
 
 int reduce_nodes(Ctx* c, const Geo& ga, const Geo& gb, int dtype, const void* a, const void* b,
                  int op, int inner_only, double* out)
 {
-    const long total = (long)ga.nx * ga.ny * ga.nz;
-    int blocks = ceil_div(total, 256 * 8);
-    if (blocks > c->red_capacity) blocks = c->red_capacity;
-    if (blocks < 1) blocks = 1;
-    if (dtype == SCAFES_F64)
-        reduce_kernel<double><<<blocks, 256, 0, c->stream>>>(ga, gb, (const double*)a,
-                                                             (const double*)b, op, inner_only,
-                                                             c->red_partial);
-    else
-        reduce_kernel<float><<<blocks, 256, 0, c->stream>>>(ga, gb, (const float*)a,
-                                                            (const float*)b, op, inner_only,
-                                                            c->red_partial);
-    SCAFES_HIP(hipGetLastError());
-    reduce_final<<<1, 256, 0, c->stream>>>(c->red_partial, blocks, op, c->red_result);
-    SCAFES_HIP(hipGetLastError());
-    SCAFES_HIP(hipMemcpyAsync(c->host_result, c->red_result, sizeof(double),
-                              hipMemcpyDeviceToHost, c->stream));
+    const int rc = dtype == SCAFES_F64
+                       ? reduce_launch<double>(c, ga, gb, (const double*)a, (const double*)b, op, inner_only)
+                       : reduce_launch<float>(c, ga, gb, (const float*)a, (const float*)b, op, inner_only);
+    if (rc) return rc;
     SCAFES_HIP(hipStreamSynchronize(c->stream));
-    *out = c->host_result[0];
+    *out = *(volatile double*)c->host_result;
     return SCAFES_OK;
 }
 
@@ -327,7 +386,8 @@ int scafes_ctx_create(int device, scafes_ctx** out)
     SCAFES_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     c->red_capacity = 4096;
     SCAFES_HIP(hipMalloc(&c->red_partial, sizeof(double) * c->red_capacity));
-    SCAFES_HIP(hipMalloc(&c->red_result, sizeof(double) * 8));
+    SCAFES_HIP(hipMalloc(&c->red_done, sizeof(double)));
+    SCAFES_HIP(hipMemset(c->red_done, 0, sizeof(double)));
     SCAFES_HIP(hipHostMalloc(&c->host_result, sizeof(double) * 8, hipHostMallocDefault));
     SCAFES_HIP(hipHostGetDevicePointer((void**)&c->host_result_dev, c->host_result, 0));
     SCAFES_HIP(hipEventCreateWithFlags(&c->ready, hipEventDisableTiming));
@@ -385,7 +445,7 @@ int scafes_ctx_destroy(scafes_ctx* ctx)
     if (c->grad_ws) (void)hipFree(c->grad_ws);
     if (c->batch_exec) (void)hipGraphExecDestroy(c->batch_exec);
     if (c->red_partial) (void)hipFree(c->red_partial);
-    if (c->red_result) (void)hipFree(c->red_result);
+    if (c->red_done) (void)hipFree(c->red_done);
     if (c->host_result) (void)hipHostFree(c->host_result);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;

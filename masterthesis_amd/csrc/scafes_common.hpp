@@ -33,7 +33,7 @@ struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     double* red_partial = nullptr;  // per-block reduction partials (device)
-    double* red_result = nullptr;   // final reduction values (device, 8 slots)
+    double* red_done = nullptr;     // count of a reduction's finished blocks (0 between reductions)
     // pinned host memory that kernels write their results to (8 slots), and the
     // device's address of it; a call that uses it waits before it returns
     double* host_result = nullptr;
@@ -254,8 +254,9 @@ int yee_tb2_launch(Ctx* c, const YeeDims& d, const Tb2Plan& pl, T s, const T* a,
 // Reductions (defined in scafes_capi.hip).
 enum RedOp { RED_MAX_ABS_DIFF = 0, RED_SUM_SQ_DIFF = 1, RED_SUM_PROD = 2 };
 // Sum of the first nblocks entries of c->red_partial (per-block FP64 partial
-// sums a kernel wrote there, nblocks <= c->red_capacity), waited for.
-int reduce_partials(Ctx* c, int nblocks, double* out);
+// sums a kernel wrote there, nblocks <= c->red_capacity) to host_result[slot];
+// valid once the stream has been waited for.
+int reduce_partials(Ctx* c, int nblocks, int slot);
 int reduce_nodes(Ctx* c, const Geo& ga, const Geo& gb, int dtype, const void* a, const void* b,
                  int op, int inner_only, double* out);
 

@@ -114,3 +114,33 @@ def test_pennes_row_ends(ctx, dtype, n):
     np.testing.assert_allclose(grad.read(t.shape)[inner], gr, rtol=0, atol=20 * 4 * 2.0 ** -53)
     for x in (a, b, dw, dq, grad):
         x.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [(1,), (2, 3), (3, 5, 4), (5, 3, 2), (32, 24, 20), (33, 17, 9), (130, 70, 61)])
+@pytest.mark.parametrize("inner", [0, 1])
+def test_reductions_row_ends(ctx, dtype, n, inner):
+    """Every node counted once, ghosts (NaN) never, over one block and many,
+    and again right after (the block counter is back at zero).  Sums: FP64, in
+    any order, nodes x 2^-53 of the summed magnitudes."""
+    rng = np.random.default_rng(sum(n))
+    a, b = (_nodes(rng, n, rng.standard_normal).astype(dtype) for _ in range(2))
+    sl = tuple(slice(1, -1) for _ in n)
+    x, y = a[sl].astype(np.float64), np.ascontiguousarray(b[sl])
+    yd = y.astype(np.float64)
+    da, db = ctx.upload(a), ctx.upload(y)  # b as a field without ghosts
+    g = capi.geom(n, h=[0.5] * len(n))
+    keep = np.ones(x.shape, bool)
+    if inner:
+        keep[...] = False
+        keep[tuple(slice(1, -1) for _ in n)] = True
+    code = capi.F32 if dtype == np.float32 else capi.F64
+    out = C.c_double(0)
+    for op in (0, 1, 2, 0):
+        capi.check(ctx.L.scafes_reduce(ctx.h, C.byref(g), code, da.ptr, 1, db.ptr, 0, op, inner, C.byref(out)))
+        terms = (np.abs(x - yd), (x - yd) ** 2, x * yd)[op][keep]
+        want = (terms.max() if terms.size else 0.0) if op == 0 else terms.sum()
+        tol = 0.0 if op == 0 else 2.0 * terms.size * 2.0 ** -53 * np.abs(terms).sum()
+        assert abs(out.value - want) <= tol, (op, out.value, want)
+    da.free()
+    db.free()
