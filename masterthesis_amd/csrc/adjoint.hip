@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "scafes_common.hpp"
+#include "stepk.hpp"
 
 namespace scafes {
 
@@ -142,7 +143,7 @@ struct Rev {
         if (family == FAMILY_HEATVAR)
             return heat7var_step_one(c, geo, g, heat_mode, a, b, lo(a), lo(b), kappa, tau, border_mode,
                                      border_value);
-        return pennes_step_launch(c, geo, g, dtype, a, b, w, q, p, lo(a), lo(b));
+        return pennes_step_launch(c, geo, g, dtype, a, b, w, q, p, lo(a), lo(b), 1, nullptr);
     }
     // the library's device copy kernel (about 1.8x the runtime's copy rate)
     int copy(void* dst, const void* src)
@@ -162,6 +163,8 @@ struct Rev {
             int k = 1;
             if (yee2 && n - done >= 2) k = 2;
             if (family == FAMILY_HEATVAR) k = heat7var_next_sweep(c, geo, heat_mode, n - done);
+            if (family == FAMILY_PENNES && pennes_steps_supported(geo, dtype, p->border_mode, false))
+                k = steps_of_sweep(n - done);
             done += k;
             void* out = (done == n) ? dst : (x == tmp[0] ? tmp[1] : tmp[0]);
             if (out == x) out = (x == tmp[0]) ? tmp[1] : tmp[0];
@@ -170,6 +173,8 @@ struct Rev {
                 fwd_steps += k;
                 if (family == FAMILY_YEE_EPS)
                     r = yee_eps_step2(c, yd, dtype, yee_s, ce, x, out);
+                else if (family == FAMILY_PENNES)
+                    r = pennes_step_launch(c, geo, g, dtype, x, out, w, q, p, lo(x), lo(out), k, nullptr);
                 else
                     r = heat7var_sweep_k(c, geo, g, heat_mode, k, x, out, lo(x), lo(out), kappa, tau, border_mode,
                                          border_value);
@@ -327,25 +332,52 @@ struct Rev {
         return r;
     }
 
-    // How the variable-kappa family forms `total` consecutive states:
-    // `single` one-step sweeps first, then `q4` four-step and the rest
-    // three-step state-writing sweeps.  Four-step sweeps (where the mode has
-    // them) replace the one or two single steps a total that is not a
-    // multiple of three would leave (4 = 4, 8 = 4 + 4, 10 = 4 + 3 + 3).
-    void states_plan(long total, long* single, long* q4) const
+    // The sweeps that form `total` consecutive states, in order, as steps per
+    // sweep (1: a plain step).  Pennes: three per state-writing sweep, two in
+    // the remainder.  Variable kappa: single steps first, then three-step
+    // sweeps; four-step sweeps (where the mode has them) replace the one or
+    // two single steps a total that is not a multiple of three would leave (4
+    // = 4, 8 = 4 + 4, 10 = 4 + 3 + 3).
+    std::vector<int> states_plan(long total) const
     {
-        *single = total;
-        *q4 = 0;
-        if (total < 3 || !heat7var_states_sweep_ok(c, geo, heat_mode)) return;
-        *single = total % 3;
-        if (!heat7var_states4_ok(c, geo, heat_mode)) return;
-        if (*single == 1 && total >= 4) {
-            *q4 = 1;
-            *single = 0;
-        } else if (*single == 2 && total >= 8) {
-            *q4 = 2;
-            *single = 0;
+        std::vector<int> plan;
+        if (family == FAMILY_PENNES && pennes_steps_supported(geo, dtype, p->border_mode, true)) {
+            for (long left = total; left > 0; left -= plan.back()) plan.push_back(steps_of_sweep(left));
+            return plan;
         }
+        long single = total, q4 = 0;
+        if (family == FAMILY_HEATVAR && total >= 3 && heat7var_states_sweep_ok(c, geo, heat_mode)) {
+            single = total % 3;
+            if (heat7var_states4_ok(c, geo, heat_mode)) {
+                if (single == 1 && total >= 4) {
+                    q4 = 1;
+                    single = 0;
+                } else if (single == 2 && total >= 8) {
+                    q4 = 2;
+                    single = 0;
+                }
+            }
+        }
+        plan.assign((size_t)single, 1);
+        plan.insert(plan.end(), (size_t)q4, 4);
+        plan.insert(plan.end(), (size_t)((total - single - 4 * q4) / 3), 3);
+        return plan;
+    }
+    // k >= 2 steps from x to sk[k-1], the states in between to sk[0..k-2]
+    // (the variable-kappa family writes their value parts only, all its
+    // adjoint reads).
+    int sweep_states(int k, const void* x, void* const* sk)
+    {
+        fwd_steps += k;
+        if (family == FAMILY_HEATVAR)
+            return heat7var_sweep_states(c, geo, g, heat_mode, k, x, sk[k - 1], lo(x), lo(sk[k - 1]), sk, kappa, tau,
+                                         border_mode, border_value);
+        StepMid mid{};
+        for (int l = 0; l < k - 1; ++l) {
+            mid.v[l] = sk[l];
+            mid.c[l] = lo(sk[l]);
+        }
+        return pennes_step_launch(c, geo, g, dtype, x, sk[k - 1], w, q, p, lo(x), lo(sk[k - 1]), k, &mid);
     }
 
     // Where snapshots are plentiful the binomial split takes one step off
@@ -370,33 +402,20 @@ struct Rev {
                 ++len;
             }
         }
-        // The variable-kappa family forms the peeled states three or four per
-        // sweep where the grid's sweeps can write the states in between
-        // (value parts, all the adjoint reads), the rest first one step at a
-        // time, so the run's last state (the right part's base) is whole.
+        // The peeled states are formed several per sweep where the grid's sweeps
+        // can write the states in between; the run's last state (the right
+        // part's base) is the output of a sweep or a step, so it is whole.
         std::vector<const void*> chain(1, base);  // chain[q] = T^{a+q}
-        long single = len, q4 = 0;
-        if (family == FAMILY_HEATVAR) states_plan(len, &single, &q4);
         int r = SCAFES_OK;
-        for (long q = 0; q < single && !r; ++q) {
-            void* sl = slots.back();
-            slots.pop_back();
-            r = advance(chain.back(), 1, sl);
-            chain.push_back(sl);
-        }
-        while (!r && (long)chain.size() - 1 < len) {
-            const int k = q4 > 0 ? 4 : 3;
-            if (q4 > 0) --q4;
+        for (const int k : states_plan(len)) {
             void* sk[4];
             for (int q = 0; q < k; ++q) {
                 sk[q] = slots.back();
                 slots.pop_back();
             }
-            const void* x = chain.back();
-            r = heat7var_sweep_states(c, geo, g, heat_mode, k, x, sk[k - 1], lo(x), lo(sk[k - 1]), sk, kappa, tau,
-                                      border_mode, border_value);
-            fwd_steps += k;
+            r = k == 1 ? step(chain.back(), sk[0]) : sweep_states(k, chain.back(), sk);
             for (int q = 0; q < k; ++q) chain.push_back(sk[q]);
+            if (r) break;
         }
         const long aa = a + len;
         const int ss = s - (int)len;
@@ -432,28 +451,16 @@ int Rev::treeverse(long a, long b, int s, const void* base)
             // take), then the steps are reversed up to kAdjMaxK per sweep.
             std::vector<const void*> st(1, base);  // st[q] = T^{a+q}
             int r = SCAFES_OK;
-            // The variable-kappa family takes the first states one step at a
-            // time, the rest three or four per sweep with the states in
-            // between written by the same sweep (value parts only: its
-            // adjoint reads no more), so that the last state of each sweep is
-            // whole.  Where the stretch ends at N and lam^N is not set yet,
-            // T^N is the last sweep's output (into tmp[0]): the m + 1 states
-            // are split instead of m and one more step for T^N.
+            // Several states per sweep as in peel_run.  Where the stretch ends
+            // at N and lam^N is not set yet, T^N is the last sweep's output
+            // (into tmp[0]): the m + 1 states are split instead of m and one
+            // more step for T^N.
             const long m = b - a - 1;
-            const bool sweeps = family == FAMILY_HEATVAR && heat7var_states_sweep_ok(c, geo, heat_mode);
+            const bool sweeps = (family == FAMILY_HEATVAR && heat7var_states_sweep_ok(c, geo, heat_mode)) ||
+                                (family == FAMILY_PENNES && pennes_steps_supported(geo, dtype, p->border_mode, true));
             const bool leaf = sweeps && b == nsteps && !lam_ready && m + 1 >= 3;
             const long total = leaf ? m + 1 : m;  // states this stretch forms
-            long single = m, q4 = 0;
-            if (family == FAMILY_HEATVAR) states_plan(total, &single, &q4);
-            for (long q = 1; q <= single && !r; ++q) {
-                void* sl = slots.back();
-                slots.pop_back();
-                r = step(st.back(), sl);
-                st.push_back(sl);
-            }
-            while (!r && (long)st.size() - 1 < total) {
-                const int k = q4 > 0 ? 4 : 3;
-                if (q4 > 0) --q4;
+            for (const int k : states_plan(total)) {
                 const bool to_leaf = leaf && (long)st.size() - 1 + k == total;
                 void* sk[4];
                 for (int q = 0; q < k; ++q) {
@@ -464,13 +471,9 @@ int Rev::treeverse(long a, long b, int s, const void* base)
                         slots.pop_back();
                     }
                 }
-                const void* x = st.back();
-                r = heat7var_sweep_states(c, geo, g, heat_mode, k, x, sk[k - 1], lo(x), lo(sk[k - 1]), sk, kappa,
-                                          tau, border_mode, border_value);
-                fwd_steps += k;
-                for (int q = 0; q < k - 1; ++q) st.push_back(sk[q]);
-                if (to_leaf) break;
-                st.push_back(sk[k - 1]);
+                r = k == 1 ? step(st.back(), sk[0]) : sweep_states(k, st.back(), sk);
+                for (int q = 0; q < k - (to_leaf ? 1 : 0); ++q) st.push_back(sk[q]);
+                if (r) break;
             }
             if (!r && leaf) r = first_leaf(nullptr);
             for (long n = b; n > a && !r;) {

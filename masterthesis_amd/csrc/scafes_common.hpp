@@ -130,9 +130,16 @@ int fit_chunk(long nxy, int nz, int fill, int zmax, int per_cu, int cu_count);
 // Pennes forward / adjoint launches (defined in stencil3d.hip).
 // dtype SCAFES_F32_KAHAN: compensated FP32 forward (cin/cout compensation fields);
 // tprev_lo != null: the adjoint reads the forward state as a (hi, lo) pair.
+// k = 1, or 2..3 steps in one sweep (pennes_steps_supported), mid (nullable):
+// the states after 1..k-1 of them are written too.
+struct StepMid;
 int pennes_step_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, const void* t_old,
                        void* t_new, const void* w, const void* q, const scafes_pennes_params* p,
-                       const void* cin, void* cout);
+                       const void* cin, void* cout, int k, const StepMid* mid);
+// Where sweeps of two and three Pennes steps (states: with the states in between
+// written) exist for the grid and beat single steps.
+bool pennes_steps_supported(const Geo& geo, int dtype, int border_mode, bool states);
+int steps_of_sweep(long left);
 int pennes_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, const void* lam,
                       void* lam_new, const void* w, const void* tprev, double* grad,
                       const scafes_pennes_params* p, const void* tprev_lo);

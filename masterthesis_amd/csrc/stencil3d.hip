@@ -26,19 +26,9 @@
 #include "exact_quot.hpp"
 #include "heatvar_ops.hpp"
 #include "scafes_common.hpp"
+#include "stepk.hpp"
 
 namespace scafes {
-
-template <typename T>
-struct St7 {
-    T c, w, e, s, n, d, u;  // centre, x-, x+, y-, y+, z-, z+
-};
-
-template <typename T>
-struct Res {
-    T v, c;
-    double g;
-};
 
 // ---------------------------------------------------------------- skeleton
 // D = prefetch depth in planes (even, >= 2).  Every value a thread needs for
@@ -350,15 +340,21 @@ struct HeatConstOp {
         }
         return t - 2.0 * u;
     }
+    // An inner node without its source, and a border node without known fields.
+    __device__ void inner(int dim, const St7<double>& s, const double*, Res<double>& r) const
+    {
+        double v = add_by_hh(hh, dim, s.c, ctau_a * ((s.w + s.e) - 2.0 * s.c), ctau_a * ((s.s + s.n) - 2.0 * s.c),
+                             ctau_a * ((s.d + s.u) - 2.0 * s.c));
+        if (has_perf) v -= ctw * s.c;
+        r.v = v;
+    }
+    __device__ double kept(double c) const { return border_mode == SCAFES_BORDER_VALUE ? border_value : c; }
     __device__ void apply(const Geo& g, int i, int j, int k, const St7<double>& s,
                           const St7<double>&, const St7<double>&, const double*, Res<double>& r) const
     {
         if (!is_border(g, i, j, k)) {
-            double v = add_by_hh(hh, g.dim, s.c, ctau_a * ((s.w + s.e) - 2.0 * s.c),
-                                 ctau_a * ((s.s + s.n) - 2.0 * s.c), ctau_a * ((s.d + s.u) - 2.0 * s.c));
-            if (has_perf) v -= ctw * s.c;
-            if (has_source) v += ctf * f_old[at(gk, i, j, k)];
-            r.v = v;
+            inner(g.dim, s, nullptr, r);
+            if (has_source) r.v += ctf * f_old[at(gk, i, j, k)];
         } else if (border_mode == SCAFES_BORDER_FIELD) {
             r.v = g_new[at(gk, i, j, k)];
         } else if (border_mode == SCAFES_BORDER_VALUE) {
@@ -469,6 +465,31 @@ struct PennesOp {
         if (idx == 0) return ((ev + (a * (T)qbc)) + ev) - (T)2 * c;
         return (wv + ev) - (T)2 * c;
     }
+    __device__ void inner(int dim, const St7<T>& s, const T* xv, Res<T>& r) const
+    {
+        if constexpr (sizeof(T) == 8) {
+            double v = add_by_hh(hh, dim, s.c, ctd * ((s.w + s.e) - 2.0 * s.c), ctd * ((s.s + s.n) - 2.0 * s.c),
+                                 ctd * ((s.d + s.u) - 2.0 * s.c));
+            v += (ctp * xv[0]) * (ta - s.c);
+            v += ctq * xv[1];
+            r.v = v;
+        } else {
+            float d = fd0 * ((s.w + s.e) - 2.0f * s.c);
+            if (dim > 1) d = __builtin_fmaf(fd1, (s.s + s.n) - 2.0f * s.c, d);
+            if (dim > 2) d = __builtin_fmaf(fd2, (s.d + s.u) - 2.0f * s.c, d);
+            d = __builtin_fmaf(fp * xv[0], fta - s.c, d);
+            d = __builtin_fmaf(fq, xv[1], d);
+            if constexpr (KAHAN) {
+                const float y = d + xv[2];
+                const float t = s.c + y;
+                r.c = y - (t - s.c);
+                r.v = t;
+            } else {
+                r.v = s.c + d;
+            }
+        }
+    }
+    __device__ T kept(T c) const { return c; }
     __device__ void apply(const Geo& g, int i, int j, int k, const St7<T>& s, const St7<T>&,
                           const St7<T>&, const T* xv, Res<T>& r) const
     {
@@ -506,27 +527,7 @@ struct PennesOp {
             }
             return;
         }
-        if constexpr (sizeof(T) == 8) {
-            double v = add_by_hh(hh, g.dim, s.c, ctd * ((s.w + s.e) - 2.0 * s.c), ctd * ((s.s + s.n) - 2.0 * s.c),
-                                 ctd * ((s.d + s.u) - 2.0 * s.c));
-            v += (ctp * xv[0]) * (ta - s.c);
-            v += ctq * xv[1];
-            r.v = v;
-        } else {
-            float d = fd0 * ((s.w + s.e) - 2.0f * s.c);
-            if (g.dim > 1) d = __builtin_fmaf(fd1, (s.s + s.n) - 2.0f * s.c, d);
-            if (g.dim > 2) d = __builtin_fmaf(fd2, (s.d + s.u) - 2.0f * s.c, d);
-            d = __builtin_fmaf(fp * xv[0], fta - s.c, d);
-            d = __builtin_fmaf(fq, xv[1], d);
-            if constexpr (KAHAN) {
-                const float y = d + xv[2];
-                const float t = s.c + y;
-                r.c = y - (t - s.c);
-                r.v = t;
-            } else {
-                r.v = s.c + d;
-            }
-        }
+        inner(g.dim, s, xv, r);
     }
 };
 
@@ -887,6 +888,27 @@ static int launch(Ctx* c, const Op& op, const Geo& g, int cfg)
     }
 }
 
+// FP64 grids up to this size keep a step's four arrays in the Infinity Cache
+// (256 MB), where single steps are as fast as sweeps (the figures in stepk.hpp).
+constexpr long kCachedNodes64 = 8000000L;
+
+// Steps of the next sweep of a run of one-field updates with `left` to go:
+// three, a remainder of two or four in twos.
+int steps_of_sweep(long left) { return left == 1 ? 1 : left == 2 || left == 4 ? 2 : 3; }
+
+// k = 1..3 steps; mid: the states after 1..k-1 of them are written too.
+template <class Op, typename T>
+static int launch_steps(Ctx* c, const Op& op, const Geo& g, int k, const StepMid* mid)
+{
+    if (k == 1) return launch_auto<Op, T>(c, op, g);
+    if ((k != 2 && k != 3) || !stepk_supported(g, (int)sizeof(T)))
+        return fail(SCAFES_ERR_UNSUPPORTED, "no sweep of this many steps for this grid");
+    if (!mid) return k == 2 ? stepk_launch<Op, T, 2, false>(c, op, g, {}) : stepk_launch<Op, T, 3, false>(c, op, g, {});
+    if constexpr (Op::kNX > 0)
+        return k == 2 ? stepk_launch<Op, T, 2, true>(c, op, g, *mid) : stepk_launch<Op, T, 3, true>(c, op, g, *mid);
+    return fail(SCAFES_ERR_UNSUPPORTED, "no state-writing sweep of this update");
+}
+
 static void hh_of(const scafes_geom* g, double hh[3])
 {
     for (int p = 0; p < 3; ++p) hh[p] = p < g->dim ? g->h[p] * g->h[p] : 1.0;
@@ -944,9 +966,17 @@ int heat7var_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, cons
     return launch<HeatVarOp<float, 2>, float>(c, op, geo, cfg);
 }
 
+bool pennes_steps_supported(const Geo& geo, int dtype, int border_mode, bool states)
+{
+    const long nodes = (long)geo.nx * geo.ny * geo.nz;
+    if (border_mode != SCAFES_BORDER_KEEP || !stepk_supported(geo, dtype == SCAFES_F64 ? 8 : 4)) return false;
+    if (dtype == SCAFES_F64) return nodes > kCachedNodes64;
+    return dtype == SCAFES_F32_KAHAN || !states || nodes < 1000000L || nodes > 3000000L;
+}
+
 int pennes_step_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, const void* t_old,
                        void* t_new, const void* w, const void* q, const scafes_pennes_params* p,
-                       const void* cin, void* cout)
+                       const void* cin, void* cout, int k, const StepMid* mid)
 {
     double hh[3];
     hh_of(g, hh);
@@ -973,7 +1003,7 @@ int pennes_step_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
         op.ta = p->t_a;
         op.hh = make_by_hh(hh);
         if (p->border_mode == SCAFES_BORDER_TUMOR) tumor(op);
-        return launch<PennesOp<double>, double>(c, op, geo, -1);
+        return launch_steps<PennesOp<double>, double>(c, op, geo, k, mid);
     }
     auto fill32 = [&](auto& op) {
         op.a = (const float*)t_old;
@@ -995,11 +1025,11 @@ int pennes_step_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
         fill32(op);
         op.x[2] = (const float*)cin;
         op.cout = (float*)cout;
-        return launch<PennesOp<float, true>, float>(c, op, geo, -1);
+        return launch_steps<PennesOp<float, true>, float>(c, op, geo, k, mid);
     }
     PennesOp<float> op{};
     fill32(op);
-    return launch<PennesOp<float>, float>(c, op, geo, -1);
+    return launch_steps<PennesOp<float>, float>(c, op, geo, k, mid);
 }
 
 // The one-step tile of a mode: the 512^3 one where its long chunks make at
@@ -1244,19 +1274,20 @@ int scafes_heat7_run_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, double* 
     HeatConstOp op;
     int rc = heat7_const_op(c, g, hw, u, u2, nullptr, nullptr, nullptr, p, &geo, &op);
     if (rc) return rc;
-    // One launch per step; a HIP graph of the launches (captured once,
-    // replayed) was measured at heat 64^3 FP64, 100 steps: 0.488 ms against
-    // 0.499 ms, so the steps are kernel-bound (about 5 us each), not
-    // launch-bound, and the graph was not kept.
+    const long nodes = (long)geo.nx * geo.ny * geo.nz;
+    const bool multi = stepk_supported(geo, 8) && (nodes <= 300000L || nodes > kCachedNodes64);
     double *a = u, *b = u2;
-    for (int s = 0; s < nsteps; ++s) {
+    int sweeps = 0;
+    for (int s = 0; s < nsteps; ++sweeps) {
+        const int k = multi ? steps_of_sweep(nsteps - s) : 1;
         op.a = a;
         op.out = b;
-        rc = launch<HeatConstOp, double>(c, op, geo, -1);
+        rc = launch_steps<HeatConstOp, double>(c, op, geo, k, nullptr);
         if (rc) return rc;
         std::swap(a, b);
+        s += k;
     }
-    if (result_in_second) *result_in_second = nsteps % 2;
+    if (result_in_second) *result_in_second = sweeps % 2;
     return SCAFES_OK;
 }
 
@@ -1525,7 +1556,7 @@ int scafes_pennes_step(scafes_ctx* ctx, const scafes_geom* g, int hw, int dtype,
     if (dtype != SCAFES_F32 && dtype != SCAFES_F64) return fail(SCAFES_ERR_ARG, "pennes: dtype F32 or F64");
     rc = pennes_check_tau(c, geo, g, hw, dtype, w, p, true, "pennes");
     if (rc) return rc;
-    return pennes_step_launch(c, geo, g, dtype, t_old, t_new, w, q, p, nullptr, nullptr);
+    return pennes_step_launch(c, geo, g, dtype, t_old, t_new, w, q, p, nullptr, nullptr, 1, nullptr);
 }
 
 int scafes_pennes_step_kahan(scafes_ctx* ctx, const scafes_geom* g, int hw, const float* t_old, float* t_new,
@@ -1543,7 +1574,7 @@ int scafes_pennes_step_kahan(scafes_ctx* ctx, const scafes_geom* g, int hw, cons
     if (rc) return rc;
     rc = pennes_check_tau(c, geo, g, hw, SCAFES_F32, w, p, true, "pennes kahan");
     if (rc) return rc;
-    return pennes_step_launch(c, geo, g, SCAFES_F32_KAHAN, t_old, t_new, w, q, p, c_old, c_new);
+    return pennes_step_launch(c, geo, g, SCAFES_F32_KAHAN, t_old, t_new, w, q, p, c_old, c_new, 1, nullptr);
 }
 
 int scafes_mri_coef_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, const double* const* mat,

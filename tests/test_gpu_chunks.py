@@ -144,3 +144,59 @@ def test_reductions_row_ends(ctx, dtype, n, inner):
         assert abs(out.value - want) <= tol, (op, out.value, want)
     da.free()
     db.free()
+
+
+@pytest.mark.parametrize("n", [(5, 4, 3), (60, 8, 32), (61, 9, 33), (64, 64, 64), (130, 21, 7), (210, 200, 200)])
+@pytest.mark.parametrize("steps", [2, 3, 4, 8])
+def test_heat_run_equals_single_steps(ctx, n, steps):
+    """scafes_heat7_run_f64 over grids whose run takes several steps per sweep
+    (small and large ones) against one call per step, with perfusion."""
+    rng = np.random.default_rng(sum(n))
+    g = capi.geom(n)
+    shape = tuple(m + 2 for m in reversed(n))
+    u0 = np.full(shape, np.nan)
+    u0[1:-1, 1:-1, 1:-1] = rng.standard_normal(tuple(reversed(n)))
+    tau = 0.9 / (sum(2 * (m - 1.0) ** 2 for m in n) + 1.0)
+    p = capi.Heat7Params(tau=tau, coeff_a=1.0, rhoc_inv=1.0, perf_c=1.0, perf_w=1.0, has_perf=1,
+                         border_mode=capi.BORDER_VALUE, border_value=0.5)
+    a, b = ctx.upload(u0), ctx.upload(u0)
+    which = C.c_int(0)
+    capi.check(ctx.L.scafes_heat7_run_f64(ctx.h, C.byref(g), 1, a.ptr, b.ptr, steps, C.byref(p), C.byref(which)))
+    got = (b if which.value else a).read(shape)[1:-1, 1:-1, 1:-1]
+    a.write(u0)
+    for _ in range(steps):
+        capi.check(ctx.L.scafes_heat7_step_f64(ctx.h, C.byref(g), 1, a.ptr, b.ptr, None, None, None, C.byref(p)))
+        a, b = b, a
+    assert np.array_equal(got, a.read(shape)[1:-1, 1:-1, 1:-1])
+    a.free()
+    b.free()
+
+
+@pytest.mark.parametrize("code", [capi.F32, capi.F64, capi.F32_KAHAN])
+@pytest.mark.parametrize("n", [(6, 5, 4), (61, 9, 33), (70, 33, 20), (210, 200, 200)])
+@pytest.mark.parametrize("steps", [4, 7, 9])
+def test_pennes_gradient_same_for_every_budget(ctx, code, n, steps):
+    """States formed one, two or three per sweep, recomputed or stored: the
+    gradient is the same bits for every snapshot budget."""
+    if n[0] == 210 and steps != 7:
+        pytest.skip("one step count at the large size")
+    dt = np.float64 if code == capi.F64 else np.float32
+    rng = np.random.default_rng(sum(n) + steps)
+    g = capi.geom(n)
+    shape = tuple(m + 2 for m in reversed(n))
+    t0, w, q, tgt = (rng.random(shape).astype(dt) for _ in range(4))
+    p = capi.PennesParams(cdiff=0.5, cperf=1.0, csrc=1.0, t_a=0.0)
+    p.tau = 0.9 / (sum(2 * 0.5 * (m - 1.0) ** 2 for m in n) + 1.0)
+    bufs = [ctx.upload(v) for v in (t0, w, q, tgt)]
+    grad = ctx.alloc(t0.size, np.float64)
+    out = []
+    for snaps in (0, 1, 3, steps):
+        J = C.c_double(0)
+        capi.check(ctx.L.scafes_pennes_gradient(ctx.h, C.byref(g), 1, code, *[b.ptr for b in bufs], C.byref(p), steps,
+                                                snaps, grad.ptr, C.byref(J), None))
+        out.append((J.value, grad.read()))
+    assert out[0][0] > 0.0 and np.abs(out[0][1]).max() > 0.0
+    for J, gr in out[1:]:
+        assert J == out[0][0] and np.array_equal(gr, out[0][1])
+    for b in bufs + [grad]:
+        b.free()
