@@ -12,10 +12,16 @@
 // time.  Thread (tx, ty) keeps a B x B block of nodes (B = ceil(n/32) <= 8
 // for n <= 256) in registers for all steps (4 waves per SIMD leave 128
 // registers per lane).  Per step it publishes its block's four edges to LDS
-// (component-major, bank-conflict free) and reads its neighbours' edges
-// back: LDS traffic is one value per edge node instead of five per node,
-// and HBM is touched only to load and store each problem once.  Border
-// nodes take the update with a zero coefficient (fma(0, lap, u) = u).
+// (whole vectors, bank-conflict free) and reads its neighbours' edges back:
+// LDS traffic is one value per edge node instead of five per node, and HBM is
+// touched only to load and store each problem once.  Border nodes take the
+// update with a zero coefficient (fma(0, lap, u) = u): per column in a
+// register, per row only in the waves that hold the first, the last or padding
+// rows.  Bound by vector issue: six instructions per node and step.  Measured
+// on an MI355X, ms, a select, a product and two differences more per node, edges
+// by component, two barriers at every size -> now: 4096 problems of 32..256
+// nodes an edge, 500 steps with the gradient 15.04 -> 12.21; 512 of 256, 100
+// steps 0.983 -> 0.793; 3000 of 2..64, 300 steps 1.600 -> 1.103.
 // Each block size B is a separate non-inlined function, so each gets its
 // own register allocation: inlined into one kernel, the B = 8 body's
 // pressure would spill in every smaller body too.  Problems are taken in
@@ -40,7 +46,6 @@ namespace scafes {
 
 constexpr int kTX = 32, kTY = 32;  // workgroup shape
 constexpr int kNmax = 256;         // largest problem edge
-constexpr int kBmax = kNmax / kTX;
 
 struct BatchArgs {
     const int* n;
@@ -56,32 +61,98 @@ struct BatchArgs {
     int nsteps;
 };
 
-// Block edges published per step (LDS): top / bottom rows indexed
-// [column][ty][tx], left / right columns [row][ty][tx].
-__shared__ float eT[kBmax][kTY][kTX];
-__shared__ float eB[kBmax][kTY][kTX];
-__shared__ float eL[kBmax][kTY][kTX];
-__shared__ float eR[kBmax][kTY][kTX];
+// Block edges published per step (LDS): top and bottom rows, left and right
+// columns.  A thread's edge of B values is two vectors of at most 4, each
+// packed over the threads, so an edge takes one or two LDS instructions and no
+// bank conflicts.  Blocks of up to 4 x 4 need one vector per edge and alternate
+// between the two halves, so their steps need one barrier instead of two.
+__shared__ float4 eT[2][kTY * kTX];
+__shared__ float4 eB[2][kTY * kTX];
+__shared__ float4 eL[2][kTY * kTX];
+__shared__ float4 eR[2][kTY * kTX];
 __shared__ double red[2][kTX * kTY / 64];
+
+template <int N>
+struct EdgeVec {
+    typedef float type __attribute__((ext_vector_type(N == 3 ? 4 : N)));
+};
+template <>
+struct EdgeVec<1> {
+    typedef float type;
+};
+
+// v[FROM..FROM+N) of an edge to / from slot `at` of a packed array.
+template <int FROM, int N>
+__device__ __forceinline__ void put_part(float4* a, int at, const float* v)
+{
+    if constexpr (N == 1) {
+        reinterpret_cast<float*>(a)[at] = v[FROM];
+    } else if constexpr (N > 1) {
+        typename EdgeVec<N>::type x;
+#pragma unroll
+        for (int q = 0; q < N; ++q) x[q] = v[FROM + q];
+        if constexpr (N == 3) x[3] = 0.0f;
+        reinterpret_cast<typename EdgeVec<N>::type*>(a)[at] = x;
+    }
+}
+template <int FROM, int N>
+__device__ __forceinline__ void get_part(const float4* a, int at, float* v)
+{
+    if constexpr (N == 1) {
+        v[FROM] = reinterpret_cast<const float*>(a)[at];
+    } else if constexpr (N > 1) {
+        const typename EdgeVec<N>::type x = reinterpret_cast<const typename EdgeVec<N>::type*>(a)[at];
+#pragma unroll
+        for (int q = 0; q < N; ++q) v[FROM + q] = x[q];
+    }
+}
+template <int B>
+__device__ __forceinline__ void put(float4 (*a)[kTY * kTX], int buf, int at, const float* v)
+{
+    put_part<0, (B < 4 ? B : 4)>(a[B > 4 ? 0 : buf], at, v);
+    put_part<4, (B > 4 ? B - 4 : 0)>(a[1], at, v);
+}
+template <int B>
+__device__ __forceinline__ void get(const float4 (*a)[kTY * kTX], int buf, int at, float* v)
+{
+    get_part<0, (B < 4 ? B : 4)>(a[B > 4 ? 0 : buf], at, v);
+    get_part<4, (B > 4 ? B - 4 : 0)>(a[1], at, v);
+}
+
+__device__ __forceinline__ float* uniform_ptr(float* q)
+{
+    const unsigned long v = reinterpret_cast<unsigned long>(q);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return reinterpret_cast<float*>(((unsigned long)hi << 32) | lo);
+}
 
 template <int B>
 __device__ __attribute__((noinline)) void run_problem(const BatchArgs& a, int p)
 {
     const int tx = threadIdx.x, ty = threadIdx.y;
-    const int n = a.n[p];
+    // the problem's number and what follows from it are the same in every
+    // lane; a call passes them in vector registers, which the block needs
+    p = __builtin_amdgcn_readfirstlane(p);
+    const int n = __builtin_amdgcn_readfirstlane(a.n[p]);
+    const int nsteps = __builtin_amdgcn_readfirstlane(a.nsteps);
     const double h = 1.0 / (n - 1);
     const float ck = (float)((double)a.tau[p] * (double)a.kappa[p] / (h * h));
-    float* __restrict__ u = a.u + a.off[p];
-    const int ox = tx * B, oy = ty * B;
+    float* __restrict__ u = uniform_ptr(a.u + a.off[p]);
     // bit c of inx / iny: column ox+c / row oy+c is inner (1..n-2); vx / vy: is a node (< n)
-    unsigned inx = 0, iny = 0, vx = 0, vy = 0;
+    int ox = tx * B, oy = ty * B;
+    unsigned inx, iny, vx, vy;
+    auto masks = [&] {
+        inx = iny = vx = vy = 0;
 #pragma unroll
-    for (int c = 0; c < B; ++c) {
-        inx |= (ox + c >= 1 && ox + c <= n - 2) ? (1u << c) : 0u;
-        vx |= (ox + c < n) ? (1u << c) : 0u;
-        iny |= (oy + c >= 1 && oy + c <= n - 2) ? (1u << c) : 0u;
-        vy |= (oy + c < n) ? (1u << c) : 0u;
-    }
+        for (int c = 0; c < B; ++c) {
+            inx |= (ox + c >= 1 && ox + c <= n - 2) ? (1u << c) : 0u;
+            vx |= (ox + c < n) ? (1u << c) : 0u;
+            iny |= (oy + c >= 1 && oy + c <= n - 2) ? (1u << c) : 0u;
+            vy |= (oy + c < n) ? (1u << c) : 0u;
+        }
+    };
+    masks();
     float s[B][B];
 #pragma unroll
     for (int r = 0; r < B; ++r) {
@@ -89,40 +160,65 @@ __device__ __attribute__((noinline)) void run_problem(const BatchArgs& a, int p)
 #pragma unroll
         for (int c = 0; c < B; ++c) s[r][c] = ((vy >> r) & (vx >> c) & 1u) ? row[c] : 0.0f;
     }
+    // coefficient per column: 0 on border and padding columns, and everywhere
+    // in a thread without inner rows
+    float kc[B];
+#pragma unroll
+    for (int c = 0; c < B; ++c) kc[c] = ((inx >> c) & 1u) && iny ? ck : 0.0f;
+    // whether every row of every thread of this wave (two thread rows) is
+    // inner, or none of the thread's: then no row needs a mask
+    const bool plain = __all(iny == (1u << B) - 1u || iny == 0u);
+    const int t = tx + kTX * ty;
+    // neighbours' slots, clamped at the workgroup's edge: the nodes next to it
+    // are border or padding nodes (coefficient 0), so any finite value serves
+    const int tl = t - (tx > 0 ? 1 : 0), tr = t + (tx < kTX - 1 ? 1 : 0);
+    const int tu = t - (ty > 0 ? kTX : 0), td = t + (ty < kTY - 1 ? kTX : 0);
     const bool want_grad = a.target != nullptr;
     // One explicit step on the register block, rows top-down in place:
-    // prev[] keeps the old row above, `wold` the old left neighbour.  `last`
-    // (the final step when a gradient is wanted) stores u^N to HBM and keeps
-    // the inner nodes' L u^{N-1} terms (zero elsewhere) in the block.
-    auto step = [&](const bool last) {
-        // the masks live in VGPRs: scalar copies would be re-derived per use
-        asm volatile("" : "+v"(inx), "+v"(iny));
+    // prev[] keeps the old row above, `wold` the old left neighbour.  Second
+    // differences as fma(-2, u, W + E): 2u is exact, so the value is that of
+    // (W + E) - 2u (for |u| < 2^127).  masked: rows outside 1..n-2 take a zero
+    // coefficient.  last (the final step when a gradient is wanted) stores u^N
+    // and keeps the inner nodes' L u^{N-1} terms (zero elsewhere) in the block.
+    auto publish = [&](const int buf) {
+        float e[B];
+        put<B>(eT, buf, t, s[0]);
+        put<B>(eB, buf, t, s[B - 1]);
 #pragma unroll
-        for (int c = 0; c < B; ++c) {
-            eT[c][ty][tx] = s[0][c];
-            eB[c][ty][tx] = s[B - 1][c];
-        }
+        for (int r = 0; r < B; ++r) e[r] = s[r][0];
+        put<B>(eL, buf, t, e);
+#pragma unroll
+        for (int r = 0; r < B; ++r) e[r] = s[r][B - 1];
+        put<B>(eR, buf, t, e);
+    };
+    auto update = [&](const bool masked, const bool last, const int buf) {
+        float prev[B], lft[4], rgt[4], bot[B];
+        // opaque per step: hoisted, the masked coefficients would be spilled
+        if (masked) asm volatile("" : "+v"(iny));
+        get<B>(eB, buf, tu, prev);
 #pragma unroll
         for (int r = 0; r < B; ++r) {
-            eL[r][ty][tx] = s[r][0];
-            eR[r][ty][tx] = s[r][B - 1];
-        }
-        __syncthreads();
-        float prev[B];
-#pragma unroll
-        for (int c = 0; c < B; ++c) prev[c] = ty > 0 ? eB[c][ty - 1][tx] : 0.0f;
-#pragma unroll
-        for (int r = 0; r < B; ++r) {
-            float wold = tx > 0 ? eR[r][ty][tx - 1] : 0.0f;
-            const float ckr = ((iny >> r) & 1u) ? ck : 0.0f;
+            // the side columns four rows at a time
+            if (r == 0) {
+                get_part<0, (B < 4 ? B : 4)>(eR[B > 4 ? 0 : buf], tl, lft);
+                get_part<0, (B < 4 ? B : 4)>(eL[B > 4 ? 0 : buf], tr, rgt);
+            }
+            if (r == 4) {
+                get_part<0, (B > 4 ? B - 4 : 0)>(eR[1], tl, lft);
+                get_part<0, (B > 4 ? B - 4 : 0)>(eL[1], tr, rgt);
+            }
+            if (r == B - 1) get<B>(eT, buf, td, bot);
+            float wold = lft[r & 3];
+            const bool in_r = ((iny >> r) & 1u) != 0;
             float* __restrict__ urow = u + (long)(oy + r) * n + ox;
 #pragma unroll
             for (int c = 0; c < B; ++c) {
                 const float uc = s[r][c];
-                const float e = c == B - 1 ? (tx < kTX - 1 ? eL[r][ty][tx + 1] : 0.0f) : s[r][c + 1];
-                const float sn = r == B - 1 ? (ty < kTY - 1 ? eT[c][ty + 1][tx] : 0.0f) : s[r + 1][c];
-                const float lap = ((wold + e) - 2.0f * uc) + ((prev[c] + sn) - 2.0f * uc);
-                const float k = ((inx >> c) & 1u) ? ckr : 0.0f;
+                const float e = c == B - 1 ? rgt[r & 3] : s[r][c + 1];
+                const float sn = r == B - 1 ? bot[c] : s[r + 1][c];
+                const float lap =
+                    __builtin_fmaf(-2.0f, uc, wold + e) + __builtin_fmaf(-2.0f, uc, prev[c] + sn);
+                const float k = masked && !in_r ? 0.0f : kc[c];
                 const float v = __builtin_fmaf(k, lap, uc);
                 if (last && ((vy >> r) & (vx >> c) & 1u)) urow[c] = v;
                 s[r][c] = last ? (k != 0.0f ? lap : 0.0f) : v;
@@ -130,14 +226,34 @@ __device__ __attribute__((noinline)) void run_problem(const BatchArgs& a, int p)
                 wold = uc;
             }
         }
-        __syncthreads();
     };
-    for (int st = 0; st + 1 < a.nsteps; ++st) step(false);
-    // The final step is the same code with a run-time flag: a second copy of
-    // the unrolled step (compile-time flag) would raise register pressure.
+    // Two loops with the same barriers (a wave takes one or the other): a
+    // choice inside one loop would make the allocator spill half the block.
+    auto steps = [&](const bool masked) {
+        for (int st = 0; st + 1 < nsteps; ++st) {
+            publish(st & 1);
+            __syncthreads();
+            update(masked, false, st & 1);
+            // the next step writes the other half: what it overwrites was read
+            // before the barrier just passed
+            if (B > 4) __syncthreads();
+        }
+    };
+    if (plain) steps(false);
+    else steps(true);
+    // The masks and offsets of the final step are formed again behind an opaque
+    // copy, so that they take no registers during the loop.
+    ox = tx * B;
+    oy = ty * B;
+    asm volatile("" : "+v"(ox), "+v"(oy));
+    masks();
+    // The final step, with a run-time flag for the gradient.
     int lastg = want_grad ? 1 : 0;
     asm volatile("" : "+v"(lastg));
-    step(lastg != 0);
+    publish((nsteps - 1) & 1);
+    __syncthreads();
+    update(true, lastg != 0, (nsteps - 1) & 1);
+    __syncthreads();
     if (want_grad) {
         // the final state was stored by this thread; the barrier at the end
         // of the step made the stores visible to its own reloads
@@ -160,7 +276,6 @@ __device__ __attribute__((noinline)) void run_problem(const BatchArgs& a, int p)
             gsum += __shfl_down(gsum, w, 64);
             jsum += __shfl_down(jsum, w, 64);
         }
-        const int t = tx + kTX * ty;
         if ((t & 63) == 0) {
             red[0][t >> 6] = gsum;
             red[1][t >> 6] = jsum;
