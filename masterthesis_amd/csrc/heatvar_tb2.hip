@@ -28,42 +28,11 @@
 #include <cstdint>
 
 #include "heatvar_ops.hpp"
+#include "heatvar_pairs.hpp"
+#include "plane_buffer.hpp"
 #include "scafes_common.hpp"
 
 namespace scafes {
-
-// Buffer access to one z plane: a wave-uniform resource (base = the plane's
-// first memAll element, range = the in-plane extent incl. ghost planes below
-// it) plus a 32-bit per-thread byte offset; the hardware range check returns
-// 0 for, and drops, accesses beyond the range.
-using Rsrc = __amdgpu_buffer_rsrc_t;
-constexpr int kRsrcWord3 = 0x00020000;  // gfx9 family: 32-bit data format, raw (stride 0) buffer
-
-__device__ inline Rsrc plane_rsrc(const char* plane, uint32_t range)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(plane), (short)0, (int)range, kRsrcWord3);
-}
-
-template <typename T>
-__device__ inline T bload(Rsrc r, uint32_t off)
-{
-    if constexpr (sizeof(T) == 4) {
-        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
-    } else {
-        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
-    }
-}
-
-template <typename T>
-__device__ inline void bstore(T v, Rsrc r, uint32_t off)
-{
-    if constexpr (sizeof(T) == 4) {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, (int)off, 0, 0);
-    } else {
-        typedef int v2i __attribute__((ext_vector_type(2)));
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i, v), r, (int)off, 0, 0);
-    }
-}
 
 template <typename T, int MODE, int TX, int TY, int D>
 __global__ __launch_bounds__(TX* TY) void heatvar_tb2_kernel(Geo g, const T* __restrict__ u, const T* __restrict__ cin,
@@ -230,10 +199,10 @@ __global__ __launch_bounds__(TX* TY) void heatvar_tb2_kernel(Geo g, const T* __r
 // wave-uniform branches; lane predicates never branch: off-ring lanes load
 // and rewrite their own centre, off-ring rows write the y ring into a sink
 // row, and lanes off the output columns store out of range.  Measured on an
-// MI355X at 512^3 (64x12, us per three-step sweep): F32 + Kahan 835 -> 813,
-// F32 701 -> 631, F64 (64x16) 1882 -> 1767 against the branching kernel;
-// SQ counters for F32 + Kahan: vector ALU 0.64 of its issue rate, scalar
-// 0.51 (0.66 / 0.65 before).
+// MI355X at 512^3 (us per three-step sweep): F64 (64x16) 1882 -> 1767 against
+// the branching kernel, 1660 with quotients by h^2 that need no division.
+// FP64 fields, and FP32 ones on the 128-lane tile; other FP32 tiles take
+// heatvar_pairs_kernel.
 // MO: the states after one and two steps are written too (u1o, u2o; the
 // value part only in the compensated mode), at every node of the output
 // tile, as the one-step kernel would write them.
@@ -329,14 +298,9 @@ __global__ __launch_bounds__(TX* TY) void heatvar_tb3_kernel(Geo g, const T* __r
     const T bv = (T)cf.border_value;
     const bool keep = cf.border_mode != SCAFES_BORDER_VALUE;
     // The z queues below (faces, level values) shift every plane with period
-    // 3; the body covers lcm(D, 3) planes (6 at D = 2).  The shifts still cost
-    // about 30 register moves per plane (the wave-uniform branches merge
-    // values), but this form needs 78 VGPRs (FP32 + Kahan): two 12-wave
-    // workgroups per CU.  Register rings indexed by the unrolled plane (no
-    // moves, 28 % fewer vector instructions) needed 102 VGPRs and took a
-    // three-step sweep at 512^3 from 815 to 880-960 us (one workgroup per CU;
-    // capped at 80 VGPRs they spill: 2100 us), the FP64 leg from 222 to 148
-    // GLUPS.  s is the prefetch slot, buf the LDS parity.
+    // 3; the body covers lcm(D, 3) planes (6 at D = 2).  Register rings indexed
+    // by the unrolled plane save the moves but need more registers (FP64 leg
+    // 222 -> 148 GLUPS).  s is the prefetch slot, buf the LDS parity.
     constexpr int U = (D == 2) ? 6 : D;
     for (int kb = kfirst; kb <= klast; kb += U) {
 #pragma unroll
@@ -933,9 +897,13 @@ static int tb_dispatch(Ctx* c, const Geo& g, const void* u, const void* cin, con
                        const VarCoef& cf, int cfg, bool fit)
 {
     const TbCfg t = kTbCfgs[cfg];
+    // FP32 fields take three and four steps on 64-lane rows with the two-row kernel
 #define SCAFES_TB(S, X, Y, DD)                                                                    \
     case S * 10000000 + X * 100000 + Y * 100 + DD:                                                \
-        return tb_launch_t<S, T, MODE, X, Y, DD>(c, g, u, cin, kap, uo, co, cf, t.zc, fit);
+        if constexpr (MODE == 0 || S == 2 || X == 128)                                            \
+            return tb_launch_t<S, T, MODE, X, Y, DD>(c, g, u, cin, kap, uo, co, cf, t.zc, fit);   \
+        else                                                                                      \
+            break;
     switch (t.steps * 10000000 + t.tx * 100000 + t.ty * 100 + t.d) {
         SCAFES_TB(2, 64, 16, 2)
         SCAFES_TB(2, 64, 8, 2)
@@ -954,9 +922,10 @@ static int tb_dispatch(Ctx* c, const Geo& g, const void* u, const void* cin, con
         SCAFES_TB(3, 64, 14, 2)
         SCAFES_TB(4, 64, 16, 2)
         SCAFES_TB(4, 64, 16, 4)
-    default: return fail(SCAFES_ERR_ARG, "bad multi-step tile configuration");
+    default: break;
     }
 #undef SCAFES_TB
+    return fail(SCAFES_ERR_ARG, "bad multi-step tile configuration");
 }
 
 // Multi-step sweeps that also write the intermediate states: the default
@@ -1003,6 +972,79 @@ bool heatvar_tb2_supported(const Geo& geo, int mode)
     return geo.dim == 3 && (geo.base + geo.e01) * bytes < kOobLimit;
 }
 
+// Two rows per thread (FP32 fields): zc planes per workgroup, or with fit the
+// chunk of at most kPairZC planes that suits the grid.
+struct PairArgs {
+    const Geo& g;
+    const void *u, *cin, *kap;
+    void *uo, *co;
+    const VarCoef& cf;
+    int zc;
+    bool fit;
+    void* const* mid;
+};
+
+template <int MODE, int TY, int K, int D, bool MO>
+static int pairs_launch_t(Ctx* c, const PairArgs& a)
+{
+    constexpr int kPerCu = TY > 8 ? 1 : 2;
+    const Geo& g = a.g;
+    const int tiles_x = ceil_div(g.nx, 64 - 2 * K), tiles_y = ceil_div(g.ny, 2 * TY - 2 * (K - 1));
+    int zc = a.zc;
+    if (a.fit) zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * K - 1, kPairZC, kPerCu, c->cu_count);
+    const long nb = (long)tiles_x * tiles_y * ceil_div(g.nz, zc);
+    if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");
+    float* m[3] = {nullptr, nullptr, nullptr};
+    if constexpr (MO)
+        for (int l = 0; l < K - 1; ++l) m[l] = (float*)a.mid[l];
+    heatvar_pairs_kernel<MODE, TY, K, D, MO><<<dim3((unsigned)nb), dim3(64, TY), 0, c->stream>>>(
+        g, (const float*)a.u, (const float*)a.cin, (const float*)a.kap, (float*)a.uo, (float*)a.co, m[0], m[1], m[2],
+        a.cf, zc, tiles_x, tiles_y);
+    SCAFES_HIP(hipGetLastError());
+    return SCAFES_OK;
+}
+
+// Wavefronts of the default tile.  Measured (us for 24 steps, 8 / 12 / 16
+// wavefronts): four steps a sweep, FP32 + Kahan 128^3 142 / 147 / 135, 256^3
+// 687 / 662 / 558, 300x320x280 1066 / 1015 / 950; FP32 128^3 122 / 126 / 119,
+// 256^3 487 / 531 / 423, 300x320x280 755 / 671 / 746 (512^3, four steps: 588 /
+// 511 / 547).  Three steps, FP32 + Kahan 32x24x20 50 / 62 / 69, 97x80x75 81 / 85 /
+// 87, 256^3 778 / 773 / 720, 300x320x280 1357 / 1178 / 1183 (512^3, 12 steps:
+// 3223 / 2839 / 3148); FP32 97x80x75 69 / 73 / 77, 300x320x280 797 / 882 / 821.
+static int pair_waves(const Geo& g, int mode, int k)
+{
+    const long nodes = (long)g.nx * g.ny * g.nz;
+    if (k == 3) return mode == SCAFES_HEATVAR_F32_KAHAN && nodes > kFourStepNodes ? 12 : 8;
+    return mode == SCAFES_HEATVAR_F32 && nodes > 20000000L ? 12 : 16;
+}
+
+template <int MODE>
+static int pairs_launch(Ctx* c, const PairArgs& a, int k, int ty, int d)
+{
+#define SCAFES_PAIRS(K, TY, DD) \
+    if (!a.mid && k == K && ty == TY && d == DD) return pairs_launch_t<MODE, TY, K, DD, false>(c, a);
+#define SCAFES_PAIRS_MO(K, TY) \
+    if (a.mid && k == K && ty == TY && d == 2) return pairs_launch_t<MODE, TY, K, 2, true>(c, a);
+    SCAFES_PAIRS(3, 8, 2)
+    SCAFES_PAIRS(3, 10, 2)
+    SCAFES_PAIRS(3, 12, 2)
+    SCAFES_PAIRS(3, 14, 2)
+    SCAFES_PAIRS(3, 16, 2)
+    SCAFES_PAIRS(3, 12, 4)
+    SCAFES_PAIRS(3, 16, 4)
+    SCAFES_PAIRS(4, 12, 2)
+    SCAFES_PAIRS(4, 16, 2)
+    SCAFES_PAIRS(4, 16, 4)
+    SCAFES_PAIRS_MO(3, 8)
+    SCAFES_PAIRS_MO(3, 12)
+    SCAFES_PAIRS_MO(3, 16)
+    SCAFES_PAIRS_MO(4, 12)
+    SCAFES_PAIRS_MO(4, 16)
+#undef SCAFES_PAIRS
+#undef SCAFES_PAIRS_MO
+    return fail(a.mid ? SCAFES_ERR_UNSUPPORTED : SCAFES_ERR_ARG, "bad multi-step tile configuration");
+}
+
 // The configuration's number of steps u -> uo (and Kahan compensation cin -> co).
 int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, const void* u, void* uo,
                        const void* cin, void* co, const void* kap, double tau, int border_mode, double border_value,
@@ -1020,12 +1062,17 @@ int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, c
     cf.c2 = (float)(0.5 * tau / hh[2]);
     cf.border_value = border_value;
     cf.border_mode = border_mode;
+    const TbCfg t = kTbCfgs[cfg];
+    if (mode != SCAFES_HEATVAR_F64 && t.steps >= 3 && t.tx == 64) {
+        const PairArgs a = {geo, u, cin, kap, uo, co, cf, t.zc, fit, mid};
+        const int ty = fit ? pair_waves(geo, mode, t.steps) : t.ty, d = fit ? 2 : t.d;
+        return mode == SCAFES_HEATVAR_F32 ? pairs_launch<1>(c, a, t.steps, ty, d)
+                                          : pairs_launch<2>(c, a, t.steps, ty, d);
+    }
     if (mid) {
-        if (mode == SCAFES_HEATVAR_F64)
-            return tb_dispatch_mo<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit, mid);
-        if (mode == SCAFES_HEATVAR_F32)
-            return tb_dispatch_mo<float, 1>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit, mid);
-        return tb_dispatch_mo<float, 2>(c, geo, u, cin, kap, uo, co, cf, cfg, fit, mid);
+        if (mode != SCAFES_HEATVAR_F64)
+            return fail(SCAFES_ERR_UNSUPPORTED, "no state-writing variant of this multi-step tile");
+        return tb_dispatch_mo<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit, mid);
     }
     if (mode == SCAFES_HEATVAR_F64) return tb_dispatch<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit);
     if (mode == SCAFES_HEATVAR_F32) return tb_dispatch<float, 1>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit);

@@ -25,6 +25,7 @@
 
 #include "exact_quot.hpp"
 #include "heatvar_ops.hpp"
+#include "heatvar_pairs.hpp"
 #include "scafes_common.hpp"
 #include "stepk.hpp"
 
@@ -799,24 +800,24 @@ static constexpr int kDefaultCfg = 3;
 // (F64 64x8 zc128 d6, F32 128x2 zc64 d4, F32+Kahan 64x16 zc128 d4); used
 // for the odd last step behind two-steps-per-sweep launches.
 static constexpr int kOneStepCfgByMode[3] = {12, 4, 9};
-// Default per mode: the fastest multi-step tile at 512^3 on an MI355X
-// (indices into heatvar_tb2.hip's table), all three steps per sweep: F64
-// 64x16 zc64 d2 (10; 620 us/step against 658 for the best two-step tile),
-// F32 and F32+Kahan 64x12 zc64 d2 (13; 234 and 280 us/step).
+// Default per mode (indices into heatvar_tb2.hip's table), all three steps per
+// sweep: F64 64x16 zc64 d2 (10; 553 us/step at 512^3), F32 and F32 + Kahan 64x12 zc64
+// d2 (13).  Where neither a caller nor the autotuner names the tile, the z chunk and
+// the FP32 tile's rows are fitted to the grid.
 static constexpr int kDefaultCfgByMode[3] = {kNumCfgs + 10, kNumCfgs + 13, kNumCfgs + 13};
 // Two-step tile per mode for a remainder of two steps behind a three-step
 // configuration (F64 64x8 zc64 d4, F32 and F32+Kahan 64x8 zc64 d2): one
 // sweep instead of two one-step sweeps.
 static constexpr int kTwoStepCfgByMode[3] = {kNumCfgs + 6, kNumCfgs + 2, kNumCfgs + 2};
-// Four-step tile per mode, or -1: F32 + Kahan 64x16 zc128 d2.  Measured on
-// two MI355X boxes at 512^3 (us per sweep): 1084-1185 for four steps
-// against 800-813 for three with the default tile (271-290 against 267-271
-// us per step) and 776-780 for the two-step tile, so 20 steps as 2 x 4 +
-// 4 x 3 took 5.42-5.61 ms against 5.64-5.66 as 6 x 3 + 2.  FP32 (963
-// against 638 for three steps: 241 and 213 us per step) and FP64 (2660
-// against 1790: 665 and 597) lose more per step with four steps and keep
-// the two-step remainder.
+// Four-step tile per mode behind a three-step default, or -1: F32 + Kahan
+// 64x16 zc128 d2.  FP32 keeps the two-step remainder (grids of up to
+// kFourStepNodes nodes); FP64 loses with four steps (2148 us against 1553 for three at
+// 512^3).
 static constexpr int kFourStepCfgByMode[3] = {-1, -1, kNumCfgs + 24};
+// Default of FP32 fields on grids of more than kFourStepNodes nodes, where
+// four steps a sweep are the fastest per step (512^3: FP32 + Kahan 183 us a step
+// against 237 for three, FP32 128 against 145).
+static constexpr int kLargeCfgByMode[3] = {-1, kNumCfgs + 24, kNumCfgs + 24};
 
 template <class Op, typename T, int TX, int TY, int D>
 static int launch_t(Ctx* c, const Op& op, const Geo& g, int zc)
@@ -1335,7 +1336,10 @@ static int resolve_heatvar_cfg(const Ctx* c, const Geo& geo, int mode, int cfg)
 {
     if (cfg < 0) {
         cfg = tuned_cfg(c, geo, mode);
-        if (cfg < 0) cfg = kDefaultCfgByMode[mode];
+        if (cfg < 0) {
+            const bool large = (long)geo.nx * geo.ny * geo.nz > kFourStepNodes;
+            cfg = large && kLargeCfgByMode[mode] >= 0 ? kLargeCfgByMode[mode] : kDefaultCfgByMode[mode];
+        }
     }
     if (cfg >= kNumCfgs && !heatvar_tb2_supported(geo, mode)) cfg = kOneStepCfgByMode[mode];
     return cfg;
@@ -1671,18 +1675,18 @@ static int cfg_steps(int cfg)
 }
 
 // Behind a three-step tile, a remainder of two steps takes one two-step
-// sweep; where the mode has a four-step tile of about the same cost per
-// step, step counts that are not a multiple of three are made of three-
-// and four-step sweeps instead (4 = 4, 7 = 4 + 3, 8 = 4 + 4, 20 = 4 + 4 +
-// 4 x 3; only 5 keeps 3 + 2), so no short sweep pays for a whole pass over
-// HBM.  A tuned four-step tile takes a remainder of three with the mode's
-// three-step default tile, of two with its two-step tile.
+// sweep; where the mode has a four-step tile, step counts that are not a
+// multiple of three are made of three- and four-step sweeps instead (4 = 4, 7 = 4
+// + 3, 8 = 4 + 4, 20 = 4 + 4 + 4 x 3; only 5 keeps 3 + 2), so no short sweep pays for
+// a whole pass over HBM.  Behind a four-step tile (large grids in FP32, or the
+// tuned choice) a remainder of two becomes two three-step sweeps (6 = 3 + 3, 10 = 3 + 4
+// + 3), of three one, and a last single step is a one-step launch.
 int heat7var_next_sweep(const Ctx* c, const Geo& geo, int mode, long left)
 {
     const int st = cfg_steps(resolve_heatvar_cfg(c, geo, mode, -1));
     if (left <= 1 || st == 1) return 1;
     if (st == 2) return 2;
-    if (st == 4) return left >= 4 ? 4 : (int)left;
+    if (st == 4) return left >= 6 && left % 4 == 2 ? 3 : left >= 4 ? 4 : (int)left;
     if (kFourStepCfgByMode[mode] >= 0 && left >= 4 && (left % 3 == 1 || (left % 3 == 2 && left >= 8))) return 4;
     return left >= 3 ? 3 : 2;
 }
@@ -1704,9 +1708,17 @@ int heat7var_sweep_k(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, int
                               cfg - kNumCfgs, cfg != tuned_cfg(c, geo, mode));
 }
 
+// The tile of state-writing three-step sweeps: the tuned choice, else the
+// mode's three-step default.
+static int states_cfg(const Ctx* c, const Geo& geo, int mode)
+{
+    const int tuned = tuned_cfg(c, geo, mode);
+    return resolve_heatvar_cfg(c, geo, mode, tuned >= 0 ? tuned : kDefaultCfgByMode[mode]);
+}
+
 bool heat7var_states_sweep_ok(const Ctx* c, const Geo& geo, int mode)
 {
-    const int cfg = resolve_heatvar_cfg(c, geo, mode, -1);
+    const int cfg = states_cfg(c, geo, mode);
     return cfg >= kNumCfgs && cfg_steps(cfg) == 3 && heatvar_tb_states_supported(cfg - kNumCfgs);
 }
 
@@ -1721,7 +1733,7 @@ int heat7var_sweep_states(Ctx* c, const Geo& geo, const scafes_geom* g, int mode
                           int border_mode, double border_value)
 {
     int cfg = -1;
-    if (k == 3 && heat7var_states_sweep_ok(c, geo, mode)) cfg = resolve_heatvar_cfg(c, geo, mode, -1);
+    if (k == 3 && heat7var_states_sweep_ok(c, geo, mode)) cfg = states_cfg(c, geo, mode);
     if (k == 4 && heat7var_states4_ok(c, geo, mode)) cfg = kFourStepCfgByMode[mode];
     if (cfg < kNumCfgs) return fail(SCAFES_ERR_UNSUPPORTED, "no state-writing sweep of this many steps for this grid");
     return heatvar_tb2_launch(c, geo, g, mode, u, un, cin, cout, kap, tau, border_mode, border_value,
