@@ -146,8 +146,9 @@ int scafes_heat7_step_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, const d
  * or VALUE and the other rules that read no G), ping-ponging u -> u2 ->
  * u ...: the loop of iterateOverTime (Problem.hpp:2558-2715) over the
  * update phase for problems whose known fields do not enter the update,
- * one launch per step and no host work in between.  *result_in_second =
- * 1 when the final state is in u2.  Bit-identical to nsteps calls of
+ * with no host work in between; where launches or memory bound a step, three
+ * steps per launch.  *result_in_second = 1 when the final state is in u2
+ * (nsteps odd).  Bit-identical to nsteps calls of
  * scafes_heat7_step_f64. */
 int scafes_heat7_run_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, double* u, double* u2, int nsteps,
                          const scafes_heat7_params* p, int* result_in_second);
@@ -165,11 +166,12 @@ int scafes_heat7_run_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, double* 
  * layout of u.  cfg: tile configuration index (-1 = autotuned/default).
  * A multi-step configuration given as cfg runs nsteps / s sweeps of s
  * steps, a remainder of two as one two-step sweep, the rest one step per
- * sweep.  With cfg = -1 the steps left behind three-step sweeps go to one
- * two-step sweep, or, where the mode has a four-step tile of the same cost
- * per step (FP32 + Kahan), to four-step sweeps (7 = 4 + 3, 20 = 2 x 4 +
- * 4 x 3); a tuned four-step tile takes its remainder with the three-, two-
- * and one-step tiles.  Stability: SCAFES_ERR_ARG unless tau * sum_p 2*kappa_max/h_p^2 <= 1
+ * sweep.  With cfg = -1 FP32 fields take four steps per sweep on grids of more
+ * than 1.5 million nodes (20 = 5 x 4, 6 = 3 + 3, 15 = 3 x 4 + 3), else three;
+ * the steps left behind three-step sweeps go to one two-step sweep, or in FP32 +
+ * Kahan to four-step sweeps (7 = 4 + 3, 20 = 2 x 4 + 4 x 3), and the z chunk (in
+ * FP32 also the tile's rows) is fitted to the grid.  A tuned four-step tile takes
+ * its remainder with the three-, two- and one-step tiles.  Stability: SCAFES_ERR_ARG unless tau * sum_p 2*kappa_max/h_p^2 <= 1
  * (kappa_max = max |kappa| over all nodes, a device reduction kept per
  * pointer until the library writes the field or scafes_coef_changed names
  * it). */
@@ -184,8 +186,8 @@ int scafes_heat7var_num_cfgs(void);
 int scafes_heat7var_cfg_desc(int cfg, int* tx, int* ty, int* zchunk, int* depth,
                              int* steps_per_sweep);
 /* The configuration scafes_heat7var_run uses for cfg = -1 on this grid
- * (autotuned choice, else the per-mode default; the two-steps-per-sweep
- * tiles need a 3-D grid). */
+ * (autotuned choice, else the default of the mode and the grid's size; the
+ * multi-step tiles need a 3-D grid). */
 int scafes_heat7var_active_cfg(scafes_ctx* ctx, const scafes_geom* g, int hw, int mode, int* cfg);
 /* How scafes_heat7var_run with cfg = -1 splits nsteps into sweeps on this
  * grid: the steps of each sweep in launch order (the first min(max, count)
