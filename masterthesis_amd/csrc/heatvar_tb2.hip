@@ -1032,14 +1032,17 @@ static int pairs_launch(Ctx* c, const PairArgs& a, int k, int ty, int d)
     SCAFES_PAIRS(3, 16, 2)
     SCAFES_PAIRS(3, 12, 4)
     SCAFES_PAIRS(3, 16, 4)
-    SCAFES_PAIRS(4, 12, 2)
+    if constexpr (MODE == 1) {
+        SCAFES_PAIRS(4, 12, 2)
+    }
     SCAFES_PAIRS(4, 16, 2)
     SCAFES_PAIRS(4, 16, 4)
     SCAFES_PAIRS_MO(3, 8)
     SCAFES_PAIRS_MO(3, 12)
     SCAFES_PAIRS_MO(3, 16)
-    SCAFES_PAIRS_MO(4, 12)
-    SCAFES_PAIRS_MO(4, 16)
+    if constexpr (MODE == 2) {
+        SCAFES_PAIRS_MO(4, 16)
+    }
 #undef SCAFES_PAIRS
 #undef SCAFES_PAIRS_MO
     return fail(a.mid ? SCAFES_ERR_UNSUPPORTED : SCAFES_ERR_ARG, "bad multi-step tile configuration");
