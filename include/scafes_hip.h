@@ -417,8 +417,8 @@ int scafes_yee_run(scafes_ctx* ctx, int ncell, int dtype, double s, void* f, voi
  * (ceil(nsteps/energy_every) FP64 entries, written in stream order, not
  * waited for).  The per-workgroup energy partials live in a static 1 MiB
  * device array per GPU (2^17 doubles, two per workgroup of a launch: boxes
- * up to about 1150 cells per axis); a larger box is refused with
- * SCAFES_ERR_ARG before anything runs.  Nothing in the array needs clearing:
+ * up to 1203 cells per axis with f2, 1023 without); a larger box is refused
+ * with SCAFES_ERR_ARG before anything runs.  Nothing in the array needs clearing:
  * every workgroup writes its slot before the slots are summed.  All calls on
  * one GPU share that array: calls that overlap on one GPU (two contexts or
  * streams at once) race and must be ordered by the caller. */

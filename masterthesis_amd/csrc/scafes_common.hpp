@@ -241,6 +241,8 @@ int yee_eps_adjoint(Ctx* c, const YeeDims& d, int dtype, double s, const void* c
 // address of the scratch array of scafes_yee_run_noalloc (yee.hip); called
 // by scafes_ctx_create.
 int yee_noalloc_setup(int device);
+// Energy partial slots that a run with records needs (scafes_yee_run_noalloc has 2^17).
+long yee_energy_slots(int ncell, int elem_bytes, bool second_buffer, int cu_count);
 // One fused leapfrog step a -> b with the E coefficient field ce (yee.hip).
 template <typename T>
 int yee_fused_eps_launch(Ctx* c, const YeeDims& d, T s, const T* a, T* b, const T* ce);

@@ -373,11 +373,47 @@ constexpr int kFTX = 64, kFTY = 8, kFD = 2;
 template <typename T>
 constexpr int kFZC = sizeof(T) == 8 ? 16 : 32;
 
-static int yee_inplace_chunk(const Ctx* c, long nxy, int planes)
+// Slots of the no-allocation entry point's scratch array (below).
+constexpr long kScratchSlots = 1L << 17;
+
+// Split of the one-step launches: the in-place passes or the fused step.
+struct YeeSplit {
+    int tiles_x, tiles_y, zc;
+    long nb;
+};
+
+// records: the launches write energy partials.  Two per workgroup have to fit
+// the scratch array, so a box whose fitted chunks make too many workgroups
+// doubles them (up to 64 planes; FP32 from 952 cells and FP64 from 756 cells per
+// axis), in both entry points, whose records are the same bits.
+static YeeSplit yee_split(int N, int elem_bytes, bool fused, bool records, int cu_count)
 {
-    int zc = fit_chunk(nxy, planes, 1, kYZC, 8, c->cu_count);
-    while (zc < kYZMax && nxy * ceil_div(planes, zc) > kYBlocks) zc *= 2;
-    return std::min(zc, kYZMax);
+    YeeSplit s;
+    s.tiles_x = ceil_div(N + 1, fused ? kFTX - 1 : kYTX);
+    s.tiles_y = ceil_div(N + 1, fused ? kFTY - 1 : kYTY);
+    const long nxy = (long)s.tiles_x * s.tiles_y;
+    if (fused)
+        s.zc = fit_chunk(nxy, N + 1, 3, elem_bytes == 8 ? kFZC<double> : kFZC<float>, 2, cu_count);
+    else
+        s.zc = fit_chunk(nxy, N + 1, 1, kYZC, 8, cu_count);
+    const long most = !fused ? kYBlocks : records ? kScratchSlots / 2 : 0x7fffffffL;
+    while (s.zc < kYZMax && nxy * ceil_div(N + 1, s.zc) > most) s.zc = std::min(2 * s.zc, kYZMax);
+    s.nb = nxy * ceil_div(N + 1, s.zc);
+    return s;
+}
+
+// Energy partial slots of a run: two sets, each for the largest launch.
+long yee_energy_slots(int N, int elem_bytes, bool second_buffer, int cu_count)
+{
+    YeeDims d;
+    d.N = N;
+    d.M = N + 1;
+    d.M2 = d.M * d.M;
+    d.nf = d.M2 * d.M;
+    long nb = yee_split(N, elem_bytes, second_buffer, true, cu_count).nb;
+    if (second_buffer && yee_tb2_supported(d, elem_bytes))
+        nb = std::max(nb, yee_tb2_plan(d, elem_bytes, cu_count).nb);
+    return 2 * nb;
 }
 
 // energy: host array of the records (allocating path: the partials and the
@@ -398,31 +434,29 @@ static int yee_run_t(Ctx* c, int N, double s, T* f, T* f2, int nsteps, int energ
     if (fused && d.M2 * (long)sizeof(T) >= (1L << 32)) return fail(SCAFES_ERR_ARG, "yee: plane too large");
     const bool tb2 = fused && yee_tb2_supported(d, (int)sizeof(T));
     const int TX = fused ? kFTX : kYTX, TY = fused ? kFTY : kYTY;
-    const int OX = fused ? TX - 1 : TX, OY = fused ? TY - 1 : TY;
-    const int tiles_x = ceil_div(N + 1, OX), tiles_y = ceil_div(N + 1, OY);
-    const long nxy = (long)tiles_x * tiles_y;
-    const int ZC = fused ? fit_chunk(nxy, N + 1, 3, kFZC<T>, 2, c->cu_count) : yee_inplace_chunk(c, nxy, N + 1);
-    const int tiles_z = ceil_div(N + 1, ZC);
-    const long nb = (long)tiles_x * tiles_y * tiles_z;
+    const int nrec = (energy_every > 0) ? (nsteps + energy_every - 1) / energy_every : 0;
+    const YeeSplit split = yee_split(N, (int)sizeof(T), fused, nrec > 0, c->cu_count);
+    const int tiles_x = split.tiles_x, tiles_y = split.tiles_y, ZC = split.zc;
+    const long nb = split.nb;
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "yee: grid too large");
     const Tb2Plan plan = yee_tb2_plan(d, (int)sizeof(T), c->cu_count);
-    const long nbp = std::max(nb, tb2 ? plan.nb : 0L);  // partial slots per step
-    const int nrec = (energy_every > 0) ? (nsteps + energy_every - 1) / energy_every : 0;
+    const long slots = nrec > 0 ? yee_energy_slots(N, (int)sizeof(T), fused, c->cu_count) : 0;
+    const long nbp = slots / 2;  // partial slots per step
     double* epart = nullptr;
     double* edev = nullptr;
     const bool noalloc = part != nullptr;
     if (nrec > 0 && noalloc) {
-        if (2 * nbp > part_slots) {
+        if (slots > part_slots) {
             char buf[200];
             std::snprintf(buf, sizeof buf,
                           "yee noalloc: %d cells per axis need %ld energy partial slots, the scratch array holds %ld",
-                          N, 2 * nbp, part_slots);
+                          N, slots, part_slots);
             return fail(SCAFES_ERR_ARG, buf);
         }
         epart = part;
         edev = edev_out;
     } else if (nrec > 0) {
-        SCAFES_HIP(hipMallocAsync((void**)&epart, sizeof(double) * 2 * nbp, c->stream));
+        SCAFES_HIP(hipMallocAsync((void**)&epart, sizeof(double) * slots, c->stream));
         SCAFES_HIP(hipMallocAsync((void**)&edev, sizeof(double) * nrec, c->stream));
     }
     auto rec = [&](int st) { return nrec > 0 && (st % energy_every) == 0; };
@@ -492,12 +526,11 @@ template int yee_fused_eps_launch<double>(Ctx*, const YeeDims&, double, const do
 
 // ---------------------------------------------------------------- no allocation
 // Energy partials of scafes_yee_run_noalloc: two slots per workgroup of a
-// launch, 2^17 doubles (1 MiB) per GPU, enough for Yee boxes of up to about
-// 1150 cells per axis.  Each GPU the library runs on holds its own copy
+// launch, 2^17 doubles (1 MiB) per GPU, enough for Yee boxes of up to 1203
+// cells per axis with a second buffer and 1023 without.  Each GPU the library runs on holds its own copy
 // until the process ends.  Host code never passes the array's name to a
 // kernel (it is a host-side stand-in); it uses the device address looked up
 // once per device by yee_noalloc_setup.
-constexpr long kScratchSlots = 1L << 17;
 static __device__ __align__(256) double scratch[kScratchSlots];
 
 constexpr int kMaxDevices = 64;
