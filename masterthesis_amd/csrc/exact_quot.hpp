@@ -11,7 +11,7 @@
 // Floating-Point Arithmetic, section on division with an FMA): z correctly
 // rounded, q within one ulp, e exact, no underflow or overflow on the way,
 // d's significand not all ones.  The remainder is exact while x is zero or
-// |x| >= 2^-900; a smaller x, and any overflow, infinity or NaN (each leaves a
+// |x| > 2^-900; a smaller x, and any overflow, infinity or NaN (each leaves a
 // NaN in the sum), takes the divisions instead.  A divisor outside
 // [2^-200, 2^60] gets a NaN reciprocal, so it always does.  Sums equal the
 // divisions' bit for bit, but for the sign of a zero sum at most.
@@ -49,11 +49,13 @@ inline ByHH make_by_hh(const double hh[3])
     return r;
 }
 
-// Exponent and leading significand bits of |x|, minus one: zero becomes the
-// largest value, so one comparison finds the nonzero values below a bound.
+// Exponent and leading significand bits of |x| from the 64-bit pattern minus one:
+// zero alone wraps to the largest value, so one comparison finds the nonzero
+// values below a bound, subnormals without a bit in their upper word included
+// (one 64-bit shift-and-add).
 __device__ inline unsigned small_key(double x)
 {
-    return ((unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32) << 1) - 1u;
+    return (unsigned)(((__builtin_bit_cast(unsigned long long, x) << 1) - 1ull) >> 32);
 }
 
 __device__ inline double quot(const ByHH& c, int p, double x)
@@ -65,7 +67,7 @@ __device__ inline double quot(const ByHH& c, int p, double x)
 // v + x0/hh0 (+ x1/hh1 (+ x2/hh2)), added in this order.
 __device__ inline double add_by_hh(const ByHH& c, int dim, double v, double x0, double x1, double x2)
 {
-    constexpr unsigned kSmall = ((1023u - 900u) << 21) - 1u;  // small_key(2^-900)
+    constexpr unsigned kSmall = (1023u - 900u) << 21;  // small_key(2^-900) + 1
     unsigned k = small_key(x0);
     double r = v + quot(c, 0, x0);
     if (dim > 1) {
