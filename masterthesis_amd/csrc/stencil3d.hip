@@ -41,8 +41,10 @@ namespace scafes {
 // apply(g, i, j, k, a7, b7, c7, xv, res): the node's new value res.v, its new
 // compensation res.c (kComp) and the increment res.g of the FP64 gradient
 // (kGrad), which the kernel stores.
+// The FP64 tiles with six planes in flight need all of 128 registers (four waves
+// per SIMD); left alone, the allocator takes 130 for two of them.
 template <class Op, typename T, int TX, int TY, int D>
-__global__ __launch_bounds__(TX* TY) void stream_kernel(Op op, Geo g, int zc, int tiles_x,
+__global__ __launch_bounds__(TX* TY, (sizeof(T) == 8 && D == 6 ? 4 : 1)) void stream_kernel(Op op, Geo g, int zc, int tiles_x,
                                                          int tiles_y)
 {
     static_assert(D >= 2 && D % 2 == 0, "prefetch depth must be even");
@@ -384,8 +386,13 @@ struct HeatConstOp {
 
 // Variable-coefficient conservative heat.  MODE 0: FP64 in the CPU path's
 // order; 1: FP32; 2: FP32 with Kahan-compensated accumulation of the
-// per-step increment (u_true ~ u + c).
-template <typename T, int MODE>
+// per-step increment (u_true ~ u + c).  DIV: FP64 with the divisions by h^2
+// themselves (same bits): the tiles of stream_kernel wait on memory and take no
+// less time with the quotients (24 steps at 150x140x130 2965 us with both),
+// whose registers cost the six-plane ones half their workgroups (134 registers
+// against 128; 24 steps at 2048x2048 1485 us against 1058, 1e6 nodes in a row
+// 2431 against 1626).
+template <typename T, int MODE, bool DIV = false>
 struct HeatVarOp {
     static constexpr bool kTwo = true;
     static constexpr bool kThree = false;
@@ -407,10 +414,16 @@ struct HeatVarOp {
     {
         if (!is_border(g, i, j, k)) {
             if constexpr (MODE == 0) {
-                r.v = add_by_hh(hh, g.dim, s.c,
-                                tau * (0.5 * (q.e + q.c) * (s.e - s.c) - 0.5 * (q.c + q.w) * (s.c - s.w)),
-                                   tau * (0.5 * (q.n + q.c) * (s.n - s.c) - 0.5 * (q.c + q.s) * (s.c - s.s)),
-                                   tau * (0.5 * (q.u + q.c) * (s.u - s.c) - 0.5 * (q.c + q.d) * (s.c - s.d)));
+                const double x0 = tau * (0.5 * (q.e + q.c) * (s.e - s.c) - 0.5 * (q.c + q.w) * (s.c - s.w));
+                const double x1 = tau * (0.5 * (q.n + q.c) * (s.n - s.c) - 0.5 * (q.c + q.s) * (s.c - s.s));
+                const double x2 = tau * (0.5 * (q.u + q.c) * (s.u - s.c) - 0.5 * (q.c + q.d) * (s.c - s.d));
+                if constexpr (DIV) {
+                    r.v = s.c + x0 / hh.d[0];
+                    if (g.dim > 1) r.v += x1 / hh.d[1];
+                    if (g.dim > 2) r.v += x2 / hh.d[2];
+                } else {
+                    r.v = add_by_hh(hh, g.dim, s.c, x0, x1, x2);
+                }
             } else {
                 float d = c0 * __builtin_fmaf(q.e + q.c, s.e - s.c, -((q.c + q.w) * (s.c - s.w)));
                 if (g.dim > 1)
@@ -929,15 +942,23 @@ int heat7var_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, cons
     double hh[3];
     hh_of(g, hh);
     if (mode == SCAFES_HEATVAR_F64) {
-        HeatVarOp<double, 0> op{};
-        op.a = (const double*)u;
-        op.b = (const double*)kap;
-        op.out = (double*)un;
-        op.tau = tau;
-        op.hh = make_by_hh(hh);
-        op.border_value = border_value;
-        op.border_mode = border_mode;
-        return launch<HeatVarOp<double, 0>, double>(c, op, geo, cfg);
+        auto fill = [&](auto& op) {
+            op.a = (const double*)u;
+            op.b = (const double*)kap;
+            op.out = (double*)un;
+            op.tau = tau;
+            op.hh = make_by_hh(hh);
+            op.border_value = border_value;
+            op.border_mode = border_mode;
+        };
+        if (cfg < 0) {
+            HeatVarOp<double, 0> op{};
+            fill(op);
+            return launch_auto<HeatVarOp<double, 0>, double>(c, op, geo);
+        }
+        HeatVarOp<double, 0, true> op{};
+        fill(op);
+        return launch<HeatVarOp<double, 0, true>, double>(c, op, geo, cfg);
     }
     const float c0 = (float)(0.5 * tau / hh[0]), c1 = (float)(0.5 * tau / hh[1]),
                 c2 = (float)(0.5 * tau / hh[2]);
