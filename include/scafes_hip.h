@@ -179,9 +179,12 @@ enum { SCAFES_HEATVAR_F64 = 0, SCAFES_HEATVAR_F32 = 1, SCAFES_HEATVAR_F32_KAHAN 
 int scafes_heat7var_run(scafes_ctx* ctx, const scafes_geom* g, int hw, int mode, void* u,
                         void* u2, void* c, void* c2, const void* kappa, double tau, int nsteps,
                         int border_mode, double border_value, int cfg, int* result_in_second);
-/* Number of tile configurations and a description of one: workgroup tile,
- * z planes per workgroup, prefetch depth in planes, and time steps per HBM
- * sweep (1, or 2 / 3 / 4 for the temporally blocked kernels). */
+/* Number of tile configurations and a description of one: workgroup tile
+ * (threads), z planes per workgroup, prefetch depth in planes, and time steps
+ * per HBM sweep (1, or 2 / 3 / 4 for the temporally blocked kernels).  With
+ * FP32 fields a thread of the 64-wide three- and four-step tiles takes two
+ * rows, and their z planes per workgroup are at most the ones described:
+ * small grids shorten them to fill the CUs. */
 int scafes_heat7var_num_cfgs(void);
 int scafes_heat7var_cfg_desc(int cfg, int* tx, int* ty, int* zchunk, int* depth,
                              int* steps_per_sweep);

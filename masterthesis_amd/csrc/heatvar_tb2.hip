@@ -972,15 +972,19 @@ bool heatvar_tb2_supported(const Geo& geo, int mode)
     return geo.dim == 3 && (geo.base + geo.e01) * bytes < kOobLimit;
 }
 
-// Two rows per thread (FP32 fields): zc planes per workgroup, or with fit the
-// chunk of at most kPairZC planes that suits the grid.
+// Two rows per thread (FP32 fields): the chunk of at most zmax planes that suits
+// the grid, also for a tile named by its index: it covers twice the rows of a
+// tile of one-node threads, so its full chunks make half the workgroups.  24 steps
+// at 150x140x130 with tiles 64x16 and 64x12 of three steps and 64x16 of four, us,
+// one-node threads -> two rows, full chunks -> fitted: FP32 445, 366, 708 -> 573,
+// 471, 937 -> 135, 134, 137; FP32 + Kahan 496, 409, 784 -> 645, 554, 1077 -> 158, 157,
+// 158.
 struct PairArgs {
     const Geo& g;
     const void *u, *cin, *kap;
     void *uo, *co;
     const VarCoef& cf;
-    int zc;
-    bool fit;
+    int zmax;
     void* const* mid;
 };
 
@@ -990,8 +994,7 @@ static int pairs_launch_t(Ctx* c, const PairArgs& a)
     constexpr int kPerCu = TY > 8 ? 1 : 2;
     const Geo& g = a.g;
     const int tiles_x = ceil_div(g.nx, 64 - 2 * K), tiles_y = ceil_div(g.ny, 2 * TY - 2 * (K - 1));
-    int zc = a.zc;
-    if (a.fit) zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * K - 1, kPairZC, kPerCu, c->cu_count);
+    const int zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * K - 1, a.zmax, kPerCu, c->cu_count);
     const long nb = (long)tiles_x * tiles_y * ceil_div(g.nz, zc);
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");
     float* m[3] = {nullptr, nullptr, nullptr};
@@ -1034,9 +1037,9 @@ static int pairs_launch(Ctx* c, const PairArgs& a, int k, int ty, int d)
     SCAFES_PAIRS(3, 16, 4)
     if constexpr (MODE == 1) {
         SCAFES_PAIRS(4, 12, 2)
+        SCAFES_PAIRS(4, 16, 4)
     }
     SCAFES_PAIRS(4, 16, 2)
-    SCAFES_PAIRS(4, 16, 4)
     SCAFES_PAIRS_MO(3, 8)
     SCAFES_PAIRS_MO(3, 12)
     SCAFES_PAIRS_MO(3, 16)
@@ -1067,8 +1070,11 @@ int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, c
     cf.border_mode = border_mode;
     const TbCfg t = kTbCfgs[cfg];
     if (mode != SCAFES_HEATVAR_F64 && t.steps >= 3 && t.tx == 64) {
-        const PairArgs a = {geo, u, cin, kap, uo, co, cf, t.zc, fit, mid};
-        const int ty = fit ? pair_waves(geo, mode, t.steps) : t.ty, d = fit ? 2 : t.d;
+        const PairArgs a = {geo, u, cin, kap, uo, co, cf, fit ? kPairZC : t.zc, mid};
+        const int ty = fit ? pair_waves(geo, mode, t.steps) : t.ty;
+        // four compensated steps with four planes in flight spill (12 steps at
+        // 512^3 6084 us, with two planes 2561)
+        const int d = fit || (mode == SCAFES_HEATVAR_F32_KAHAN && t.steps == 4) ? 2 : t.d;
         return mode == SCAFES_HEATVAR_F32 ? pairs_launch<1>(c, a, t.steps, ty, d)
                                           : pairs_launch<2>(c, a, t.steps, ty, d);
     }

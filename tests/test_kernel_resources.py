@@ -63,3 +63,9 @@ def test_fp64_one_step_tiles_keep_four_waves(kernels):
     assert len(tiles) == 3
     for n, k in tiles.items():
         assert k[".vgpr_count"] <= 128 and k[".private_segment_fixed_size"] == 0, (n, k[".vgpr_count"])
+
+
+def test_two_row_sweeps_do_not_spill(kernels):
+    pairs = {n: k for n, k in kernels.items() if "heatvar_pairs_kernel" in n}
+    assert len(pairs) > 20
+    assert [n for n, k in pairs.items() if k[".private_segment_fixed_size"]] == []
