@@ -8,7 +8,8 @@
 // 1.6 nodes per stored one.  Here
 //   - a wavefront is a 64-lane row pair: x neighbours come from the lanes beside
 //     (DPP, one vector instruction, instead of an LDS read), so the tile gives up K
-//     columns on each side and needs no x ring;
+//     columns on each inner side and needs no x ring; rows of up to 64 nodes are one
+//     tile (60 nodes as two: 24 steps at 60x512x512 FP32 674 us, as one 382);
 //   - each product of a face and the difference across it is formed once and used by
 //     both nodes (lane below, row below, plane before), which also drops the west,
 //     south and lower faces and the second old plane of each level;
@@ -117,10 +118,12 @@ __global__ __launch_bounds__(64 * TY) void heatvar_pairs_kernel(Geo g, const flo
     const int rr = lb - tz * per_plane;
     const int tyi = rr / tiles_x;
     const int txi = rr - tyi * tiles_x;
-    const int i = txi * OX - K + tx, j0 = tyi * OY - (K - 1) + 2 * ty;
-    const int ic = min(max(i, 0), g.nx - 1);
+    // the first tile needs no columns before it and the last none after it: the
+    // border nodes there take no neighbour values
+    const int i = txi * OX + tx, j0 = tyi * OY - (K - 1) + 2 * ty;
+    const int ic = min(i, g.nx - 1);
     const bool inner_x = i >= g.nl0 && i <= g.nx - 1 - g.nl0;
-    const bool col_out = tx >= K && tx <= 63 - K && i < g.nx;
+    const bool col_out = (tx >= K || txi == 0) && (tx <= 63 - K || txi == tiles_x - 1) && i < g.nx;
     const int k0 = tz * zc, k1 = min(k0 + zc, g.nz);
     const int kfirst = k0 - (K - 1);  // first plane with a level-1 value
     const int klast = k1 + K - 2;     // last iteration

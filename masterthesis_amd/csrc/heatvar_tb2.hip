@@ -972,6 +972,9 @@ bool heatvar_tb2_supported(const Geo& geo, int mode)
     return geo.dim == 3 && (geo.base + geo.e01) * bytes < kOobLimit;
 }
 
+// Column tiles of a row of nx nodes in sweeps of k steps (heatvar_pairs_kernel).
+int pair_tiles_x(int nx, int k) { return nx <= 64 ? 1 : 1 + ceil_div(nx - 64, 64 - 2 * k); }
+
 // Two rows per thread (FP32 fields): the chunk of at most zmax planes that suits
 // the grid, also for a tile named by its index: it covers twice the rows of a
 // tile of one-node threads, so its full chunks make half the workgroups.  24 steps
@@ -993,7 +996,7 @@ static int pairs_launch_t(Ctx* c, const PairArgs& a)
 {
     constexpr int kPerCu = TY > 8 ? 1 : 2;
     const Geo& g = a.g;
-    const int tiles_x = ceil_div(g.nx, 64 - 2 * K), tiles_y = ceil_div(g.ny, 2 * TY - 2 * (K - 1));
+    const int tiles_x = pair_tiles_x(g.nx, K), tiles_y = ceil_div(g.ny, 2 * TY - 2 * (K - 1));
     const int zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * K - 1, a.zmax, kPerCu, c->cu_count);
     const long nb = (long)tiles_x * tiles_y * ceil_div(g.nz, zc);
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");

@@ -211,6 +211,7 @@ int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, c
                        const void* cin, void* co, const void* kap, double tau, int border_mode, double border_value,
                        int cfg, bool fit, void* const* mid = nullptr);
 bool heatvar_tb_states_supported(int cfg);
+int pair_tiles_x(int nx, int k);
 
 // Yee box of N cells per axis; fields hold N+1 nodes per axis, x fastest.
 struct YeeDims {
