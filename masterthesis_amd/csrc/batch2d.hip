@@ -119,6 +119,19 @@ __device__ __forceinline__ void get(const float4 (*a)[kTY * kTX], int buf, int a
     get_part<4, (B > 4 ? B - 4 : 0)>(a[1], at, v);
 }
 
+// __syncthreads as the hardware does it: s_barrier counts the waves of the
+// workgroup that have arrived, wherever in the program each of them stands, so
+// waves may wait at different places as long as all pass the same number.
+__device__ __forceinline__ void wave_barrier()
+{
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "barriers at several places of the program: known to hold on gfx950"
+#endif
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 __device__ __forceinline__ float* uniform_ptr(float* q)
 {
     const unsigned long v = reinterpret_cast<unsigned long>(q);
@@ -167,7 +180,7 @@ __device__ __attribute__((noinline)) void run_problem(const BatchArgs& a, int p)
     for (int c = 0; c < B; ++c) kc[c] = ((inx >> c) & 1u) && iny ? ck : 0.0f;
     // whether every row of every thread of this wave (two thread rows) is
     // inner, or none of the thread's: then no row needs a mask
-    const bool plain = __all(iny == (1u << B) - 1u || iny == 0u);
+    const bool plain = __builtin_amdgcn_readfirstlane(__all(iny == (1u << B) - 1u || iny == 0u)) != 0;
     const int t = tx + kTX * ty;
     // neighbours' slots, clamped at the workgroup's edge: the nodes next to it
     // are border or padding nodes (coefficient 0), so any finite value serves
@@ -227,16 +240,17 @@ __device__ __attribute__((noinline)) void run_problem(const BatchArgs& a, int p)
             }
         }
     };
-    // Two loops with the same barriers (a wave takes one or the other): a
-    // choice inside one loop would make the allocator spill half the block.
+    // Two loops with the same barriers; a wave takes one or the other (`plain` is
+    // one value per wave).  A choice inside one loop makes the allocator spill
+    // twice as much (B = 8: 548 bytes a thread against 328).
     auto steps = [&](const bool masked) {
         for (int st = 0; st + 1 < nsteps; ++st) {
             publish(st & 1);
-            __syncthreads();
+            wave_barrier();
             update(masked, false, st & 1);
             // the next step writes the other half: what it overwrites was read
             // before the barrier just passed
-            if (B > 4) __syncthreads();
+            if (B > 4) wave_barrier();
         }
     };
     if (plain) steps(false);
