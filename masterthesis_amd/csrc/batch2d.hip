@@ -65,11 +65,13 @@ struct BatchArgs {
 // columns.  A thread's edge of B values is two vectors of at most 4, each
 // packed over the threads, so an edge takes one or two LDS instructions and no
 // bank conflicts.  Blocks of up to 4 x 4 need one vector per edge and alternate
-// between the two halves, so their steps need one barrier instead of two.
-__shared__ float4 eT[2][kTY * kTX];
-__shared__ float4 eB[2][kTY * kTX];
-__shared__ float4 eL[2][kTY * kTX];
-__shared__ float4 eR[2][kTY * kTX];
+// between the two halves, so their steps need one barrier instead of two.  Two
+// slots hold zeros, the neighbours of the threads at the workgroup's edge: before
+// the first and after the last thread of a row or column, each on a bank that the
+// reads beside it leave free.
+constexpr int kAfter = kTX * kTY, kBefore = kAfter + 63, kSlots = kBefore + 1;
+enum { kTop, kBottom, kLeft, kRight };
+__shared__ float4 edges[2][4][kSlots];  // the four edges of a half within one offset's reach
 __shared__ double red[2][kTX * kTY / 64];
 
 template <int N>
@@ -107,16 +109,16 @@ __device__ __forceinline__ void get_part(const float4* a, int at, float* v)
     }
 }
 template <int B>
-__device__ __forceinline__ void put(float4 (*a)[kTY * kTX], int buf, int at, const float* v)
+__device__ __forceinline__ void put(int edge, int buf, int at, const float* v)
 {
-    put_part<0, (B < 4 ? B : 4)>(a[B > 4 ? 0 : buf], at, v);
-    put_part<4, (B > 4 ? B - 4 : 0)>(a[1], at, v);
+    put_part<0, (B < 4 ? B : 4)>(edges[B > 4 ? 0 : buf][edge], at, v);
+    put_part<4, (B > 4 ? B - 4 : 0)>(edges[1][edge], at, v);
 }
 template <int B>
-__device__ __forceinline__ void get(const float4 (*a)[kTY * kTX], int buf, int at, float* v)
+__device__ __forceinline__ void get(int edge, int buf, int at, float* v)
 {
-    get_part<0, (B < 4 ? B : 4)>(a[B > 4 ? 0 : buf], at, v);
-    get_part<4, (B > 4 ? B - 4 : 0)>(a[1], at, v);
+    get_part<0, (B < 4 ? B : 4)>(edges[B > 4 ? 0 : buf][edge], at, v);
+    get_part<4, (B > 4 ? B - 4 : 0)>(edges[1][edge], at, v);
 }
 
 // __syncthreads as the hardware does it: s_barrier counts the waves of the
@@ -182,10 +184,21 @@ __device__ __attribute__((noinline)) void run_problem(const BatchArgs& a, int p)
     // inner, or none of the thread's: then no row needs a mask
     const bool plain = __builtin_amdgcn_readfirstlane(__all(iny == (1u << B) - 1u || iny == 0u)) != 0;
     const int t = tx + kTX * ty;
-    // neighbours' slots, clamped at the workgroup's edge: the nodes next to it
-    // are border or padding nodes (coefficient 0), so any finite value serves
-    const int tl = t - (tx > 0 ? 1 : 0), tr = t + (tx < kTX - 1 ? 1 : 0);
-    const int tu = t - (ty > 0 ? kTX : 0), td = t + (ty < kTY - 1 ? kTX : 0);
+    // neighbours' slots; nothing lies beyond the workgroup's edge (the nodes next
+    // to it are border or padding nodes: coefficient 0, and a value that is not
+    // finite must not reach them from the other end of their block)
+    const int tl = tx > 0 ? t - 1 : kBefore, tr = tx < kTX - 1 ? t + 1 : kAfter;
+    const int tu = ty > 0 ? t - kTX : kBefore, td = ty < kTY - 1 ? t + kTX : kAfter;
+    if (t == 0) {  // the slots' places depend on B; the first step's barrier follows
+        const float zero[B] = {};
+#pragma unroll
+        for (int buf = 0; buf < 2; ++buf) {
+            put<B>(kTop, buf, kAfter, zero);
+            put<B>(kLeft, buf, kAfter, zero);
+            put<B>(kBottom, buf, kBefore, zero);
+            put<B>(kRight, buf, kBefore, zero);
+        }
+    }
     const bool want_grad = a.target != nullptr;
     // One explicit step on the register block, rows top-down in place:
     // prev[] keeps the old row above, `wold` the old left neighbour.  Second
@@ -195,32 +208,32 @@ __device__ __attribute__((noinline)) void run_problem(const BatchArgs& a, int p)
     // and keeps the inner nodes' L u^{N-1} terms (zero elsewhere) in the block.
     auto publish = [&](const int buf) {
         float e[B];
-        put<B>(eT, buf, t, s[0]);
-        put<B>(eB, buf, t, s[B - 1]);
+        put<B>(kTop, buf, t, s[0]);
+        put<B>(kBottom, buf, t, s[B - 1]);
 #pragma unroll
         for (int r = 0; r < B; ++r) e[r] = s[r][0];
-        put<B>(eL, buf, t, e);
+        put<B>(kLeft, buf, t, e);
 #pragma unroll
         for (int r = 0; r < B; ++r) e[r] = s[r][B - 1];
-        put<B>(eR, buf, t, e);
+        put<B>(kRight, buf, t, e);
     };
     auto update = [&](const bool masked, const bool last, const int buf) {
         float prev[B], lft[4], rgt[4], bot[B];
         // opaque per step: hoisted, the masked coefficients would be spilled
         if (masked) asm volatile("" : "+v"(iny));
-        get<B>(eB, buf, tu, prev);
+        get<B>(kBottom, buf, tu, prev);
 #pragma unroll
         for (int r = 0; r < B; ++r) {
             // the side columns four rows at a time
             if (r == 0) {
-                get_part<0, (B < 4 ? B : 4)>(eR[B > 4 ? 0 : buf], tl, lft);
-                get_part<0, (B < 4 ? B : 4)>(eL[B > 4 ? 0 : buf], tr, rgt);
+                get_part<0, (B < 4 ? B : 4)>(edges[B > 4 ? 0 : buf][kRight], tl, lft);
+                get_part<0, (B < 4 ? B : 4)>(edges[B > 4 ? 0 : buf][kLeft], tr, rgt);
             }
             if (r == 4) {
-                get_part<0, (B > 4 ? B - 4 : 0)>(eR[1], tl, lft);
-                get_part<0, (B > 4 ? B - 4 : 0)>(eL[1], tr, rgt);
+                get_part<0, (B > 4 ? B - 4 : 0)>(edges[1][kRight], tl, lft);
+                get_part<0, (B > 4 ? B - 4 : 0)>(edges[1][kLeft], tr, rgt);
             }
-            if (r == B - 1) get<B>(eT, buf, td, bot);
+            if (r == B - 1) get<B>(kTop, buf, td, bot);
             float wold = lft[r & 3];
             const bool in_r = ((iny >> r) & 1u) != 0;
             float* __restrict__ urow = u + (long)(oy + r) * n + ox;
