@@ -387,7 +387,9 @@ int scafes_ctx_create(int device, scafes_ctx** out)
     c->red_capacity = 4096;
     SCAFES_HIP(hipMalloc(&c->red_partial, sizeof(double) * c->red_capacity));
     SCAFES_HIP(hipMalloc(&c->red_done, sizeof(double)));
-    SCAFES_HIP(hipMemset(c->red_done, 0, sizeof(double)));
+    // on the stream that the reductions use: a non-blocking stream does not wait
+    // for the null stream
+    SCAFES_HIP(hipMemsetAsync(c->red_done, 0, sizeof(double), c->stream));
     SCAFES_HIP(hipHostMalloc(&c->host_result, sizeof(double) * 8, hipHostMallocDefault));
     SCAFES_HIP(hipHostGetDevicePointer((void**)&c->host_result_dev, c->host_result, 0));
     SCAFES_HIP(hipEventCreateWithFlags(&c->ready, hipEventDisableTiming));
