@@ -147,9 +147,9 @@ int scafes_heat7_step_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, const d
  * u ...: the loop of iterateOverTime (Problem.hpp:2558-2715) over the
  * update phase for problems whose known fields do not enter the update,
  * with no host work in between; where launches or memory bound a step, three
- * steps per launch.  *result_in_second = 1 when the final state is in u2
- * (nsteps odd).  Bit-identical to nsteps calls of
- * scafes_heat7_step_f64. */
+ * steps per launch, the last step alone.  *result_in_second = 1 when the final
+ * state is in u2 (nsteps odd); the other buffer holds the state one step
+ * before.  Bit-identical to nsteps calls of scafes_heat7_step_f64. */
 int scafes_heat7_run_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, double* u, double* u2, int nsteps,
                          const scafes_heat7_params* p, int* result_in_second);
 

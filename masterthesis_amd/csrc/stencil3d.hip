@@ -1301,8 +1301,9 @@ int scafes_heat7_run_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, double* 
     double *a = u, *b = u2;
     int sweeps = 0;
     for (int s = 0; s < nsteps; ++sweeps) {
-        // an odd count per sweep, so the result lies where single steps leave it
-        const int k = multi && nsteps - s >= 3 ? 3 : 1;
+        // an odd count per sweep, so the result lies where single steps leave it,
+        // and a single step last, so the other buffer holds the state before it
+        const int k = multi && nsteps - s >= 4 ? 3 : 1;
         op.a = a;
         op.out = b;
         rc = launch_steps<HeatConstOp, double>(c, op, geo, k, nullptr);
