@@ -201,12 +201,14 @@ int scafes_heat7var_active_cfg(scafes_ctx* ctx, const scafes_geom* g, int hw, in
 int scafes_heat7var_plan(scafes_ctx* ctx, const scafes_geom* g, int hw, int mode, int nsteps, int* sweeps,
                          int max, int* count);
 /* Project autotuner (no counterpart in the reference, whose device stub
- * fixes BLOCK_SIZE 32, src/ScaFES_ProblemCuda.hpp:22): times every
- * configuration on the given buffers over 24*ceil(nsteps/24) steps (a
- * multiple of every configuration's steps per sweep, so no remainder sweep
- * enters the timing) and keeps the fastest for this grid (extents, hw) and
- * mode: later calls with cfg = -1 on the same grid use it (at most eight
- * grids per context).  The buffers are overwritten: u/u2 (and c/c2) are
+ * fixes BLOCK_SIZE 32, src/ScaFES_ProblemCuda.hpp:22): times the default of
+ * cfg = -1 and every configuration on the given buffers over
+ * 24*ceil(nsteps/24) steps (a multiple of every configuration's steps per
+ * sweep, so no remainder sweep enters the timing).  Where a configuration is
+ * at least 2 % faster than the default, the fastest is kept for this grid
+ * (extents, hw) and mode, and later calls with cfg = -1 on the same grid use it
+ * (at most eight grids per context); else nothing is kept and *best_cfg is the
+ * default's configuration.  The buffers are overwritten: u/u2 (and c/c2) are
  * advanced with border KEEP, an even number of sweeps per configuration. */
 int scafes_autotune_heat7var(scafes_ctx* ctx, const scafes_geom* g, int hw, int mode, void* u,
                              void* u2, void* c, void* c2, const void* kappa, double tau,
