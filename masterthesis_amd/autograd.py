@@ -46,7 +46,11 @@ class _DeviceFields:
     def _staging(self, nbytes):
         nbytes = min(nbytes, _STAGE)
         if self.stage is None or self.stage.numel() < nbytes:
-            self.stage = torch.empty(nbytes, dtype=torch.uint8, pin_memory=torch.cuda.is_available())
+            # kept for later calls: host memory whatever the default device, and no
+            # inference tensor, which a call outside inference mode could not write
+            with torch.inference_mode(False):
+                self.stage = torch.empty(nbytes, dtype=torch.uint8, device="cpu",
+                                         pin_memory=torch.cuda.is_available())
         return self.stage
 
     def array(self, name, count, dtype):
@@ -78,7 +82,7 @@ class _DeviceFields:
 
     def get(self, d, shape):
         """A host copy of device array d."""
-        out = torch.empty(d.count, dtype=torch.float64 if d.dtype == np.float64 else torch.float32)
+        out = torch.empty(d.count, dtype=torch.float64 if d.dtype == np.float64 else torch.float32, device="cpu")
         for part, ptr, lo, n in self._chunks(d):
             capi.check(self.ctx.L.scafes_memcpy_d2h(self.ctx.h, capi.vp(part.data_ptr()), ptr, n * d.dtype.itemsize))
             out[lo:lo + n].copy_(part)
