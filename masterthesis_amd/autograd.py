@@ -46,11 +46,7 @@ class _DeviceFields:
     def _staging(self, nbytes):
         nbytes = min(nbytes, _STAGE)
         if self.stage is None or self.stage.numel() < nbytes:
-            # kept for later calls: host memory whatever the default device, and no
-            # inference tensor, which a call outside inference mode could not write
-            with torch.inference_mode(False):
-                self.stage = torch.empty(nbytes, dtype=torch.uint8, device="cpu",
-                                         pin_memory=torch.cuda.is_available())
+            self.stage = torch.empty(nbytes, dtype=torch.uint8, device="cpu", pin_memory=torch.cuda.is_available())
         return self.stage
 
     def array(self, name, count, dtype):
