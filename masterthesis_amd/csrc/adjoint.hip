@@ -71,8 +71,10 @@ __global__ __launch_bounds__(256) void lam_init_kernel(Geo g, const T* __restric
         const long m = at(g, i, j, k);
         double v = (double)t[m] - (double)target[m];
         if (tlo) v += (double)tlo[m];
-        // is_border as one mask: written with short-circuit branches, ROCm 7.2's
-        // clang zeroes l on every lane of the FP64 instance of this loop
+        // is_border as one mask: with short-circuit branches, ROCm 7.2's clang
+        // writes the zero of this select over v on every lane of the FP64
+        // instance and leaves the region that should keep v empty (no other
+        // kernel here has such a region)
         const bool inner = (i >= g.nl0) & (i <= g.nx - 1 - g.nl0) & (j >= g.nl1) & (j <= g.ny - 1 - g.nl1) &
                            (k >= g.nl2) & (k <= g.nz - 1 - g.nl2);
         const T l = (every_node != 0) | inner ? (T)v : T(0);

@@ -1,7 +1,9 @@
 """Registers and scratch of the built kernels, read from the metadata that the
 compiler wrote into the library: limits on which workgroups per CU depend."""
+import os
 import re
 import struct
+import subprocess
 
 import msgpack
 import pytest
@@ -69,3 +71,25 @@ def test_two_row_sweeps_do_not_spill(kernels):
     pairs = {n: k for n, k in kernels.items() if "heatvar_pairs_kernel" in n}
     assert len(pairs) > 20
     assert [n for n, k in pairs.items() if k[".private_segment_fixed_size"]] == []
+
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
+def test_no_empty_lane_regions(tmp_path):
+    """A region that selects lanes and then does nothing: what ROCm 7.2's clang left
+    of `c ? v : 0` in the FP64 start of the adjoint when c was a chain of
+    short-circuit branches; the zero had been written over v on every lane."""
+    with open(LIB_PATH, "rb") as f:
+        objects = list(_device_objects(f.read()))
+    assert objects
+    for n, elf in enumerate(objects):
+        path = tmp_path / f"{n}.elf"
+        path.write_bytes(elf)
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", str(path)], check=True,
+                              capture_output=True, text=True).stdout
+        code = "\n".join(x.split("//")[0].strip() for x in text.splitlines())
+        assert "s_and_saveexec_b64" in code or "s_endpgm" in code
+        bad = re.findall(r"s_and_saveexec_b64 (s\[\d+:\d+\]), \S+\ns_or_b64 exec, exec, \1\n", code)
+        assert not bad, (n, len(bad))
