@@ -1,0 +1,218 @@
+"""Rows around the vector length of the one-step updates, whose loads reach one
+ghost node to either side of a row: with NaN in every field's ghosts the nodes
+get the same bits as with zeros there, in every update and border rule.  FP64
+results against the oracle or the LDS tiles, FP32 against FP64, within their
+rounding."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from masterthesis_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+N3 = [(nx, 4 + nx % 3, 3 + nx % 2) for nx in range(1, 10)] + [(130, 3, 4)]
+NS = N3 + [(3, 5), (5, 4), (8, 3), (6,), (9,)]
+F32, F64, KAHAN = capi.F32, capi.F64, capi.F32_KAHAN
+HEATVAR = {F64: capi.HEATVAR_F64, F32: capi.HEATVAR_F32, KAHAN: capi.HEATVAR_F32_KAHAN}
+
+
+@pytest.fixture(scope="module")
+def ctx(hip):
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+def _node(n):
+    return tuple(slice(1, -1) for _ in n)
+
+
+def _both(ctx, n, code, fields, call, outs):
+    """Runs call(ptrs) on the fields (node arrays) with zero and with NaN ghosts;
+    returns the nodes of outs, which must agree."""
+    dt = np.float64 if code == F64 else np.float32
+    shape, got = tuple(m + 2 for m in reversed(n)), []
+    for ghost in (0.0, np.nan):
+        d = {}
+        for k, v in fields.items():
+            kind = np.float64 if k == "grad" else dt
+            a = np.full(shape, ghost, kind)
+            a[_node(n)] = v.astype(kind)
+            d[k] = ctx.upload(a)
+        call({k: x.ptr for k, x in d.items()})
+        got.append([d[k].read(shape)[_node(n)] for k in outs])
+        for x in d.values():
+            x.free()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+        assert np.isfinite(a).all()
+    return got[0]
+
+
+def _rand(n, seed, count):
+    rng = np.random.default_rng(seed + sum(n))
+    return [rng.random(tuple(reversed(n))) for _ in range(count)]
+
+
+def _h(n):
+    return [0.5 + 0.1 * p for p in range(len(n))]
+
+
+def _ograd(n, nodes):
+    """The oracle's grid of these extents with spacing _h, and its memAll fields."""
+    g = O.make_grid(n, x0=[0.0] * len(n), x1=[h * (m - 1) for h, m in zip(_h(n), n)])
+    out = []
+    for v in nodes:
+        a = np.zeros(O.memall_shape(g))
+        O.nodes_view(g, a)[...] = v
+        out.append(a)
+    return g, out
+
+
+def _view(n, g, a):
+    return O.nodes_view(g, a).reshape(tuple(reversed(n)))
+
+
+@pytest.mark.parametrize("n", NS)
+@pytest.mark.parametrize("border", ["KEEP", "FIELD", "VALUE", "NEUMANN", "CAUCHY", "RADIATION"])
+def test_heat(ctx, n, border):
+    u, f, g0, g1 = _rand(n, 1, 4)
+    mode = getattr(capi, "BORDER_" + border)
+    p = capi.Heat7Params(tau=0.02, coeff_a=1.0, rhoc_inv=1.0, perf_c=1.0, perf_w=0.5, has_perf=1, has_source=1,
+                         border_mode=mode, border_value=0.5, lam=1.0, alpha=1.0, epsilon=1.0, sigma=1.0)
+    g = capi.geom(n, h=_h(n))
+    known = [ctx.upload(v) for v in (f, g0, g1)]
+    _both(ctx, n, F64, {"u": u, "v": 0 * u},
+          lambda d: capi.check(ctx.L.scafes_heat7_step_f64(ctx.h, C.byref(g), 1, d["u"], d["v"],
+                                                           *[k.ptr for k in known], C.byref(p))), ["v"])
+    for k in known:
+        k.free()
+
+
+def _pennes(tumor):
+    p = capi.PennesParams(tau=0.02, cdiff=0.3, cperf=0.7, csrc=0.4, t_a=0.25)
+    if tumor:
+        p.border_mode, p.k_cond, p.h_conv, p.t_inf, p.q_bc = capi.BORDER_TUMOR, 0.5, 2.0, -0.5, 0.2
+    return p
+
+
+@pytest.mark.parametrize("n", NS)
+@pytest.mark.parametrize("tumor", [False, True])
+def test_pennes(ctx, n, tumor):
+    t, w, q, lam, c, grad = _rand(n, 2, 6)
+    c = 1e-8 * c
+    p, g = _pennes(tumor), capi.geom(n, h=_h(n))
+    step, adj = {}, {}
+    for code in (F64, F32):
+        step[code], = _both(ctx, n, code, {"t": t, "v": 0 * t, "w": w, "q": q},
+                            lambda d: capi.check(ctx.L.scafes_pennes_step(ctx.h, C.byref(g), 1, code, d["t"], d["v"],
+                                                                          d["w"], d["q"], C.byref(p))), ["v"])
+        adj[code] = _both(ctx, n, code, {"l": lam, "v": 0 * t, "w": w, "t": t, "grad": grad},
+                          lambda d: capi.check(ctx.L.scafes_pennes_adjoint_step(
+                              ctx.h, C.byref(g), 1, code, d["l"], d["v"], d["w"], d["t"], d["grad"], C.byref(p))),
+                          ["v", "grad"])
+    kahan, comp = _both(ctx, n, KAHAN, {"t": t, "v": 0 * t, "c": c, "d": 0 * t, "w": w, "q": q},
+                        lambda d: capi.check(ctx.L.scafes_pennes_step_kahan(
+                            ctx.h, C.byref(g), 1, d["t"], d["v"], d["c"], d["d"], d["w"], d["q"], C.byref(p))),
+                        ["v", "d"])
+    # about 20 roundings of terms below 4
+    tol = 20 * 4 * 2.0 ** -24
+    np.testing.assert_allclose(step[F32], step[F64], rtol=0, atol=tol)
+    np.testing.assert_allclose(kahan.astype(np.float64) + comp, step[F64], rtol=0, atol=tol)
+    for a, b in zip(adj[F32], adj[F64]):
+        np.testing.assert_allclose(a, b, rtol=0, atol=tol)
+    if tumor and min(n) > 1:
+        og, (mt, mw, mq, ml) = _ograd(n, (t, w, q, lam))
+        oc, ob = O.pennes_coef(p.tau, p.cdiff, p.cperf, p.csrc, p.t_a), O.tumor_border(0.5, 2.0, -0.5, 0.2)
+        np.testing.assert_allclose(step[F64], _view(n, og, O.pennes_tumor_step(og, mt, mw, mq, oc, ob)), rtol=0,
+                                   atol=20 * 4 * 2.0 ** -53)
+        np.testing.assert_allclose(adj[F64][0], _view(n, og, O.pennes_tumor_adjoint_step(og, ml, mw, oc, ob)),
+                                   rtol=0, atol=20 * 4 * 2.0 ** -53)
+
+
+@pytest.mark.parametrize("n", NS)
+@pytest.mark.parametrize("border", [capi.BORDER_KEEP, capi.BORDER_VALUE])
+def test_heatvar_step(ctx, n, border):
+    u, k, c = _rand(n, 3, 3)
+    k, c = 0.5 + k, 1e-8 * c
+    g, which, out = capi.geom(n, h=_h(n)), C.c_int(0), {}
+    for code in (F64, F32, KAHAN):
+        fields = {"u": u, "v": 0 * u, "c": c, "d": 0 * u, "k": k}
+        out[code] = _both(ctx, n, code, fields, lambda d: capi.check(ctx.L.scafes_heat7var_run(
+            ctx.h, C.byref(g), 1, HEATVAR[code], d["u"], d["v"], d["c"], d["d"], d["k"], 0.02, 1, border, 0.5, -1,
+            C.byref(which))), ["v", "d"])
+        tile = _both(ctx, n, code, fields, lambda d: capi.check(ctx.L.scafes_heat7var_run(
+            ctx.h, C.byref(g), 1, HEATVAR[code], d["u"], d["v"], d["c"], d["d"], d["k"], 0.02, 1, border, 0.5, 3,
+            C.byref(which))), ["v", "d"])
+        np.testing.assert_array_equal(out[code][0], tile[0])
+        if code == KAHAN:
+            np.testing.assert_array_equal(out[code][1], tile[1])
+    np.testing.assert_allclose(out[F32][0], out[F64][0], rtol=0, atol=20 * 4 * 2.0 ** -24)
+
+
+@pytest.mark.parametrize("n", [m for m in NS if min(m) > 2])
+@pytest.mark.parametrize("steps", [1, 2, 5])
+def test_gradients(ctx, n, steps):
+    """The kappa and perfusion adjoints (three stencil fields, face sums at border
+    nodes, (hi, lo) states): FP64 against the oracle, FP32 against FP64."""
+    u, k, tgt, w, q = _rand(n, 4, 5)
+    k = 0.5 + k
+    g, J = capi.geom(n, h=_h(n)), C.c_double(0)
+    kap, per = {}, {}
+    for code in (F64, F32, KAHAN):
+        kap[code], = _both(ctx, n, code, {"u": u, "k": k, "t": tgt, "grad": 0 * u}, lambda d: capi.check(
+            ctx.L.scafes_heat7var_gradient(ctx.h, C.byref(g), 1, HEATVAR[code], d["u"], d["k"], d["t"], 0.02,
+                                           capi.BORDER_KEEP, 0.0, steps, 3, d["grad"], C.byref(J), None)), ["grad"])
+        for tumor in (False, True):
+            p = _pennes(tumor)
+            per[code, tumor], = _both(ctx, n, code, {"u": u, "w": w, "q": q, "t": tgt, "grad": 0 * u},
+                                      lambda d: capi.check(ctx.L.scafes_pennes_gradient(
+                                          ctx.h, C.byref(g), 1, code, d["u"], d["w"], d["q"], d["t"], C.byref(p),
+                                          steps, 3, d["grad"], C.byref(J), None)), ["grad"])
+    og, (mu, mk, mt) = _ograd(n, (u, k, tgt))
+    states = O.heat7var_forward_all(og, mu, mk, 0.02, steps, border=O.BORDER_KEEP)
+    _, want = O.heat7var_grad(og, states, mk, mt, 0.02, steps)
+    scale = np.abs(kap[F64]).max()
+    np.testing.assert_allclose(kap[F64], _view(n, og, want), rtol=0, atol=1e-13 * scale)
+    # each step rounds states and terms of one size a few tens of times
+    for code in (F32, KAHAN):
+        np.testing.assert_allclose(kap[code], kap[F64], rtol=0, atol=steps * 100 * 2.0 ** -24 * scale)
+        for tumor in (False, True):
+            ref = per[F64, tumor]
+            np.testing.assert_allclose(per[code, tumor], ref, rtol=0,
+                                       atol=steps * 100 * 2.0 ** -24 * max(np.abs(ref).max(), 1e-3))
+
+
+@pytest.mark.parametrize("n", NS)
+def test_mri(ctx, n):
+    rng = np.random.default_rng(5 + sum(n))
+    shape = tuple(reversed(n))
+    mats = [1040.0 * (1 + 0.1 * rng.random(shape)), 3650.0 * (1 + 0.1 * rng.random(shape)), 0.5 + rng.random(shape),
+            np.full(shape, 1052.0), np.full(shape, 3800.0), 0.006 * rng.random(shape), 35.0 + rng.random(shape),
+            25000.0 * rng.random(shape), (rng.random(shape) < 0.5).astype(float)]
+    h = [0.003] * len(n)
+    g = capi.geom(n, h=h)
+    p = capi.MriParams(tau=2.0, h_conv=10.0, t_amb=22.0, q_bc=35.0, q_skull=-12.0, epsilon=0.98, sigma=5.670373e-8)
+    dm = [ctx.upload(np.ascontiguousarray(m)) for m in mats]
+    ptrs = (capi.vp * 9)(*[d.ptr for d in dm])
+    size = int(np.prod([m + 2 for m in n]))
+
+    def call(d):
+        coef = ctx.upload(np.full(capi.MRI_NCOEF * size, np.nan))  # the coefficients' ghosts stay NaN
+        capi.check(ctx.L.scafes_mri_coef_f64(ctx.h, C.byref(g), 1, ptrs, C.byref(p), coef.ptr))
+        capi.check(ctx.L.scafes_mri_step_f64(ctx.h, C.byref(g), 1, d["t"], d["v"], ptrs, coef.ptr, C.byref(p)))
+        ctx.sync()
+        coef.free()
+    t = 36.0 + rng.standard_normal(shape)
+    got, = _both(ctx, n, F64, {"t": t, "v": 0 * t}, call, ["v"])
+    if min(n) > 1:
+        og = O.make_grid(n, x0=[0.0] * len(n), x1=[q * (m - 1) for q, m in zip(h, n)])
+        u = np.zeros(O.memall_shape(og))
+        O.nodes_view(og, u)[...] = t
+        want = _view(n, og, O.mri_step(og, u, mats, O.mri_coef(2.0, 10.0, 22.0, 35.0, -12.0, 0.98)))
+        np.testing.assert_allclose(got, want, rtol=1e-13)
+    for d in dm:
+        d.free()
