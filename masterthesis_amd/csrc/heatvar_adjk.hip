@@ -46,16 +46,16 @@ struct AdjkStates {
     const void* u[kAdjMaxK];  // u[l] = u^{n-1-l}
 };
 
-template <typename T, int TX, int TY, int K, int D>
-__global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __restrict__ lam,
-                                                               T* __restrict__ lamo, const T* __restrict__ kap,
+template <int TX, int TY, int K, int D>
+__global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const float* __restrict__ lam,
+                                                               float* __restrict__ lamo, const float* __restrict__ kap,
                                                                AdjkStates st, double* __restrict__ grad,
                                                                AdjVarCoef cf, int zc, int tiles_x, int tiles_y)
 {
     static_assert(D >= 2 && D % 2 == 0, "prefetch depth must be even");
     static_assert(K >= 2 && K <= kAdjMaxK, "2 <= K <= kAdjMaxK");
     static_assert(TX % 64 == 0, "whole rows per wavefront: ty is wave-uniform");
-    constexpr int MODE = sizeof(T) == 8 ? 0 : 1;
+    constexpr int MODE = 1;
     constexpr int R = K - 1;  // rings the tile loses over the sweep
     constexpr int OX = TX - 2 * R, OY = TY - 2 * R;
     static_assert(OX >= 1 && OY >= 1, "tile too small for K levels");
@@ -67,10 +67,10 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
     auto ring = [](int c) { return ((c % H) + H) % H; };
     // lam^n and kappa with ring; row TY + 2 takes the y-ring writes of the
     // rows off the ring (a sink that is never read)
-    __shared__ T s0[2][TY + 3][TX + 2];
-    __shared__ T sk[2][TY + 3][TX + 2];
-    __shared__ T sl[K - 1][2][TY][TX];  // levels 1..K-1
-    __shared__ T su[K][2][TY][TX];      // u^{n-1-l} for the step-(n-l) term
+    __shared__ float s0[2][TY + 3][TX + 2];
+    __shared__ float sk[2][TY + 3][TX + 2];
+    __shared__ float sl[K - 1][2][TY][TX];  // levels 1..K-1
+    __shared__ float su[K][2][TY][TX];      // u^{n-1-l} for the step-(n-l) term
     const int tx = threadIdx.x;
     const int ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
     // the tile: only lanes whose result is discarded read a clamped position
     const int txm = max(tx - 1, 0), txp = min(tx + 1, TX - 1);
     const int tym = max(ty - 1, 0), typ = min(ty + 1, TY - 1);
-    constexpr uint32_t B = sizeof(T);
+    constexpr uint32_t B = sizeof(float);
     const uint32_t oc = (uint32_t)(g.base + ic + g.e0 * jc) * B;
     const uint32_t ohx = hx ? (uint32_t)(g.base + hxi + g.e0 * jc) * B : oc;
     const uint32_t ohy = hy ? (uint32_t)(g.base + ic + g.e0 * hyj) * B : kSkip;
@@ -122,13 +122,13 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
 #pragma unroll
     for (int l = 0; l < K; ++l) ru[l] = chunk_rsrc((const char*)st.u[l] + (size_t)kbase * pb);
 
-    T qa[D], qax[D], qay[D], qk[D], qkx[D], qky[D], qu[K][D];
+    float qa[D], qax[D], qay[D], qk[D], qkx[D], qky[D], qu[K][D];
     double qg[D];
 #pragma unroll
     for (int s = 0; s < D; ++s) {
-        qa[s] = qax[s] = qay[s] = qk[s] = qkx[s] = qky[s] = T(0);
+        qa[s] = qax[s] = qay[s] = qk[s] = qkx[s] = qky[s] = 0.0f;
 #pragma unroll
-        for (int l = 0; l < K; ++l) qu[l][s] = T(0);
+        for (int l = 0; l < K; ++l) qu[l][s] = 0.0f;
         qg[s] = 0.0;
     }
     // slot <- plane kk's lam^n and kappa (centre and ring), its stored
@@ -137,39 +137,39 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
     // values no output node needs are skipped through the offset.
     auto fetch = [&](const int slot, const int kk) {
         const uint32_t p = pl(kk) * pb;
-        qa[slot] = cload<T>(rl, oc, p);
-        qax[slot] = cload<T>(rl, ohx, p);
-        qay[slot] = cload<T>(rl, ohy, p);
-        qk[slot] = cload<T>(rk, oc, p);
-        qkx[slot] = cload<T>(rk, ohx, p);
-        qky[slot] = cload<T>(rk, ohy, p);
+        qa[slot] = cload<float>(rl, oc, p);
+        qax[slot] = cload<float>(rl, ohx, p);
+        qay[slot] = cload<float>(rl, ohy, p);
+        qk[slot] = cload<float>(rk, oc, p);
+        qkx[slot] = cload<float>(rk, ohx, p);
+        qky[slot] = cload<float>(rk, ohy, p);
 #pragma unroll
         for (int l = 0; l < K; ++l) {
             const int pp = kk - l;
-            qu[l][slot] = cload<T>(ru[l], (pp >= k0 - 1 && pp <= k1) ? ous : kSkip, pl(pp) * pb);
+            qu[l][slot] = cload<float>(ru[l], (pp >= k0 - 1 && pp <= k1) ? ous : kSkip, pl(pp) * pb);
         }
         qg[slot] = cload<double>(rg, (kk >= k0 && kk < k1) ? og : kSkip, pl(kk) * pg);
     };
 #pragma unroll
     for (int s = 0; s < D; ++s) fetch(s, kstart + s);
 
-    T hist[K][H];         // hist[l][ring(it)]: level l at the plane it computed in iteration it
-    Faces<T> fr[H];       // fr[ring(it)]: faces of plane kstart + it
+    float hist[K][H];         // hist[l][ring(it)]: level l at the plane it computed in iteration it
+    Faces<float> fr[H];       // fr[ring(it)]: faces of plane kstart + it
     double sum[H];        // sum[ring(it)]: running gradient of plane kstart + it
-    T um[K];              // u^{n-1-l} one plane below the plane its term is formed at
+    float um[K];              // u^{n-1-l} one plane below the plane its term is formed at
 #pragma unroll
     for (int a = 0; a < H; ++a) {
-        fr[a] = Faces<T>{};
+        fr[a] = Faces<float>{};
         sum[a] = 0.0;
 #pragma unroll
-        for (int l = 0; l < K; ++l) hist[l][a] = T(0);
+        for (int l = 0; l < K; ++l) hist[l][a] = 0.0f;
     }
-    hist[0][ring(-1)] = cload<T>(rl, oc, pl(kstart - 1) * pb);
-    fr[ring(-1)].u = face<T, MODE>(qk[0], cload<T>(rk, oc, pl(kstart - 1) * pb));
+    hist[0][ring(-1)] = cload<float>(rl, oc, pl(kstart - 1) * pb);
+    fr[ring(-1)].u = face<float, MODE>(qk[0], cload<float>(rk, oc, pl(kstart - 1) * pb));
 #pragma unroll
     for (int l = 0; l < K; ++l) {
         const int pp = kstart - l - 1;
-        um[l] = cload<T>(ru[l], (pp >= k0 - 1 && pp <= k1) ? ous : kSkip, pl(pp) * pb);
+        um[l] = cload<float>(ru[l], (pp >= k0 - 1 && pp <= k1) ? ous : kSkip, pl(pp) * pb);
     }
     for (int kb = kstart; kb <= kend; kb += U) {
 #pragma unroll
@@ -179,9 +179,9 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
             // the exit leaves the register rings dead (no copies on this path)
             if (k > kend) return;
             const int s = u % D, buf = u & 1, pbf = buf ^ 1;
-            const T ac = qa[s], ap = qa[(s + 1) % D], am = hist[0][ring(u - 1)];
-            const T bc = qk[s], bp = qk[(s + 1) % D];
-            T uc[K], up[K];
+            const float ac = qa[s], ap = qa[(s + 1) % D], am = hist[0][ring(u - 1)];
+            const float bc = qk[s], bp = qk[(s + 1) % D];
+            float uc[K], up[K];
 #pragma unroll
             for (int l = 0; l < K; ++l) {
                 uc[l] = qu[l][s];
@@ -200,27 +200,27 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
             fetch(s, k + D);
             __syncthreads();
             // ---- level 1: lam^{n-1} at plane k, every thread; the faces of plane k
-            const T lw = s0[buf][ty + 1][tx], le = s0[buf][ty + 1][tx + 2];
-            const T ls = s0[buf][ty][tx + 1], ln = s0[buf][ty + 2][tx + 1];
-            Faces<T> f;
-            f.e = face<T, MODE>(sk[buf][ty + 1][tx + 2], bc);
-            f.w = face<T, MODE>(bc, sk[buf][ty + 1][tx]);
-            f.n = face<T, MODE>(sk[buf][ty + 2][tx + 1], bc);
-            f.s = face<T, MODE>(bc, sk[buf][ty][tx + 1]);
-            f.u = face<T, MODE>(bp, bc);
+            const float lw = s0[buf][ty + 1][tx], le = s0[buf][ty + 1][tx + 2];
+            const float ls = s0[buf][ty][tx + 1], ln = s0[buf][ty + 2][tx + 1];
+            Faces<float> f;
+            f.e = face<float, MODE>(sk[buf][ty + 1][tx + 2], bc);
+            f.w = face<float, MODE>(bc, sk[buf][ty + 1][tx]);
+            f.n = face<float, MODE>(sk[buf][ty + 2][tx + 1], bc);
+            f.s = face<float, MODE>(bc, sk[buf][ty][tx + 1]);
+            f.u = face<float, MODE>(bp, bc);
             f.d = fr[ring(u - 1)].u;
             fr[ring(u)] = f;
             {
-                T dummy;
-                T l1 = var_update<T, MODE>(cf.v, ac, lw, le, ls, ln, am, ap, f, T(0), &dummy);
+                float dummy;
+                float l1 = var_update<float, MODE>(cf.v, ac, lw, le, ls, ln, am, ap, f, 0.0f, &dummy);
                 const bool in1 = inner_i && inner_j && k >= klo && k <= khi;
-                l1 = in1 ? l1 : T(0);
+                l1 = in1 ? l1 : 0.0f;
                 hist[1][ring(u)] = l1;
                 sl[0][buf][ty][tx] = l1;
             }
             // ---- step-n term at plane k (output rows and planes)
             if (row_out && k >= k0 && k < k1) {  // wave-uniform
-                const double t = adj_term3<T>(cf, xlo, xhi, ylo, yhi, k > 0, k < g.nz - 1, ac, lw, le, ls, ln, am,
+                const double t = adj_term3(cf, xlo, xhi, ylo, yhi, k > 0, k < g.nz - 1, ac, lw, le, ls, ln, am,
                                               ap, uc[0], su[0][buf][ty][txm], su[0][buf][ty][txp],
                                               su[0][buf][tym][tx], su[0][buf][typ][tx], um[0], up[0]);
                 sum[ring(u)] = gl + t;
@@ -230,20 +230,20 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
             for (int L = 2; L <= K; ++L) {
                 const int p = k - (L - 1);
                 const bool inz = p >= klo && p <= khi;
-                const T lc = hist[L - 1][ring(u - 1)], lm = hist[L - 1][ring(u - 2)], lp = hist[L - 1][ring(u)];
-                T v = T(0);
+                const float lc = hist[L - 1][ring(u - 1)], lm = hist[L - 1][ring(u - 2)], lp = hist[L - 1][ring(u)];
+                float v = 0.0f;
                 if (ty >= L - 1 && ty <= TY - L && inner_j && inz) {  // wave-uniform
-                    T dummy;
-                    v = var_update<T, MODE>(cf.v, lc, sl[L - 2][pbf][ty][txm], sl[L - 2][pbf][ty][txp],
+                    float dummy;
+                    v = var_update<float, MODE>(cf.v, lc, sl[L - 2][pbf][ty][txm], sl[L - 2][pbf][ty][txp],
                                             sl[L - 2][pbf][tym][tx], sl[L - 2][pbf][typ][tx], lm, lp,
-                                            fr[ring(u - (L - 1))], T(0), &dummy);
-                    v = (tx >= L - 1 && tx <= TX - L && inner_i) ? v : T(0);
+                                            fr[ring(u - (L - 1))], 0.0f, &dummy);
+                    v = (tx >= L - 1 && tx <= TX - L && inner_i) ? v : 0.0f;
                 }
                 if (row_out && p >= k0 && p < k1) {  // wave-uniform
                     // level L-1 (lam^{n-L+1}) at plane p with u^{n-L} = state L-1
                     const int l = L - 1;
                     const double t =
-                        adj_term3<T>(cf, xlo, xhi, ylo, yhi, p > 0, p < g.nz - 1, lc, sl[l - 1][pbf][ty][txm],
+                        adj_term3(cf, xlo, xhi, ylo, yhi, p > 0, p < g.nz - 1, lc, sl[l - 1][pbf][ty][txm],
                                      sl[l - 1][pbf][ty][txp], sl[l - 1][pbf][tym][tx], sl[l - 1][pbf][typ][tx], lm,
                                      lp, uc[l], su[l][buf][ty][txm], su[l][buf][ty][txp], su[l][buf][tym][tx],
                                      su[l][buf][typ][tx], um[l], up[l]);
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
                     hist[L][ring(u)] = v;
                     sl[L - 1][buf][ty][tx] = v;
                 } else if (row_out && p >= k0) {  // wave-uniform; p < k1 always
-                    cstore<T>(v, rlo, oo, pl(p) * pb);
+                    cstore<float>(v, rlo, oo, pl(p) * pb);
                     cstore<double>(sum[ring(u - R)], rg, og, pl(p) * pg);
                 }
             }
@@ -284,34 +284,33 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adjk_kernel(Geo g, const T* __
 // (fit_chunk): K = 4 FP32 at 97x80x75 123 -> 24 us per sweep, 128^3 127 -> 57.
 // FP32, K = 3: 64 x 12 (64 x 16 caps a thread at 128 VGPRs, which the
 // three-step rings exceed by a 16-byte spill).
-template <typename T, int K>
+template <int K>
 struct AdjkTile {
     static constexpr int TX = 64, TY = K == 3 ? 12 : 16, D = 2, ZC = 64, PER_CU = 1;
 };
 
-template <typename T, int K>
+template <int K>
 int adjk_launch_t(Ctx* c, const Geo& g, const void* lam, void* lamo, const void* kap, const AdjkStates& st,
                   double* grad, const AdjVarCoef& cf)
 {
-    typedef AdjkTile<T, K> A;
+    typedef AdjkTile<K> A;
     constexpr int R = K - 1;
     const int tiles_x = ceil_div(g.nx, A::TX - 2 * R), tiles_y = ceil_div(g.ny, A::TY - 2 * R);
     const int zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * R + 1, A::ZC, A::PER_CU, c->cu_count);
     const long nb = (long)tiles_x * tiles_y * ceil_div(g.nz, zc);
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");
-    heatvar_adjk_kernel<T, A::TX, A::TY, K, A::D><<<dim3((unsigned)nb), dim3(A::TX, A::TY), 0, c->stream>>>(
-        g, (const T*)lam, (T*)lamo, (const T*)kap, st, grad, cf, zc, tiles_x, tiles_y);
+    heatvar_adjk_kernel<A::TX, A::TY, K, A::D><<<dim3((unsigned)nb), dim3(A::TX, A::TY), 0, c->stream>>>(
+        g, (const float*)lam, (float*)lamo, (const float*)kap, st, grad, cf, zc, tiles_x, tiles_y);
     SCAFES_HIP(hipGetLastError());
     return SCAFES_OK;
 }
 
-template <typename T>
 int adjk_launch_k(Ctx* c, const Geo& g, int K, const void* lam, void* lamo, const void* kap, const AdjkStates& st,
                   double* grad, const AdjVarCoef& cf)
 {
-    if (K == 2) return adjk_launch_t<T, 2>(c, g, lam, lamo, kap, st, grad, cf);
-    if (K == 3) return adjk_launch_t<T, 3>(c, g, lam, lamo, kap, st, grad, cf);
-    if (K == 4) return adjk_launch_t<T, 4>(c, g, lam, lamo, kap, st, grad, cf);
+    if (K == 2) return adjk_launch_t<2>(c, g, lam, lamo, kap, st, grad, cf);
+    if (K == 3) return adjk_launch_t<3>(c, g, lam, lamo, kap, st, grad, cf);
+    if (K == 4) return adjk_launch_t<4>(c, g, lam, lamo, kap, st, grad, cf);
     return fail(SCAFES_ERR_ARG, "multi-step var-kappa adjoint: K out of range");
 }
 
@@ -350,13 +349,10 @@ int heatvar_adjk_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype,
     cf.v.c2 = (float)(0.5 * tau / hh[2]);
     cf.v.border_value = 0.0;
     cf.v.border_mode = SCAFES_BORDER_VALUE;
-    cf.th0 = tau / hh[0];
-    cf.th1 = tau / hh[1];
-    cf.th2 = tau / hh[2];
-    cf.f0 = (float)(0.5 * cf.th0);
-    cf.f1 = (float)(0.5 * cf.th1);
-    cf.f2 = (float)(0.5 * cf.th2);
-    return adjk_launch_k<float>(c, geo, K, lam, lamo, kap, st, grad, cf);
+    cf.f0 = (float)(0.5 * (tau / hh[0]));
+    cf.f1 = (float)(0.5 * (tau / hh[1]));
+    cf.f2 = (float)(0.5 * (tau / hh[2]));
+    return adjk_launch_k(c, geo, K, lam, lamo, kap, st, grad, cf);
 }
 
 }  // namespace scafes

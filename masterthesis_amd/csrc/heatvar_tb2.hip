@@ -406,15 +406,11 @@ __global__ __launch_bounds__(TX* TY) void heatvar_tb3_kernel(Geo g, const T* __r
 // three-step kernel: wave-uniform row branches, off-ring rows writing the y
 // ring into a sink row, lanes off the output columns storing out of range.
 // Per four steps HBM moves one sweep of u, kappa (and c) plus the ring.
-// MO: the states after one, two and three steps are written too (u1o, u2o,
-// u3o; the value part only in the compensated mode) at every node of the
-// output tile, as the one-step kernel would write them.
-template <typename T, int MODE, int TX, int TY, int D, bool MO = false>
+template <typename T, int MODE, int TX, int TY, int D>
 __global__ __launch_bounds__(TX* TY) void heatvar_tb4_kernel(Geo g, const T* __restrict__ u, const T* __restrict__ cin,
                                                               const T* __restrict__ kap, T* __restrict__ uout,
-                                                              T* __restrict__ cout, T* __restrict__ u1o,
-                                                              T* __restrict__ u2o, T* __restrict__ u3o, VarCoef cf,
-                                                              int zc, int tiles_x, int tiles_y)
+                                                              T* __restrict__ cout, VarCoef cf, int zc, int tiles_x,
+                                                              int tiles_y)
 {
     static_assert(D >= 2 && D % 2 == 0, "prefetch depth must be even");
     static_assert(TX % 64 == 0, "whole rows per wavefront: ty is wave-uniform");
@@ -531,10 +527,6 @@ __global__ __launch_bounds__(TX* TY) void heatvar_tb4_kernel(Geo g, const T* __r
                 c1 = keep ? c0 : T(0);
             }
             s1[buf][ty][tx] = l1;
-            if constexpr (MO) {
-                const uint32_t os1 = (k >= k0 && k < k1 && row_out) ? oo : range;
-                bstore<T>(l1, plane_rsrc((const char*)u1o + plane(k), range), os1);
-            }
             // ---- level 2 at plane k-1 on rows 1..TY-2
             const int k2 = k - 1;
             T c2 = T(0), l2 = T(0);
@@ -547,10 +539,6 @@ __global__ __launch_bounds__(TX* TY) void heatvar_tb4_kernel(Geo g, const T* __r
                 }
             }
             s2[buf][ty][tx] = l2;
-            if constexpr (MO) {
-                const uint32_t os2 = (k2 >= k0 && k2 < k1 && row_out) ? oo : range;
-                bstore<T>(l2, plane_rsrc((const char*)u2o + plane(k2), range), os2);
-            }
             // ---- level 3 at plane k-2 on rows 2..TY-3
             const int k3 = k - 2;
             T c3 = T(0), l3 = T(0);
@@ -563,10 +551,6 @@ __global__ __launch_bounds__(TX* TY) void heatvar_tb4_kernel(Geo g, const T* __r
                 }
             }
             s3[buf][ty][tx] = l3;
-            if constexpr (MO) {
-                const uint32_t os3 = (k3 >= k0 && k3 < k1 && row_out) ? oo : range;
-                bstore<T>(l3, plane_rsrc((const char*)u3o + plane(k3), range), os3);
-            }
             // ---- level 4 at plane k-3 on the output rows and planes
             const int k4 = k - 3;
             {
@@ -622,21 +606,21 @@ __global__ __launch_bounds__(TX* TY) void heatvar_tb4_kernel(Geo g, const T* __r
 // Per two reverse steps HBM moves lam r+w, kappa, u^{n-1}, u^{n-2} and the
 // FP64 gradient r+w once: 36 B per node for FP32 fields (18 per step,
 // against 32 for one-step launches).
-template <typename T, int TX, int TY, int D>
-__global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __restrict__ lam,
-                                                               const T* __restrict__ kap, const T* __restrict__ u1,
-                                                               const T* __restrict__ u2, T* __restrict__ lamo,
+template <int TX, int TY, int D>
+__global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const float* __restrict__ lam,
+                                                               const float* __restrict__ kap, const float* __restrict__ u1,
+                                                               const float* __restrict__ u2, float* __restrict__ lamo,
                                                                double* __restrict__ grad, AdjVarCoef cf, int zc,
                                                                int tiles_x, int tiles_y)
 {
     static_assert(D >= 2 && D % 2 == 0, "prefetch depth must be even");
     constexpr int OX = TX - 2, OY = TY - 2;
-    constexpr int MODE = sizeof(T) == 8 ? 0 : 1;
-    __shared__ T s0[2][TY + 2][TX + 2];  // lam^n plane with ring
-    __shared__ T sk[2][TY + 2][TX + 2];  // kappa plane with ring
-    __shared__ T sa[2][TY][TX];          // u^{n-1} plane
-    __shared__ T s1[2][TY][TX];          // lam^{n-1} plane
-    __shared__ T sb[2][TY][TX];          // u^{n-2} plane
+    constexpr int MODE = 1;
+    __shared__ float s0[2][TY + 2][TX + 2];  // lam^n plane with ring
+    __shared__ float sk[2][TY + 2][TX + 2];  // kappa plane with ring
+    __shared__ float sa[2][TY][TX];          // u^{n-1} plane
+    __shared__ float s1[2][TY][TX];          // lam^{n-1} plane
+    __shared__ float sb[2][TY][TX];          // u^{n-2} plane
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
     const int per_plane = tiles_x * tiles_y;
@@ -658,7 +642,7 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
     const int hyj = (ty == 0) ? max(jc - 1, 0) : min(jc + 1, g.ny - 1);
     const int sxh = (tx == 0) ? 0 : TX + 1;
     const int syh = (ty == 0) ? 0 : TY + 1;
-    constexpr uint32_t B = sizeof(T);
+    constexpr uint32_t B = sizeof(float);
     const uint32_t oc = (uint32_t)(g.base + ic + g.e0 * jc) * B;
     const uint32_t ohx = (uint32_t)(g.base + hxi + g.e0 * jc) * B;
     const uint32_t ohy = (uint32_t)(g.base + ic + g.e0 * hyj) * B;
@@ -674,11 +658,11 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
     const char* gb8 = (const char*)grad;
     auto plane = [&](int kk) { return (size_t)min(max(kk, 0), g.nz - 1); };
 
-    T qa[D], qk[D], qu1[D], qu2[D], qax[D], qkx[D], qay[D], qky[D];
+    float qa[D], qk[D], qu1[D], qu2[D], qax[D], qkx[D], qay[D], qky[D];
     double qg[D];
 #pragma unroll
     for (int s = 0; s < D; ++s) {
-        qa[s] = qk[s] = qu1[s] = qu2[s] = qax[s] = qkx[s] = qay[s] = qky[s] = T(0);
+        qa[s] = qk[s] = qu1[s] = qu2[s] = qax[s] = qkx[s] = qay[s] = qky[s] = 0.0f;
         qg[s] = 0.0;
     }
     auto fetch = [&](const int slot, const int kk) {
@@ -688,37 +672,37 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
         const bool cen = kk <= kcen, mid = kk <= k1;
         const uint32_t occ = cen ? oc : range, ocm = mid ? oc : range;
         const uint32_t ox = (mid && hx) ? ohx : range, oy = (mid && hy) ? ohy : range;
-        qa[slot] = bload<T>(rl, occ);
-        qk[slot] = bload<T>(rk, occ);
-        qu1[slot] = bload<T>(plane_rsrc(ab8 + o, range), occ);
-        qu2[slot] = bload<T>(plane_rsrc(bb8 + o, range), ocm);
-        qax[slot] = bload<T>(rl, ox);
-        qkx[slot] = bload<T>(rk, ox);
-        qay[slot] = bload<T>(rl, oy);
-        qky[slot] = bload<T>(rk, oy);
+        qa[slot] = bload<float>(rl, occ);
+        qk[slot] = bload<float>(rk, occ);
+        qu1[slot] = bload<float>(plane_rsrc(ab8 + o, range), occ);
+        qu2[slot] = bload<float>(plane_rsrc(bb8 + o, range), ocm);
+        qax[slot] = bload<float>(rl, ox);
+        qkx[slot] = bload<float>(rk, ox);
+        qay[slot] = bload<float>(rl, oy);
+        qky[slot] = bload<float>(rk, oy);
         qg[slot] = bload<double>(plane_rsrc(gb8 + pk * pg, rangeg), (mid && out_thread) ? og : rangeg);
     };
-    T am = bload<T>(plane_rsrc(lb8 + plane(kstart - 1) * pb, range), oc);
-    T u1m = bload<T>(plane_rsrc(ab8 + plane(kstart - 1) * pb, range), oc);
-    const T km = bload<T>(plane_rsrc(kb8 + plane(kstart - 1) * pb, range), oc);
+    float am = bload<float>(plane_rsrc(lb8 + plane(kstart - 1) * pb, range), oc);
+    float u1m = bload<float>(plane_rsrc(ab8 + plane(kstart - 1) * pb, range), oc);
+    const float km = bload<float>(plane_rsrc(kb8 + plane(kstart - 1) * pb, range), oc);
 #pragma unroll
     for (int s = 0; s < D; ++s) fetch(s, kstart + s);
 
-    T l1m2 = T(0), l1m1 = T(0);     // level 1 at planes k-2, k-1
-    T u2m2 = T(0), u2m1 = T(0);     // u^{n-2} at planes k-2, k-1
+    float l1m2 = 0.0f, l1m1 = 0.0f;     // level 1 at planes k-2, k-1
+    float u2m2 = 0.0f, u2m1 = 0.0f;     // u^{n-2} at planes k-2, k-1
     double t1m1 = 0.0, gm1 = 0.0;   // step-n term and gradient of plane k-1
-    Faces<T> fp = {};
-    T fup = face<T, MODE>(qk[0], km);
+    Faces<float> fp = {};
+    float fup = face<float, MODE>(qk[0], km);
     for (int kb = kstart; kb <= k1; kb += D) {
 #pragma unroll
         for (int s = 0; s < D; ++s) {
             const int k = kb + s;
             if (k > k1) break;  // uniform over the workgroup
             const int buf = s & 1, pbf = buf ^ 1;
-            const T ac = qa[s], ap = qa[(s + 1) % D];
-            const T bc = qk[s], bp = qk[(s + 1) % D];
-            const T uc = qu1[s], up = qu1[(s + 1) % D];
-            const T vc = qu2[s];
+            const float ac = qa[s], ap = qa[(s + 1) % D];
+            const float bc = qk[s], bp = qk[(s + 1) % D];
+            const float uc = qu1[s], up = qu1[(s + 1) % D];
+            const float vc = qu2[s];
             const double gk = qg[s];
             s0[buf][ty + 1][tx + 1] = ac;
             sk[buf][ty + 1][tx + 1] = bc;
@@ -734,18 +718,18 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
             fetch(s, k + D);
             __syncthreads();
             // ---- level 1 at (i, j, k): lam^{n-1}, every position
-            const T lw = s0[buf][ty + 1][tx], le = s0[buf][ty + 1][tx + 2];
-            const T ls = s0[buf][ty][tx + 1], ln = s0[buf][ty + 2][tx + 1];
-            Faces<T> f;
-            f.e = face<T, MODE>(sk[buf][ty + 1][tx + 2], bc);
-            f.w = face<T, MODE>(bc, sk[buf][ty + 1][tx]);
-            f.n = face<T, MODE>(sk[buf][ty + 2][tx + 1], bc);
-            f.s = face<T, MODE>(bc, sk[buf][ty][tx + 1]);
-            f.u = face<T, MODE>(bp, bc);
+            const float lw = s0[buf][ty + 1][tx], le = s0[buf][ty + 1][tx + 2];
+            const float ls = s0[buf][ty][tx + 1], ln = s0[buf][ty + 2][tx + 1];
+            Faces<float> f;
+            f.e = face<float, MODE>(sk[buf][ty + 1][tx + 2], bc);
+            f.w = face<float, MODE>(bc, sk[buf][ty + 1][tx]);
+            f.n = face<float, MODE>(sk[buf][ty + 2][tx + 1], bc);
+            f.s = face<float, MODE>(bc, sk[buf][ty][tx + 1]);
+            f.u = face<float, MODE>(bp, bc);
             f.d = fup;
-            T dummy;
-            T l1 = var_update<T, MODE>(cf.v, ac, lw, le, ls, ln, am, ap, f, T(0), &dummy);
-            if (!(inner_xy && k >= klo && k <= khi)) l1 = T(0);
+            float dummy;
+            float l1 = var_update<float, MODE>(cf.v, ac, lw, le, ls, ln, am, ap, f, 0.0f, &dummy);
+            if (!(inner_xy && k >= klo && k <= khi)) l1 = 0.0f;
             // planes read one iteration later are written after the barrier
             // (a write before it could overtake a slower thread still reading
             // the same buffer two planes back)
@@ -756,7 +740,7 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
             double t1 = 0.0;
             if (out_thread) {
                 const int txm = tx - 1, txp = tx + 1, tym = ty - 1, typ = ty + 1;
-                t1 = adj_term3<T>(cf, i > 0, i < g.nx - 1, j > 0, j < g.ny - 1, k > 0, k < g.nz - 1, ac, lw, le, ls,
+                t1 = adj_term3(cf, i > 0, i < g.nx - 1, j > 0, j < g.ny - 1, k > 0, k < g.nz - 1, ac, lw, le, ls,
                                   ln, am, ap, uc, sa[buf][ty][txm], sa[buf][ty][txp], sa[buf][tym][tx],
                                   sa[buf][typ][tx], u1m, up);
             }
@@ -764,15 +748,15 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
             const int k2 = k - 1;
             {
                 const bool st = k2 >= k0 && out_thread;
-                T v = T(0);
+                float v = 0.0f;
                 double gv = 0.0;
                 if (st) {
-                    const T pw = s1[pbf][ty][tx - 1], pe = s1[pbf][ty][tx + 1];
-                    const T ps = s1[pbf][ty - 1][tx], pn = s1[pbf][ty + 1][tx];
-                    T dummy2;
-                    v = var_update<T, MODE>(cf.v, l1m1, pw, pe, ps, pn, l1m2, l1, fp, T(0), &dummy2);
-                    if (!(inner_xy && k2 >= klo && k2 <= khi)) v = T(0);
-                    const double t2 = adj_term3<T>(cf, i > 0, i < g.nx - 1, j > 0, j < g.ny - 1, k2 > 0,
+                    const float pw = s1[pbf][ty][tx - 1], pe = s1[pbf][ty][tx + 1];
+                    const float ps = s1[pbf][ty - 1][tx], pn = s1[pbf][ty + 1][tx];
+                    float dummy2;
+                    v = var_update<float, MODE>(cf.v, l1m1, pw, pe, ps, pn, l1m2, l1, fp, 0.0f, &dummy2);
+                    if (!(inner_xy && k2 >= klo && k2 <= khi)) v = 0.0f;
+                    const double t2 = adj_term3(cf, i > 0, i < g.nx - 1, j > 0, j < g.ny - 1, k2 > 0,
                                                    k2 < g.nz - 1, l1m1, pw, pe, ps, pn, l1m2, l1, u2m1,
                                                    sb[pbf][ty][tx - 1], sb[pbf][ty][tx + 1], sb[pbf][ty - 1][tx],
                                                    sb[pbf][ty + 1][tx], u2m2, vc);
@@ -780,7 +764,7 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
                     gv = gv + t2;
                 }
                 const uint32_t os = st ? oo : range;
-                bstore<T>(v, plane_rsrc((const char*)lamo + plane(k2) * pb, range), os);
+                bstore<float>(v, plane_rsrc((const char*)lamo + plane(k2) * pb, range), os);
                 bstore<double>(gv, plane_rsrc((const char*)grad + plane(k2) * pg, rangeg), st ? og : rangeg);
             }
             l1m2 = l1m1;
@@ -802,7 +786,6 @@ __global__ __launch_bounds__(TX* TY) void heatvar_adj2_kernel(Geo g, const T* __
 // Measured at 512^3 FP32 on an MI355X (us per two-step launch): 64x8 with
 // 64-plane chunks 1372, with 32 1395; 64x16 with 64 1408, with 32 1461;
 // 64x12 with 32 1724 (the results are bit-identical across tiles).
-template <typename T>
 struct Adj2Tile {
     static constexpr int TX = 64, TY = 8, D = 2, ZC = 64;
 };
@@ -813,16 +796,15 @@ bool heatvar_adj2_supported(const Geo& geo)
     return geo.dim == 3 && (geo.base + geo.e01) * 8 < kOobLimit;
 }
 
-template <typename T>
-static int adj2_launch_t(Ctx* c, const Geo& g, const void* lam, void* lamo, const void* kap, const void* u1,
+static int adj2_launch_f32(Ctx* c, const Geo& g, const void* lam, void* lamo, const void* kap, const void* u1,
                          const void* u2, double* grad, const AdjVarCoef& cf)
 {
-    typedef Adj2Tile<T> A;
+    typedef Adj2Tile A;
     const int tiles_x = ceil_div(g.nx, A::TX - 2), tiles_y = ceil_div(g.ny, A::TY - 2);
     const long nb = (long)tiles_x * tiles_y * ceil_div(g.nz, A::ZC);
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");
-    heatvar_adj2_kernel<T, A::TX, A::TY, A::D><<<dim3((unsigned)nb), dim3(A::TX, A::TY), 0, c->stream>>>(
-        g, (const T*)lam, (const T*)kap, (const T*)u1, (const T*)u2, (T*)lamo, grad, cf, A::ZC, tiles_x, tiles_y);
+    heatvar_adj2_kernel<A::TX, A::TY, A::D><<<dim3((unsigned)nb), dim3(A::TX, A::TY), 0, c->stream>>>(
+        g, (const float*)lam, (const float*)kap, (const float*)u1, (const float*)u2, (float*)lamo, grad, cf, A::ZC, tiles_x, tiles_y);
     SCAFES_HIP(hipGetLastError());
     return SCAFES_OK;
 }
@@ -841,14 +823,11 @@ int heatvar_adj2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype,
     cf.v.c2 = (float)(0.5 * tau / hh[2]);
     cf.v.border_value = 0.0;
     cf.v.border_mode = SCAFES_BORDER_VALUE;
-    cf.th0 = tau / hh[0];
-    cf.th1 = tau / hh[1];
-    cf.th2 = tau / hh[2];
-    cf.f0 = (float)(0.5 * cf.th0);
-    cf.f1 = (float)(0.5 * cf.th1);
-    cf.f2 = (float)(0.5 * cf.th2);
+    cf.f0 = (float)(0.5 * (tau / hh[0]));
+    cf.f1 = (float)(0.5 * (tau / hh[1]));
+    cf.f2 = (float)(0.5 * (tau / hh[2]));
     if (dtype == SCAFES_F64) return fail(SCAFES_ERR_UNSUPPORTED, "FP64 kappa adjoints take one step per launch");
-    return adj2_launch_t<float>(c, geo, lam, lamo, kap, u1, u2, grad, cf);
+    return adj2_launch_f32(c, geo, lam, lamo, kap, u1, u2, grad, cf);
 }
 
 // Multi-step tiles: steps per sweep (2, 3 or 4), workgroup tile, z planes
@@ -881,9 +860,8 @@ static int tb_launch_t(Ctx* c, const Geo& g, const void* u, const void* cin, con
         heatvar_tb2_kernel<T, MODE, TX, TY, D><<<dim3((unsigned)nb), dim3(TX, TY), 0, c->stream>>>(
             g, (const T*)u, (const T*)cin, (const T*)kap, (T*)uo, (T*)co, cf, zc, tiles_x, tiles_y);
     else if constexpr (STEPS == 4)
-        heatvar_tb4_kernel<T, MODE, TX, TY, D, MO><<<dim3((unsigned)nb), dim3(TX, TY), 0, c->stream>>>(
-            g, (const T*)u, (const T*)cin, (const T*)kap, (T*)uo, (T*)co, MO ? (T*)mid[0] : nullptr,
-            MO ? (T*)mid[1] : nullptr, MO ? (T*)mid[2] : nullptr, cf, zc, tiles_x, tiles_y);
+        heatvar_tb4_kernel<T, MODE, TX, TY, D><<<dim3((unsigned)nb), dim3(TX, TY), 0, c->stream>>>(
+            g, (const T*)u, (const T*)cin, (const T*)kap, (T*)uo, (T*)co, cf, zc, tiles_x, tiles_y);
     else
         heatvar_tb3_kernel<T, MODE, TX, TY, D, MO><<<dim3((unsigned)nb), dim3(TX, TY), 0, c->stream>>>(
             g, (const T*)u, (const T*)cin, (const T*)kap, (T*)uo, (T*)co, MO ? (T*)mid[0] : nullptr,
@@ -928,29 +906,25 @@ static int tb_dispatch(Ctx* c, const Geo& g, const void* u, const void* cin, con
     return fail(SCAFES_ERR_ARG, "bad multi-step tile configuration");
 }
 
-// Multi-step sweeps that also write the intermediate states: the default
-// three-step tiles (F64 64x16, F32 64x12, prefetch depth 2) and the 64x16
-// four-step tile with prefetch depth 2.
-template <typename T, int MODE>
-static int tb_dispatch_mo(Ctx* c, const Geo& g, const void* u, const void* cin, const void* kap, void* uo, void* co,
-                          const VarCoef& cf, int cfg, bool fit, void* const* mid)
+// FP64 sweeps that also write the intermediate states: the default three-step
+// tile and the 64x12 one.
+static int tb_dispatch_mo(Ctx* c, const Geo& g, const void* u, const void* kap, void* uo, const VarCoef& cf, int cfg,
+                          bool fit, void* const* mid)
 {
     const TbCfg t = kTbCfgs[cfg];
     if (t.steps == 3 && t.tx == 64 && t.ty == 16 && t.d == 2)
-        return tb_launch_t<3, T, MODE, 64, 16, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, fit, mid);
+        return tb_launch_t<3, double, 0, 64, 16, 2, true>(c, g, u, nullptr, kap, uo, nullptr, cf, t.zc, fit, mid);
     if (t.steps == 3 && t.tx == 64 && t.ty == 12 && t.d == 2)
-        return tb_launch_t<3, T, MODE, 64, 12, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, fit, mid);
-    if (t.steps == 4 && t.tx == 64 && t.ty == 16 && t.d == 2)
-        return tb_launch_t<4, T, MODE, 64, 16, 2, true>(c, g, u, cin, kap, uo, co, cf, t.zc, fit, mid);
+        return tb_launch_t<3, double, 0, 64, 12, 2, true>(c, g, u, nullptr, kap, uo, nullptr, cf, t.zc, fit, mid);
     return fail(SCAFES_ERR_UNSUPPORTED, "no state-writing variant of this multi-step tile");
 }
 
-bool heatvar_tb_states_supported(int cfg)
+bool heatvar_tb_states_supported(int cfg, int mode)
 {
     if (cfg < 0 || cfg >= kNumTb) return false;
     const TbCfg t = kTbCfgs[cfg];
     return (t.steps == 3 && t.tx == 64 && (t.ty == 16 || t.ty == 12) && t.d == 2) ||
-           (t.steps == 4 && t.tx == 64 && t.ty == 16 && t.d == 2);
+           (mode == SCAFES_HEATVAR_F32_KAHAN && t.steps == 4 && t.tx == 64 && t.ty == 16 && t.d == 2);
 }
 
 int heatvar_tb2_num_cfgs() { return kNumTb; }
@@ -1084,7 +1058,7 @@ int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, c
     if (mid) {
         if (mode != SCAFES_HEATVAR_F64)
             return fail(SCAFES_ERR_UNSUPPORTED, "no state-writing variant of this multi-step tile");
-        return tb_dispatch_mo<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit, mid);
+        return tb_dispatch_mo(c, geo, u, kap, uo, cf, cfg, fit, mid);
     }
     if (mode == SCAFES_HEATVAR_F64) return tb_dispatch<double, 0>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit);
     if (mode == SCAFES_HEATVAR_F32) return tb_dispatch<float, 1>(c, geo, u, nullptr, kap, uo, nullptr, cf, cfg, fit);

@@ -210,7 +210,7 @@ bool heatvar_tb2_supported(const Geo& geo, int mode);  // 3-D grids with 32-bit 
 int heatvar_tb2_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, const void* u, void* uo,
                        const void* cin, void* co, const void* kap, double tau, int border_mode, double border_value,
                        int cfg, bool fit, void* const* mid = nullptr);
-bool heatvar_tb_states_supported(int cfg);
+bool heatvar_tb_states_supported(int cfg, int mode);
 int pair_tiles_x(int nx, int k);
 
 // Yee box of N cells per axis; fields hold N+1 nodes per axis, x fastest.

@@ -808,7 +808,6 @@ static const TileCfg kCfgs[] = {
     {64, 8, 256, 4},  {64, 4, 128, 6}, {64, 8, 128, 6}, {128, 4, 128, 6}, {64, 4, 256, 8},
 };
 static constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]);
-static constexpr int kDefaultCfg = 3;
 // Fastest one-step tile per heat7var mode, measured on an MI355X at 512^3
 // (F64 64x8 zc128 d6, F32 128x2 zc64 d4, F32+Kahan 64x16 zc128 d4); used
 // for the odd last step behind two-steps-per-sweep launches.
@@ -880,10 +879,8 @@ static int launch_auto(Ctx* c, const Op& op, const Geo& g)
 }
 
 template <class Op, typename T>
-static int launch(Ctx* c, const Op& op, const Geo& g, int cfg)
+static int launch_tile(Ctx* c, const Op& op, const Geo& g, int cfg)
 {
-    if (cfg < 0) return launch_auto<Op, T>(c, op, g);
-    if (cfg >= kNumCfgs) cfg = kDefaultCfg;
     const TileCfg t = kCfgs[cfg];
     switch (t.tx * 100000 + t.ty * 100 + t.d) {
     case 6400404: return launch_t<Op, T, 64, 4, 4>(c, op, g, t.zc);
@@ -917,10 +914,12 @@ static int launch_steps(Ctx* c, const Op& op, const Geo& g, int k, const StepMid
     if (k == 1) return launch_auto<Op, T>(c, op, g);
     if ((k != 2 && k != 3) || !stepk_supported(g, (int)sizeof(T)))
         return fail(SCAFES_ERR_UNSUPPORTED, "no sweep of this many steps for this grid");
-    if (!mid) return k == 2 ? stepk_launch<Op, T, 2, false>(c, op, g, {}) : stepk_launch<Op, T, 3, false>(c, op, g, {});
-    if constexpr (Op::kNX > 0)
+    if (k == 3 && !mid) return stepk_launch<Op, T, 3, false>(c, op, g, {});
+    if constexpr (Op::kNX > 0) {  // the constant-coefficient run takes three steps or one
+        if (!mid) return stepk_launch<Op, T, 2, false>(c, op, g, {});
         return k == 2 ? stepk_launch<Op, T, 2, true>(c, op, g, *mid) : stepk_launch<Op, T, 3, true>(c, op, g, *mid);
-    return fail(SCAFES_ERR_UNSUPPORTED, "no state-writing sweep of this update");
+    }
+    return fail(SCAFES_ERR_UNSUPPORTED, "no such sweep of this update");
 }
 
 static void hh_of(const scafes_geom* g, double hh[3])
@@ -958,7 +957,7 @@ int heat7var_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, cons
         }
         HeatVarOp<double, 0, true> op{};
         fill(op);
-        return launch<HeatVarOp<double, 0, true>, double>(c, op, geo, cfg);
+        return launch_tile<HeatVarOp<double, 0, true>, double>(c, op, geo, cfg);
     }
     const float c0 = (float)(0.5 * tau / hh[0]), c1 = (float)(0.5 * tau / hh[1]),
                 c2 = (float)(0.5 * tau / hh[2]);
@@ -972,7 +971,8 @@ int heat7var_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, cons
         op.c2 = c2;
         op.border_value = (float)border_value;
         op.border_mode = border_mode;
-        return launch<HeatVarOp<float, 1>, float>(c, op, geo, cfg);
+        return cfg < 0 ? launch_auto<HeatVarOp<float, 1>, float>(c, op, geo)
+                       : launch_tile<HeatVarOp<float, 1>, float>(c, op, geo, cfg);
     }
     HeatVarOp<float, 2> op{};
     op.a = (const float*)u;
@@ -985,7 +985,8 @@ int heat7var_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, cons
     op.c2 = c2;
     op.border_value = (float)border_value;
     op.border_mode = border_mode;
-    return launch<HeatVarOp<float, 2>, float>(c, op, geo, cfg);
+    return cfg < 0 ? launch_auto<HeatVarOp<float, 2>, float>(c, op, geo)
+                   : launch_tile<HeatVarOp<float, 2>, float>(c, op, geo, cfg);
 }
 
 bool pennes_steps_supported(const Geo& geo, int dtype, int border_mode, bool states)
@@ -1096,7 +1097,7 @@ int heatvar_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
         op.c3 = (const double*)uprev;
         op.out = (double*)lam_new;
         fill(op);
-        return launch<HeatVarAdjOp<double>, double>(c, op, geo, -1);
+        return launch_auto<HeatVarAdjOp<double>, double>(c, op, geo);
     }
     HeatVarAdjOp<float> op{};
     op.a = (const float*)lam;
@@ -1104,7 +1105,7 @@ int heatvar_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, 
     op.c3 = (const float*)uprev;
     op.out = (float*)lam_new;
     fill(op);
-    return launch<HeatVarAdjOp<float>, float>(c, op, geo, -1);
+    return launch_auto<HeatVarAdjOp<float>, float>(c, op, geo);
 }
 
 int pennes_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, const void* lam,
@@ -1134,7 +1135,7 @@ int pennes_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, c
         op.ta = p->t_a;
         op.hh = make_by_hh(hh);
         tumor(op);
-        return launch<PennesAdjOp<double>, double>(c, op, geo, -1);
+        return launch_auto<PennesAdjOp<double>, double>(c, op, geo);
     }
     auto fill32 = [&](auto& op) {
         op.a = (const float*)lam;
@@ -1154,11 +1155,11 @@ int pennes_adj_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int dtype, c
         PennesAdjOp<float, true> op{};
         fill32(op);
         op.x[2] = (const float*)tprev_lo;
-        return launch<PennesAdjOp<float, true>, float>(c, op, geo, -1);
+        return launch_auto<PennesAdjOp<float, true>, float>(c, op, geo);
     }
     PennesAdjOp<float> op{};
     fill32(op);
-    return launch<PennesAdjOp<float>, float>(c, op, geo, -1);
+    return launch_auto<PennesAdjOp<float>, float>(c, op, geo);
 }
 
 // ---------------------------------------------------------------- init
@@ -1282,7 +1283,7 @@ int scafes_heat7_step_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, const d
     HeatConstOp op;
     const int rc = heat7_const_op(c, g, hw, u_old, u_new, f_old, g_old, g_new, p, &geo, &op);
     if (rc) return rc;
-    return launch<HeatConstOp, double>(c, op, geo, -1);
+    return launch_auto<HeatConstOp, double>(c, op, geo);
 }
 
 int scafes_heat7_run_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, double* u, double* u2, int nsteps,
@@ -1677,7 +1678,7 @@ int scafes_mri_step_f64(scafes_ctx* ctx, const scafes_geom* g, int hw, const dou
     op.sigma = p->sigma;
     const double ta = p->t_amb + 273.15;
     op.tamb4 = ((ta * ta) * ta) * ta;
-    return launch<MriOp, double>(c, op, geo, -1);
+    return launch_auto<MriOp, double>(c, op, geo);
 }
 
 int scafes_pennes_adjoint_step(scafes_ctx* ctx, const scafes_geom* g, int hw, int dtype, const void* lam,
@@ -1755,13 +1756,13 @@ static int states_cfg(const Ctx* c, const Geo& geo, int mode)
 bool heat7var_states_sweep_ok(const Ctx* c, const Geo& geo, int mode)
 {
     const int cfg = states_cfg(c, geo, mode);
-    return cfg >= kNumCfgs && cfg_steps(cfg) == 3 && heatvar_tb_states_supported(cfg - kNumCfgs);
+    return cfg >= kNumCfgs && cfg_steps(cfg) == 3 && heatvar_tb_states_supported(cfg - kNumCfgs, mode);
 }
 
 bool heat7var_states4_ok(const Ctx* c, const Geo& geo, int mode)
 {
     const int f = kFourStepCfgByMode[mode];
-    return heat7var_states_sweep_ok(c, geo, mode) && f >= kNumCfgs && heatvar_tb_states_supported(f - kNumCfgs);
+    return heat7var_states_sweep_ok(c, geo, mode) && f >= kNumCfgs && heatvar_tb_states_supported(f - kNumCfgs, mode);
 }
 
 int heat7var_sweep_states(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, int k, const void* u, void* un,

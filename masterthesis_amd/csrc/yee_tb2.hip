@@ -21,39 +21,12 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "plane_buffer.hpp"
 #include "scafes_common.hpp"
 
 namespace scafes {
 
 namespace {
-
-using Rsrc = __amdgpu_buffer_rsrc_t;
-constexpr int kRsrcWord3 = 0x00020000;  // gfx9 family: 32-bit data format, raw (stride 0) buffer
-
-__device__ inline Rsrc rsrc(const char* p, uint32_t range)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p), (short)0, (int)range, kRsrcWord3);
-}
-
-template <typename T>
-__device__ inline T bld(Rsrc r, uint32_t off)
-{
-    if constexpr (sizeof(T) == 4)
-        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
-    else
-        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
-}
-
-template <typename T>
-__device__ inline void bst(T v, Rsrc r, uint32_t off)
-{
-    if constexpr (sizeof(T) == 4) {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, (int)off, 0, 0);
-    } else {
-        typedef int v2i __attribute__((ext_vector_type(2)));
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i, v), r, (int)off, 0, 0);
-    }
-}
 
 template <typename T>
 struct V3 {
@@ -145,20 +118,20 @@ __global__ __launch_bounds__(TX* TY) void yee_tb2_kernel(YeeDims d, T s, const T
     // plane consumes instead of for every outstanding access.
     auto fetch = [&](const int slot, const int kk) {
         const char* p = a8 + plane(kk);
-        const Rsrc rEx = rsrc(p, range), rEy = rsrc(p + fs, range), rEz = rsrc(p + 2 * fs, range);
+        const Rsrc rEx = plane_rsrc(p, range), rEy = plane_rsrc(p + fs, range), rEz = plane_rsrc(p + 2 * fs, range);
         const bool in = kk <= klast;
         const uint32_t o0 = in ? oc : range, o1 = (in && rx) ? ox : range, o2 = (in && ry) ? oy : range;
-        qex[slot] = bld<T>(rEx, o0);
-        qey[slot] = bld<T>(rEy, o0);
-        qez[slot] = bld<T>(rEz, o0);
-        qhx[slot] = bld<T>(rsrc(p + 3 * fs, range), o0);
-        qhy[slot] = bld<T>(rsrc(p + 4 * fs, range), o0);
-        qhz[slot] = bld<T>(rsrc(p + 5 * fs, range), o0);
-        rxy[slot] = bld<T>(rEy, o1);
-        rxz[slot] = bld<T>(rEz, o1);
-        ryx[slot] = bld<T>(rEx, o2);
-        ryz[slot] = bld<T>(rEz, o2);
-        if constexpr (EPS) qce[slot] = bld<T>(rsrc(c8 + plane(kk), range), o0);
+        qex[slot] = bload<T>(rEx, o0);
+        qey[slot] = bload<T>(rEy, o0);
+        qez[slot] = bload<T>(rEz, o0);
+        qhx[slot] = bload<T>(plane_rsrc(p + 3 * fs, range), o0);
+        qhy[slot] = bload<T>(plane_rsrc(p + 4 * fs, range), o0);
+        qhz[slot] = bload<T>(plane_rsrc(p + 5 * fs, range), o0);
+        rxy[slot] = bload<T>(rEy, o1);
+        rxz[slot] = bload<T>(rEz, o1);
+        ryx[slot] = bload<T>(rEx, o2);
+        ryz[slot] = bload<T>(rEz, o2);
+        if constexpr (EPS) qce[slot] = bload<T>(plane_rsrc(c8 + plane(kk), range), o0);
     };
     const int kfirst = k0 - 2;
 #pragma unroll
@@ -203,9 +176,9 @@ __global__ __launch_bounds__(TX* TY) void yee_tb2_kernel(YeeDims d, T s, const T
                 const size_t o = plane(kk);
                 const uint32_t os = (out && kk >= k0 && kk < k1) ? oc : range;
                 char* m8 = (char*)fm;
-                bst<T>(h1.x, rsrc(m8 + o + 3 * fs, range), os);
-                bst<T>(h1.y, rsrc(m8 + o + 4 * fs, range), os);
-                bst<T>(h1.z, rsrc(m8 + o + 5 * fs, range), os);
+                bstore<T>(h1.x, plane_rsrc(m8 + o + 3 * fs, range), os);
+                bstore<T>(h1.y, plane_rsrc(m8 + o + 4 * fs, range), os);
+                bstore<T>(h1.z, plane_rsrc(m8 + o + 5 * fs, range), os);
             }
             if (out && kk >= k0 && kk < k1 && ep0) {
                 es0 += 0.5 * ((double)e0.x * e0.x + (double)e0.y * e0.y + (double)e0.z * e0.z) +
@@ -222,9 +195,9 @@ __global__ __launch_bounds__(TX* TY) void yee_tb2_kernel(YeeDims d, T s, const T
                 const size_t o = plane(kb1);
                 const uint32_t os = (out && kb1 >= k0 && kb1 < k1) ? oc : range;
                 char* m8 = (char*)fm;
-                bst<T>(e1.x, rsrc(m8 + o, range), os);
-                bst<T>(e1.y, rsrc(m8 + o + fs, range), os);
-                bst<T>(e1.z, rsrc(m8 + o + 2 * fs, range), os);
+                bstore<T>(e1.x, plane_rsrc(m8 + o, range), os);
+                bstore<T>(e1.y, plane_rsrc(m8 + o + fs, range), os);
+                bstore<T>(e1.z, plane_rsrc(m8 + o + 2 * fs, range), os);
             }
             // ---- C: H2 at plane kk-2 (E1 plane kk-2 from the previous iteration, E1(kk-1) in registers)
             const int kc = kk - 2;
@@ -237,9 +210,9 @@ __global__ __launch_bounds__(TX* TY) void yee_tb2_kernel(YeeDims d, T s, const T
                 const bool st = out && kc >= k0 && kc < k1;
                 const size_t o = plane(kc);
                 const uint32_t os = st ? oc : range;
-                bst<T>(h2.x, rsrc(b8 + o + 3 * fs, range), os);
-                bst<T>(h2.y, rsrc(b8 + o + 4 * fs, range), os);
-                bst<T>(h2.z, rsrc(b8 + o + 5 * fs, range), os);
+                bstore<T>(h2.x, plane_rsrc(b8 + o + 3 * fs, range), os);
+                bstore<T>(h2.y, plane_rsrc(b8 + o + 4 * fs, range), os);
+                bstore<T>(h2.z, plane_rsrc(b8 + o + 5 * fs, range), os);
                 if (st && ep1)
                     es1 += 0.5 * ((double)e1m1.x * e1m1.x + (double)e1m1.y * e1m1.y + (double)e1m1.z * e1m1.z) +
                            0.5 * ((double)h1m2.x * h2.x + (double)h1m2.y * h2.y + (double)h1m2.z * h2.z);
@@ -254,9 +227,9 @@ __global__ __launch_bounds__(TX* TY) void yee_tb2_kernel(YeeDims d, T s, const T
                                      L.h2[0][pbf][tym][tx], L.h2[2][pbf][ty][txm], L.h2[1][pbf][ty][txm]);
                 const size_t o = plane(kd);
                 const uint32_t os = st ? oc : range;
-                bst<T>(e2.x, rsrc(b8 + o, range), os);
-                bst<T>(e2.y, rsrc(b8 + o + fs, range), os);
-                bst<T>(e2.z, rsrc(b8 + o + 2 * fs, range), os);
+                bstore<T>(e2.x, plane_rsrc(b8 + o, range), os);
+                bstore<T>(e2.y, plane_rsrc(b8 + o + fs, range), os);
+                bstore<T>(e2.z, plane_rsrc(b8 + o + 2 * fs, range), os);
             }
             // ---- shift the z queues
             h2m2x = h2m1.x;

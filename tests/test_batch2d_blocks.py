@@ -44,7 +44,7 @@ def test_border_untouched_by_the_far_side_of_a_block(hip, bad, gradient):
                 u[at, 2:-2] = bad
                 u[2:-2, at] = bad
     with capi.Context(0) as ctx:
-        d = [ctx.upload(a) for a in (n, off, kappa, tau, np.arange(len(n), dtype=np.int32), u0, 0 * u0)]
+        d = [ctx.upload(a) for a in (n, off, kappa, tau, np.arange(len(n), dtype=np.int32), u0, np.zeros_like(u0))]
         J, G = ctx.alloc(len(n)), ctx.alloc(len(n))
         p = [x.ptr for x in d]
         capi.check(ctx.L.scafes_batch2d_run(ctx.h, len(n), *p[:6], p[6] if gradient else None,
