@@ -301,7 +301,10 @@ void coef_invalidate(Ctx* c, const void* p, size_t bytes)
 // pipeline behind them), so long chunks waste least and short ones fill the
 // CUs: per_cu workgroups run at once on a CU, a last round of at most one
 // workgroup per CU takes about 0.65 of one of two, and the chunk with the
-// least rounds x (planes + fill) is taken (the longest of equals).  Where the
+// least rounds x (planes + fill) is taken, of equals the shortest: chunks 128 planes
+// apart at 512^3 start on the same memory channels (four-step sweeps of FP32 + Kahan,
+// 8 steps from one arrangement of the arrays 1752 us with 128 planes, 1612 with 74;
+// from another 1679 and 1559).  Where the
 // full chunk already makes four rounds it stays: there the measured default
 // tiles hold.  Measured on an MI355X against chunks of 4..64 planes on grids
 // of 48^3 to 384x300x320, the choice is within 8 % of the best of them for
@@ -320,7 +323,7 @@ int fit_chunk(long nxy, int nz, int fill, int zmax, int per_cu, int cu_count)
         const long rem = nb % slots;
         const double rounds = (double)(nb / slots) + (rem == 0 ? 0.0 : rem <= cus && per_cu > 1 ? 0.65 : 1.0);
         const double cost = rounds * (zc + fill);
-        if (least == 0.0 || cost < least) {
+        if (least == 0.0 || cost <= least) {
             least = cost;
             best = zc;
         }
