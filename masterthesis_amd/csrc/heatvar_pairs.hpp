@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64 * TY) void heatvar_pairs_kernel(Geo g, const flo
                                                                  const float* __restrict__ kap, float* __restrict__ uout,
                                                                  float* __restrict__ cout, float* __restrict__ u1o,
                                                                  float* __restrict__ u2o, float* __restrict__ u3o, VarCoef cf,
-                                                                 int zc, int tiles_x, int tiles_y)
+                                                                 int zc, int tiles_x, int tiles_y, int x0)
 {
     static_assert(K == 3 || K == 4, "three or four steps");
     static_assert(D == 2 || D == 4, "the prefetch slots repeat within the unrolled planes");
@@ -120,10 +120,10 @@ __global__ __launch_bounds__(64 * TY) void heatvar_pairs_kernel(Geo g, const flo
     const int txi = rr - tyi * tiles_x;
     // the first tile needs no columns before it and the last none after it: the
     // border nodes there take no neighbour values
-    const int i = txi * OX + tx, j0 = tyi * OY - (K - 1) + 2 * ty;
-    const int ic = min(i, g.nx - 1);
+    const int i = txi * OX - x0 + tx, j0 = tyi * OY - (K - 1) + 2 * ty;
+    const int ic = min(max(i, 0), g.nx - 1);
     const bool inner_x = i >= g.nl0 && i <= g.nx - 1 - g.nl0;
-    const bool col_out = (tx >= K || txi == 0) && (tx <= 63 - K || txi == tiles_x - 1) && i < g.nx;
+    const bool col_out = (tx >= K || (txi == 0 && i >= 0)) && (tx <= 63 - K || txi == tiles_x - 1) && i < g.nx;
     const int k0 = tz * zc, k1 = min(k0 + zc, g.nz);
     const int kfirst = k0 - (K - 1);  // first plane with a level-1 value
     const int klast = k1 + K - 2;     // last iteration

@@ -971,6 +971,9 @@ static int pairs_launch_t(Ctx* c, const PairArgs& a)
     constexpr int kPerCu = TY > 8 ? 1 : 2;
     const Geo& g = a.g;
     const int tiles_x = pair_tiles_x(g.nx, K), tiles_y = ceil_div(g.ny, 2 * TY - 2 * (K - 1));
+    // one column before the row where it costs no tile: with one ghost layer and
+    // an even nx the tiles of even offset then start on whole 8 bytes
+    const int x0 = pair_tiles_x(g.nx + 1, K) == tiles_x ? 1 : 0;
     const int zc = fit_chunk((long)tiles_x * tiles_y, g.nz, 2 * K - 1, a.zmax, kPerCu, c->cu_count);
     const long nb = (long)tiles_x * tiles_y * ceil_div(g.nz, zc);
     if (nb > 0x7fffffffL) return fail(SCAFES_ERR_ARG, "grid too large");
@@ -979,7 +982,7 @@ static int pairs_launch_t(Ctx* c, const PairArgs& a)
         for (int l = 0; l < K - 1; ++l) m[l] = (float*)a.mid[l];
     heatvar_pairs_kernel<MODE, TY, K, D, MO><<<dim3((unsigned)nb), dim3(64, TY), 0, c->stream>>>(
         g, (const float*)a.u, (const float*)a.cin, (const float*)a.kap, (float*)a.uo, (float*)a.co, m[0], m[1], m[2],
-        a.cf, zc, tiles_x, tiles_y);
+        a.cf, zc, tiles_x, tiles_y, x0);
     SCAFES_HIP(hipGetLastError());
     return SCAFES_OK;
 }

@@ -15,8 +15,11 @@ def test_tiles_cover_the_row(k):
     step = 64 - 2 * k
     for nx in range(3, 1500):
         t = f(nx, k)
-        stored = [q for x in range(t) for q in range(x * step + (k if x else 0),
-                                                     min(x * step + (64 - k if x < t - 1 else 64), nx))]
+        x0 = 1 if f(nx + 1, k) == t else 0  # columns before the row
+        stored = []
+        for x in range(t):
+            first, last = k if x else x0, 63 - k if x < t - 1 else 63
+            stored += [q for q in range(x * step - x0 + first, x * step - x0 + last + 1) if q < nx]
         assert stored == list(range(nx)), nx
     assert [f(nx, k) for nx in (60, 64, 65, 120)] == [1, 1, 2, 2]
 
