@@ -411,8 +411,9 @@ def bench_heat64(ctx, capi, n=64, nsteps=100):
     exact_discrete = (1.0 - tau * lam_h) ** nsteps * mode
     analytic = np.exp(-3 * np.pi ** 2 * t) * mode
     return {"workload": f"heat {n}^3 FP64, sine mode, zero Dirichlet, tau = 0.9 h^2/6, {nsteps} steps",
-            "kernel": ("stepk_kernel<HeatConstOp> (three steps per sweep)" if n ** 3 <= 300000 or n ** 3 > 8000000
-                       else "row_kernel<HeatConstOp> (one step per launch)") + ", scafes_heat7_run_f64", "ms": round(ms, 4),
+            "kernel": "scafes_heat7_run_f64: stepk_kernel<HeatConstOp> (three steps per sweep, the last step "
+                      "alone) on small and very large grids, row_kernel<HeatConstOp> (one step) between",
+            "ms": round(ms, 4),
             "GLUPS": round(float(n) ** 3 * nsteps / (ms * 1e-3) / 1e9, 3),
             "rel_err_vs_discrete_closed_form": float(np.abs(u - exact_discrete).max() / np.abs(exact_discrete).max()),
             "rel_err_vs_analytic": float(np.abs(u - analytic).max() / np.abs(analytic).max())}
@@ -489,9 +490,9 @@ def bench_kappa_grad(ctx, capi, g, n, u0, k0, tau, nsteps, t_fwd_ms, snapshots=(
                         "three) writing the states in between (heatvar_pairs_kernel<2, 12, 3, 2, true>, 28 "
                         "B/node per sweep; heatvar_pairs_kernel<2, 16, 4, 2, true>, 32 B/node per sweep); else "
                         "one step",
-           "adjoint_kernels": "heatvar_adjk_kernel<float, 64, 16, K, 2> (K <= 4 reverse steps per sweep where the "
+           "adjoint_kernels": "heatvar_adjk_kernel<64, TY, K, 2> (K <= 4 reverse steps per sweep where the "
                               "schedule has the states at hand, (28 + 4K) B/node per sweep: lam r+w, kappa, "
-                              "u^{n-1..n-K}, FP64 gradient r+w); stream_kernel<HeatVarAdjOp<float>> (one step, "
+                              "u^{n-1..n-K}, FP64 gradient r+w); row_kernel<HeatVarAdjOp<float>> (one step, "
                               "32 B) elsewhere",
            "adjoint_profile": _profile_fields("heat7var_adjoint_512.md", n == 512),
            "gradient": []}
@@ -925,7 +926,7 @@ def main():
         "data": "synthetic (device-seeded splitmix64 noise on the analytic sine mode)",
         "config": {"workload": f"heat7var {n}^3 nodes, variable kappa, FP32 + Kahan, {args.steps} Euler steps",
                    "nodes": n ** 3, "tau": tau, "kernel": kname, "cfg": cfg, "steps_per_launch": sps,
-                   "z_planes_per_workgroup": zc,
+                   "z_planes_per_workgroup_at_most": zc,
                    "sweeps": ", ".join(f"{m} x {kk} steps ({SWEEP_KERNEL[kk]})" for kk, m in plan32),
                    "warmup_note": f"{args.warmup} warm-up steps, one sweep of each kind the timed run launches, "
                                   f"then untimed sweeps of the same kernels until the GPU has been busy "

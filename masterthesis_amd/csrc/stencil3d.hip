@@ -900,7 +900,14 @@ static int launch_tile(Ctx* c, const Op& op, const Geo& g, int cfg)
 }
 
 // FP64 grids up to this size keep a step's four arrays in the Infinity Cache
-// (256 MB), where single steps are as fast as sweeps (the figures in stepk.hpp).
+// (256 MB), where single steps come close to sweeps or pass them; how close
+// depends on how well the 60x8 output tile fits the grid, which the lines drawn
+// here by size leave aside.  Measured on an MI355X, us, single steps / three per
+// sweep: heat, 100 steps, 30^3 326 / 247, 64^3 373 / 361, 72^3 425 / 436, 97x80x75 513 /
+// 490, 120^3 900 / 748, 128^3 952 / 1095, 180^3 2098 / 1682, 200x200x199 2589 / 2536,
+// 240^3 4114 / 3600; Pennes gradient of 31 steps with every state stored, FP64 120^3 829
+// / 749, 128^3 1013 / 990, 200^3 3135 / 3088, 240^3 5473 / 4551; FP32 97x80x75 311 / 294,
+// 120^3 491 / 458, 128^3 559 / 587, 140^3 666 / 633, 150^3 782 / 730.
 constexpr long kCachedNodes64 = 8000000L;
 
 // Steps of the next sweep of a run of one-field updates with `left` to go:
@@ -989,6 +996,8 @@ int heat7var_launch(Ctx* c, const Geo& geo, const scafes_geom* g, int mode, cons
                    : launch_tile<HeatVarOp<float, 2>, float>(c, op, geo, cfg);
 }
 
+// FP32 sweeps that write the states in between lose where 60 columns and 12 rows
+// leave the last tiles nearly empty, as at 124..132 nodes (figures above).
 bool pennes_steps_supported(const Geo& geo, int dtype, int border_mode, bool states)
 {
     const long nodes = (long)geo.nx * geo.ny * geo.nz;
