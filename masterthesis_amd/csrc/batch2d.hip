@@ -20,8 +20,8 @@
 // rows.  Bound by vector issue: six instructions per node and step.  Measured
 // on an MI355X, ms, a select, a product and two differences more per node, edges
 // by component, two barriers at every size -> now: 4096 problems of 32..256
-// nodes an edge, 500 steps with the gradient 15.04 -> 12.21; 512 of 256, 100
-// steps 0.983 -> 0.793; 3000 of 2..64, 300 steps 1.600 -> 1.103.
+// nodes an edge, 500 steps with the gradient 15.04 -> 12.15; 512 of 256, 100
+// steps 0.976 -> 0.793; 3000 of 2..64, 300 steps 1.577 -> 1.052.
 // Each block size B is a separate non-inlined function, so each gets its
 // own register allocation: inlined into one kernel, the B = 8 body's
 // pressure would spill in every smaller body too.  Problems are taken in

@@ -18,8 +18,8 @@
 //
 // Four full-rate instructions stand for the eleven of a division, one of them
 // the quarter-rate reciprocal.  Measured on an MI355X, us, divisions ->
-// quotients: var-kappa FP64 three-step sweep 512^3 1890 -> 1660; 50 steps at
-// 201x150x131 1211 -> 1044; one constant-coefficient step 300x200x200 (bound by
+// quotients: var-kappa FP64 three-step sweep 512^3 1890 -> 1490; 50 steps at
+// 201x150x131 1211 -> 996; one constant-coefficient step 300x200x200 (bound by
 // memory) 60 -> 57; MRI step 120x120x50 15.6 -> 15.0.
 #pragma once
 

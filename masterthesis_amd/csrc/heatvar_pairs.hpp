@@ -15,10 +15,10 @@
 //     south and lower faces and the second old plane of each level;
 //   - LDS carries only the rows that the wavefronts above and below read: 8 reads and
 //     10 writes per row pair and plane for three levels (48 before).
-// 78-116 vector registers, no spills.  The faces and prefetch slots are rings
+// 78-128 vector registers, no spills.  The faces and prefetch slots are rings
 // indexed by the unrolled plane (four planes; six for three steps cost 15
 // registers more).  Measured on an MI355X, us for 20 steps of FP32 + Kahan at 512^3
-// 5620 -> 3620 (three steps of one sweep 800 -> 710, four 1084 -> 730); FP32 at
+// 5620 -> 3460 (three steps of one sweep 800 -> 710, four 1084 -> 690); FP32 at
 // 512^3, four steps, 637 (three) -> 511; 24 steps, FP32 + Kahan 128^3 188 -> 135, 256^3
 // 943 -> 558, 97x80x75 93 -> 81.  What is left at 512^3 is the copy rate: 2.7 GB per
 // sweep take 565 us.  FP64 keeps one node per thread: this form needs 174 registers
@@ -35,7 +35,7 @@ namespace scafes {
 // Planes of a workgroup's z chunk at most, and the grids from which four steps
 // a sweep are the default (FP32 and FP32 + Kahan; us for 24 steps as three /
 // four per sweep, FP32 + Kahan: 64^3 70 / 67, 97x80x75 81 / 78, 128^3 145 / 135,
-// 256^3 720 / 558; 512^3, per step, 237 / 183).
+// 256^3 720 / 558; 512^3, per step, 237 / 172).
 constexpr int kPairZC = 128;
 constexpr long kFourStepNodes = 1500000;
 

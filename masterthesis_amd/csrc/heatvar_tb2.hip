@@ -200,7 +200,7 @@ __global__ __launch_bounds__(TX* TY) void heatvar_tb2_kernel(Geo g, const T* __r
 // and rewrite their own centre, off-ring rows write the y ring into a sink
 // row, and lanes off the output columns store out of range.  Measured on an
 // MI355X at 512^3 (us per three-step sweep): F64 (64x16) 1882 -> 1767 against
-// the branching kernel, 1660 with quotients by h^2 that need no division.
+// the branching kernel, 1490 with quotients by h^2 that need no division.
 // FP64 fields, and FP32 ones on the 128-lane tile; other FP32 tiles take
 // heatvar_pairs_kernel.
 // MO: the states after one and two steps are written too (u1o, u2o; the

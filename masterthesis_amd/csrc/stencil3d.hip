@@ -813,7 +813,7 @@ static constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]);
 // for the odd last step behind two-steps-per-sweep launches.
 static constexpr int kOneStepCfgByMode[3] = {12, 4, 9};
 // Default per mode (indices into heatvar_tb2.hip's table), all three steps per
-// sweep: F64 64x16 zc64 d2 (10; 553 us/step at 512^3), F32 and F32 + Kahan 64x12 zc64
+// sweep: F64 64x16 zc64 d2 (10; 495 us/step at 512^3), F32 and F32 + Kahan 64x12 zc64
 // d2 (13).  Where neither a caller nor the autotuner names the tile, the z chunk and
 // the FP32 tile's rows are fitted to the grid.
 static constexpr int kDefaultCfgByMode[3] = {kNumCfgs + 10, kNumCfgs + 13, kNumCfgs + 13};
@@ -823,11 +823,11 @@ static constexpr int kDefaultCfgByMode[3] = {kNumCfgs + 10, kNumCfgs + 13, kNumC
 static constexpr int kTwoStepCfgByMode[3] = {kNumCfgs + 6, kNumCfgs + 2, kNumCfgs + 2};
 // Four-step tile per mode behind a three-step default, or -1: F32 + Kahan
 // 64x16 zc128 d2.  FP32 keeps the two-step remainder (grids of up to
-// kFourStepNodes nodes); FP64 loses with four steps (2148 us against 1553 for three at
+// kFourStepNodes nodes); FP64 loses with four steps (2148 us against 1490 for three at
 // 512^3).
 static constexpr int kFourStepCfgByMode[3] = {-1, -1, kNumCfgs + 24};
 // Default of FP32 fields on grids of more than kFourStepNodes nodes, where
-// four steps a sweep are the fastest per step (512^3: FP32 + Kahan 183 us a step
+// four steps a sweep are the fastest per step (512^3: FP32 + Kahan 172 us a step
 // against 237 for three, FP32 128 against 145).
 static constexpr int kLargeCfgByMode[3] = {-1, kNumCfgs + 24, kNumCfgs + 24};
 

@@ -23,7 +23,7 @@
 // 9.1, 256^3 47 -> 29; with the states in between written 4.2 -> 3.6, 7.0 -> 7.9, 11.3
 // -> 10.3, 47 -> 42; FP32 + Kahan 97x80x75 5.0 -> 3.5, 128^3 9.5 -> 7.3, 256^3 79 ->
 // 43; FP64 128^3 12.5 -> 12.5, 201x150x131 20.5 -> 20.1, 256^3 106 -> 71; heat FP64
-// 64^3 3.9 -> 3.8, 128^3 11.5 -> 12.1, 256^3 63 -> 52.  Under the Tumor border the
+// 64^3 3.7 -> 3.6, 128^3 9.5 -> 10.9, 256^3 61 -> 47.  Under the Tumor border the
 // sweep lost to the rows up to 201x150x131 (13.8 against 12.2 us).
 #pragma once
 
