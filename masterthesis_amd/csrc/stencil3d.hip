@@ -858,15 +858,23 @@ static int launch_t(Ctx* c, const Op& op, const Geo& g, int zc)
 // 67 / 63 / 63; MRI 120x120x50 15.7 -> 10.1 / 10.6 / 13.1 / 19.1, 201x150x131
 // 49.5 -> 34.6 / 35.9 / 36.9 / 40.8; Pennes adjoint FP32 97x80x75 10.3 -> 6.0 /
 // 6.0 / 7.1 / 10.1; kappa adjoint FP64 201x150x131 69 -> 45 / 40 / 37 / 37.
-// Rows shorter than a vector take the LDS tile.
+// Rows shorter than a vector take the LDS tile, in chunks that shrink from 8 planes
+// towards four workgroups per CU (five Pennes FP32 steps at 3x40x40 35 us with 8
+// planes, 20 with one).
 template <class Op, typename T>
 static int launch_auto(Ctx* c, const Op& op, const Geo& g)
 {
     constexpr int V = 16 / (int)sizeof(T);
-    if (g.nx < V) return launch_t<Op, T, 64, 4, 4>(c, op, g, 8);
+    const long cus = c->cu_count > 0 ? c->cu_count : 256;
+    if (g.nx < V) {
+        const long per_plane = ceil_div(g.ny, 4);
+        int zc = 8;
+        if (per_plane * ceil_div(g.nz, zc) < cus)
+            zc = (int)std::max(1L, std::min((long)zc, per_plane * g.nz / (4 * cus)));
+        return launch_t<Op, T, 64, 4, 4>(c, op, g, zc);
+    }
     const int cpr = ceil_div(g.nx, V);
     const long bxy = ceil_div((long)cpr * g.ny, 256);
-    const long cus = c->cu_count > 0 ? c->cu_count : 256;
     const int zmax = Op::kTwo ? 8 : Op::kNX >= 3 ? 2 : 4;
     int zc = 1;
     if (bxy * g.nz > 8 * cus) zc = 2;
