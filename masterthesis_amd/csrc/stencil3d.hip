@@ -183,10 +183,9 @@ struct VecOf {
     typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T))));
 };
 
-template <class Op, typename T>
+template <class Op, typename T, int V = 16 / (int)sizeof(T)>
 __global__ __launch_bounds__(256) void row_kernel(Op op, Geo g, int zc, int cpr, int blocks_xy)
 {
-    constexpr int V = 16 / (int)sizeof(T);
     constexpr int NF = Op::kThree ? 3 : Op::kTwo ? 2 : 1;
     constexpr int NX = Op::kNX;
     constexpr int NXA = NX > 0 ? NX : 1;
@@ -861,6 +860,32 @@ static int launch_t(Ctx* c, const Op& op, const Geo& g, int zc)
 // Rows shorter than a vector take the LDS tile, in chunks that shrink from 8 planes
 // towards four workgroups per CU (five Pennes FP32 steps at 3x40x40 35 us with 8
 // planes, 20 with one).
+template <class Op, typename T, int V>
+static int launch_rows(Ctx* c, const Op& op, const Geo& g, long cus)
+{
+    const int cpr = ceil_div(g.nx, V);
+    const long bxy = ceil_div((long)cpr * g.ny, 256);
+    const int zmax = Op::kTwo ? 8 : Op::kNX >= 3 ? 2 : 4;
+    int zc = 1;
+    if (bxy * g.nz > 8 * cus) zc = 2;
+    if (bxy * g.nz > 24 * cus) zc = zmax;
+    const long nb = bxy * ceil_div(g.nz, zc);
+    if (nb > 0x7fffffffL || (long)cpr * g.ny > 0x7fffffffL - 256) return fail(SCAFES_ERR_ARG, "grid too large");
+    row_kernel<Op, T, V><<<dim3((unsigned)nb), dim3(256), 0, c->stream>>>(op, g, zc, cpr, (int)bxy);
+    SCAFES_HIP(hipGetLastError());
+    return SCAFES_OK;
+}
+
+// The MRI step's border nodes make a chain of up to seven divisions, and a thread
+// with two nodes runs it twice: grids whose vector rows make at most one workgroup
+// per CU take one node per thread (us for 20 steps, the LDS tile / vectors / one
+// node: 20^3 84 / 94 / 81, 26x59x13 85 / 97 / 80, 40^3 87 / 90 / 81, 50^3 100 / 88 / 82,
+// 60^3 132 / 100 / 101, 120x120x50 315 / 193 / 197).
+template <class Op>
+constexpr bool kOneNodeRows = false;
+template <>
+constexpr bool kOneNodeRows<MriOp> = true;
+
 template <class Op, typename T>
 static int launch_auto(Ctx* c, const Op& op, const Geo& g)
 {
@@ -873,17 +898,10 @@ static int launch_auto(Ctx* c, const Op& op, const Geo& g)
             zc = (int)std::max(1L, std::min((long)zc, per_plane * g.nz / (4 * cus)));
         return launch_t<Op, T, 64, 4, 4>(c, op, g, zc);
     }
-    const int cpr = ceil_div(g.nx, V);
-    const long bxy = ceil_div((long)cpr * g.ny, 256);
-    const int zmax = Op::kTwo ? 8 : Op::kNX >= 3 ? 2 : 4;
-    int zc = 1;
-    if (bxy * g.nz > 8 * cus) zc = 2;
-    if (bxy * g.nz > 24 * cus) zc = zmax;
-    const long nb = bxy * ceil_div(g.nz, zc);
-    if (nb > 0x7fffffffL || (long)cpr * g.ny > 0x7fffffffL - 256) return fail(SCAFES_ERR_ARG, "grid too large");
-    row_kernel<Op, T><<<dim3((unsigned)nb), dim3(256), 0, c->stream>>>(op, g, zc, cpr, (int)bxy);
-    SCAFES_HIP(hipGetLastError());
-    return SCAFES_OK;
+    if constexpr (kOneNodeRows<Op>)
+        if ((long)ceil_div((long)ceil_div(g.nx, V) * g.ny, 256) * g.nz <= cus)
+            return launch_rows<Op, T, 1>(c, op, g, cus);
+    return launch_rows<Op, T, V>(c, op, g, cus);
 }
 
 template <class Op, typename T>

@@ -186,8 +186,9 @@ def test_gradients(ctx, n, steps):
                                        atol=steps * 100 * 2.0 ** -24 * max(np.abs(ref).max(), 1e-3))
 
 
-@pytest.mark.parametrize("n", NS)
+@pytest.mark.parametrize("n", NS + [(130, 120, 9), (131, 121, 9), (60, 64, 32), (61, 65, 33)])
 def test_mri(ctx, n):
+    """The last four on both sides of the size from which a thread takes a vector."""
     rng = np.random.default_rng(5 + sum(n))
     shape = tuple(reversed(n))
     mats = [1040.0 * (1 + 0.1 * rng.random(shape)), 3650.0 * (1 + 0.1 * rng.random(shape)), 0.5 + rng.random(shape),
